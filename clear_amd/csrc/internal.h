@@ -153,6 +153,14 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
                        clr_lbvh_leaf* leaves, hipStream_t stream);
 
 // ---- rendering (render.hip, wavefront.hip) ----
+// The traversal layout a call needs: none (the reference walks read the
+// drop-in nodes), the binary records (the visualiser's counting walk), or the
+// 4-wide records (every other walk).
+enum class AccelKind { kNone, kBinary, kWide };
+inline AccelKind accelFor(const clr_render_params& rp) {
+    return (rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL) ? AccelKind::kNone : AccelKind::kWide;
+}
+int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, AccelKind kind, hipStream_t stream);
 int ensureRenderScratch(clr_ctx* ctx, uint32_t numFaces);
 int renderMegakernel(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_params& rp,
                      uint32_t* states, clr_float3* pixels, hipStream_t stream);
@@ -186,7 +194,8 @@ int checkRenderArgs(clr_ctx* ctx, const clr_scene_dev* scene, const clr_render_p
 // ---- traversal (traverse.hip) ----
 int ensureTraceSpill(clr_ctx* ctx, size_t bytes);
 // Launches the traversal-layout build into caller-given arrays (from the
-// LBVH pair, or from a CPU midpoint BVH when bvh is not null).
+// LBVH pair, or from a CPU midpoint BVH when bvh is not null; without node
+// records when anodes is null).
 void launchAccelBuild(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
                       uint32_t n, const clr_float3* vertices, const clr_face* faces, float4* anodes, float4* atris,
                       hipStream_t stream);
@@ -199,9 +208,9 @@ void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, 
 // Face -> first light map and first environment light of one scene.
 void launchFaceLights(const clr_light_info* lights, uint32_t numLights, uint32_t numFaces, uint32_t* faceLight,
                       int* envLight, hipStream_t stream);
-// Builds the ordered walk's traversal layout from the drop-in nodes on `stream`
-// into context memory and returns its two arrays, and with `wnodes` the
-// renderers' 4-wide records too.
+// Builds the ordered traversal's layout from the drop-in nodes on `stream`
+// into context memory: the triangle records, with `anodes` the binary node
+// records, with `wnodes` the 4-wide records.
 int buildAccel(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
                uint32_t n, const clr_float3* vertices, const clr_face* faces, const float4** anodes,
                const float4** atris, hipStream_t stream, const float4** wnodes = nullptr);

@@ -470,19 +470,17 @@ __device__ __forceinline__ void renderTile(const dev::RScene& S, uint32_t tile, 
     dev::V3 acc = dev::v3z();
     dev::NoHook hook;
     // MERGED: the sample and bounce loops merged (tracePixel).
-    if constexpr (LDS < dev::kStackDepth) {
-        const dev::SpillStack<LDS> stk{s_stack + threadIdx.x, 64, spill + lane, lanes};
+    auto trace = [&](const auto& stk) {
         if constexpr (MERGED)
             acc = dev::tracePixel<WALK>(S, gx, gy, spp, maxDepth, flags, rng, stk);
         else
             for (uint32_t k = 0; k < spp; ++k) acc += dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook);
-    } else {
-        const dev::LdsStack stk{s_stack + threadIdx.x, 64};
-        if constexpr (MERGED)
-            acc = dev::tracePixel<WALK>(S, gx, gy, spp, maxDepth, flags, rng, stk);
-        else
-            for (uint32_t k = 0; k < spp; ++k) acc += dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook);
-    }
+    };
+    if constexpr (WALK == dev::kWalkOrdered)
+        trace(dev::PairStack<LDS / 2, dev::kStackDepth / 2>{reinterpret_cast<uint2*>(s_stack) + threadIdx.x, 64,
+                                                            reinterpret_cast<uint2*>(spill) + lane, lanes});
+    else
+        trace(dev::LdsStack{s_stack + threadIdx.x, 64});
     reinterpret_cast<uint4*>(states)[pi] = make_uint4(rng.s0, rng.s1, rng.s2, rng.s3);
     float4 p = reinterpret_cast<float4*>(pixels)[pi];
     p.x += acc.x;
@@ -552,7 +550,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MERGED ? 4 :
     uint32_t* __restrict__ states, clr_float3* __restrict__ pixels, uint32_t* __restrict__ tileCounter,
     uint32_t* __restrict__ spill) {
     constexpr int kLds = WALK == dev::kWalkOrdered ? kMegaLds : dev::kStackDepth;
-    __shared__ uint32_t s_stack[kLds * 64];
+    __shared__ __align__(8) uint32_t s_stack[kLds * 64];
     renderTiles<WALK, kLds, MERGED>(scene, width, height, spp, maxDepth, flags, states, pixels, tileCounter, spill,
                                     s_stack);
 }
@@ -567,7 +565,7 @@ __global__ __launch_bounds__(64) void k_render_mega_few(dev::RScene scene, uint3
                                                         uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
                                                         uint32_t* __restrict__ tileCounter,
                                                         uint32_t* __restrict__ spill) {
-    __shared__ uint32_t s_stack[dev::kStackDepth * 64];
+    __shared__ __align__(8) uint32_t s_stack[dev::kStackDepth * 64];
     renderTiles<WALK, dev::kStackDepth, MERGED>(scene, width, height, spp, maxDepth, flags, states, pixels,
                                                 tileCounter, spill, s_stack);
 }
@@ -578,7 +576,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MERGED ? 4 :
     const dev::RScene* __restrict__ table, uint32_t numScenes, uint32_t width, uint32_t height, uint32_t spp,
     uint32_t maxDepth, uint32_t flags, uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
     uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill) {
-    __shared__ uint32_t s_stack[kMegaLds * 64];
+    __shared__ __align__(8) uint32_t s_stack[kMegaLds * 64];
     renderBatchTiles<dev::kWalkOrdered, kMegaLds, MERGED>(table, numScenes, width, height, spp, maxDepth, flags,
                                                           states, pixels, tileCounter, spill, s_stack);
 }
@@ -587,7 +585,7 @@ __global__ __launch_bounds__(64) void k_render_mega_batch_few(
     const dev::RScene* __restrict__ table, uint32_t numScenes, uint32_t width, uint32_t height, uint32_t spp,
     uint32_t maxDepth, uint32_t flags, uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
     uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill) {
-    __shared__ uint32_t s_stack[dev::kStackDepth * 64];
+    __shared__ __align__(8) uint32_t s_stack[dev::kStackDepth * 64];
     renderBatchTiles<dev::kWalkOrdered, dev::kStackDepth, MERGED>(table, numScenes, width, height, spp, maxDepth,
                                                                   flags, states, pixels, tileCounter, spill, s_stack);
 }
@@ -602,7 +600,7 @@ __global__ __launch_bounds__(64) void k_render_mega_batch_few(
 template <int WALK>
 __global__ __launch_bounds__(64) void k_bvh_visualizer(dev::RScene scene, uint32_t width, uint32_t height,
                                                        clr_float3* __restrict__ pixels) {
-    __shared__ uint32_t s_stack[dev::kStackDepth * 64];
+    __shared__ __align__(8) uint32_t s_stack[dev::kStackDepth * 64];
     dev::RScene S = scene;
     dev::finishScene(S);
     const uint32_t tilesX = (width + kTile - 1) / kTile;
@@ -617,8 +615,7 @@ __global__ __launch_bounds__(64) void k_bvh_visualizer(dev::RScene scene, uint32
     const dev::LdsStack stk{s_stack + threadIdx.x, 64};
     uint32_t face;
     if constexpr (WALK == dev::kWalkOrdered)
-        face = dev::orderedHit<true, false, dev::TexAlpha>(S.g, org, dir, t, stk, st, &b1, &b2, dev::TexAlpha{&S},
-                                                          &over);
+        face = dev::orderedHit(S.g, org, dir, t, stk, st, b1, b2, dev::TexAlpha{&S}, over);
     else if constexpr (WALK == dev::kWalkMidpoint)
         face = dev::bvhWalk<true, false>(S.g, org, dir, t, stk, st, &b1, &b2, dev::TexAlpha{&S}, &over);
     else
@@ -654,7 +651,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     uint32_t numMat, uint32_t lightProp, float* __restrict__ gAlb, float* __restrict__ gSig, float* __restrict__ gEm,
     uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill) {
     constexpr int kLds = WALK == dev::kWalkOrdered ? kAdjLds : dev::kStackDepth;
-    __shared__ uint32_t s_stack[kLds * 64];
+    __shared__ __align__(8) uint32_t s_stack[kLds * 64];
     __shared__ dev::AdjAcc s_acc;
     for (uint32_t i = threadIdx.x; i < dev::kMaxDiffMaterials * 3; i += 64) s_acc.alb[i] = 0.0f;
     for (uint32_t i = threadIdx.x; i < dev::kMaxDiffMaterials; i += 64) s_acc.sig[i] = 0.0f;
@@ -687,7 +684,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const float4 a = dLdI[pi];
         dev::AdjHook hook{S, table, lightProp, M, {a.x * inv, a.y * inv, a.z * inv}, &s_acc, 0};
         if constexpr (WALK == dev::kWalkOrdered) {
-            const dev::SpillStack<kLds> stk{s_stack + threadIdx.x, 64, spill + lane, lanes};
+            const dev::PairStack<kLds / 2, dev::kStackDepth / 2> stk{reinterpret_cast<uint2*>(s_stack) + threadIdx.x, 64,
+                                                                     reinterpret_cast<uint2*>(spill) + lane, lanes};
             for (uint32_t k = 0; k < spp; ++k) hook.finish(dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook));
         } else {
             const dev::LdsStack stk{s_stack + threadIdx.x, 64};
@@ -769,7 +767,7 @@ void launchResolveScenes(dev::RScene* table, uint32_t count, hipStream_t stream)
 // Scene.cpp:39-41) is read by the kernels themselves; the face->light map and
 // the first environment light are built on the stream. No host round trip, so
 // a render call can be captured into a graph.
-int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, hipStream_t stream) {
+int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, AccelKind kind, hipStream_t stream) {
     int rc = ensureRenderScratch(ctx, sd.numFaces);
     if (rc) return rc;
     rc = ensureStatus(ctx);
@@ -781,9 +779,12 @@ int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, hi
         k_face_lights_fill<<<(sd.numLights + 255) / 256, 256, 0, stream>>>(sd.lights, sd.numLights,
                                                                            sd.numFaces, faceLight, envLight);
     const float4 *anodes = nullptr, *atris = nullptr, *wnodes = nullptr;
-    rc = buildAccel(ctx, sd.internalNodes, sd.leafNodes, sd.bvhNodes, sd.numFaces, sd.vertices, sd.faces, &anodes,
-                    &atris, stream, &wnodes);
-    if (rc) return rc;
+    if (kind != AccelKind::kNone) {
+        rc = buildAccel(ctx, sd.internalNodes, sd.leafNodes, sd.bvhNodes, sd.numFaces, sd.vertices, sd.faces,
+                        kind == AccelKind::kBinary ? &anodes : nullptr, &atris, stream,
+                        kind == AccelKind::kWide ? &wnodes : nullptr);
+        if (rc) return rc;
+    }
     S.g = dev::GeomScene{sd.internalNodes, sd.leafNodes, sd.numFaces, sd.vertices, sd.faces, anodes, atris,
                          reinterpret_cast<const float4*>(sd.bvhNodes), wnodes};
     S.normals = sd.normals;
@@ -806,7 +807,7 @@ int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, hi
 int renderMegakernel(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_params& rp,
                      uint32_t* states, clr_float3* pixels, hipStream_t stream) {
     dev::RScene S;
-    int rc = prepareRenderScene(ctx, sd, S, stream);
+    int rc = prepareRenderScene(ctx, sd, S, accelFor(rp), stream);
     if (rc) return rc;
     const uint32_t tiles = ((rp.width + kTile - 1) / kTile) * ((rp.height + kTile - 1) / kTile);
     const uint32_t flags = rp.flags;
@@ -877,7 +878,8 @@ int renderMegakernelBatch(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t nu
 int renderBvhVisualizer(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_params& rp, clr_float3* pixels,
                         hipStream_t stream) {
     dev::RScene S;
-    int rc = prepareRenderScene(ctx, sd, S, stream);
+    const bool reference = (rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL) != 0;
+    int rc = prepareRenderScene(ctx, sd, S, reference ? AccelKind::kNone : AccelKind::kBinary, stream);
     if (rc) return rc;
     const uint32_t tiles = ((rp.width + kTile - 1) / kTile) * ((rp.height + kTile - 1) / kTile);
     if (!(rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL))
@@ -910,7 +912,7 @@ int renderAdjoint(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_params
     k_adj_clear<<<256, 256, 0, stream>>>(table, gAlb, gSig, gEm, dp.numMaterials);
     if (dp.numMaterials) k_adj_fill<<<1, 256, 0, stream>>>(table, offsets, dp.numMaterials);
     dev::RScene S;
-    rc = prepareRenderScene(ctx, sd, S, stream);
+    rc = prepareRenderScene(ctx, sd, S, accelFor(rp), stream);
     if (rc) return rc;
     const uint32_t tiles = ((rp.width + kTile - 1) / kTile) * ((rp.height + kTile - 1) / kTile);
     const uint32_t flags = rp.flags;

@@ -360,8 +360,7 @@ __device__ __forceinline__ bool intersect(const RScene& S, V3 org, V3 dir, const
     bool over = false;
     uint32_t face;
     if constexpr (WALK == kWalkOrdered)  // over the 4-wide records (every render builds them)
-        face = wideHit<false, false, TexAlpha, Stack, kStackDepth>(S.g, org, dir, t, stack, st, &b1, &b2,
-                                                                   TexAlpha{&S}, &over);
+        face = wideHit(S.g, org, dir, t, stack, b1, b2, TexAlpha{&S}, over);
     else if constexpr (WALK == kWalkMidpoint)
         face = bvhWalk<false, false>(S.g, org, dir, t, stack, st, &b1, &b2, TexAlpha{&S}, &over);
     else

@@ -53,13 +53,26 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_closest(
     }
 }
 
+// Triangle record of face i (see GeomScene): p0 | alpha flag, the two edges.
+__device__ __forceinline__ void storeTri(const clr_float3* __restrict__ verts, const clr_face* __restrict__ faces,
+                                         uint32_t i, float4* __restrict__ atris) {
+    const clr_face& f = faces[i];
+    const dev::V3 p0 = dev::loadV3(verts, f.p0), p1 = dev::loadV3(verts, f.p1), p2 = dev::loadV3(verts, f.p2);
+    const uint32_t flag = f.uv0 != dev::kNone && f.alphaTexPtr != dev::kNone ? 1u : 0u;
+    const dev::V3 e1 = p1 - p0, e2 = p2 - p0;
+    float4* o = atris + 3 * (size_t)i;
+    o[0] = make_float4(p0.x, p0.y, p0.z, __uint_as_float(flag));
+    o[1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
+    o[2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
+}
+
 // Traversal layout (see GeomScene): node i gets both children's boxes and
-// references, face f its three vertices.
+// references (unless anodes is null), face i its triangle record.
 __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves,
                               uint32_t n, const clr_float3* __restrict__ verts, const clr_face* __restrict__ faces,
                               float4* __restrict__ anodes, float4* __restrict__ atris) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i + 1 < n) {
+    if (anodes && i + 1 < n) {
         const uint4 c = reinterpret_cast<const uint4*>(inodes + i)[2];
         float4 box[2][2];
         uint32_t ref[2];
@@ -78,14 +91,7 @@ __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const c
         o[2] = make_float4(box[1][0].x, box[1][0].y, box[1][0].z, 0.0f);
         o[3] = make_float4(box[1][1].x, box[1][1].y, box[1][1].z, 0.0f);
     }
-    if (i < n) {
-        const uint32_t* f = reinterpret_cast<const uint32_t*>(faces + i);
-        float4* o = atris + 3 * (size_t)i;
-        for (int k = 0; k < 3; ++k) {
-            const float4 v = *reinterpret_cast<const float4*>(verts + f[k]);
-            o[k] = make_float4(v.x, v.y, v.z, 0.0f);
-        }
-    }
+    if (i < n) storeTri(verts, faces, i, atris);
 }
 
 // Traversal layout of a CPU midpoint BVH, indexed by node number: internal
@@ -97,7 +103,7 @@ __global__ void k_accel_build_bvh(const float4* __restrict__ bvh, uint32_t n, co
                                   float4* __restrict__ atris) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t numNodes = 2 * n - 1;
-    if (i < numNodes) {
+    if (anodes && i < numNodes) {
         const uint2 c = *reinterpret_cast<const uint2*>(bvh + 3 * (size_t)i + 2);
         if (c.y != kEmpty && c.x < numNodes && c.y < numNodes) {
             float4 box[2][2];
@@ -117,14 +123,7 @@ __global__ void k_accel_build_bvh(const float4* __restrict__ bvh, uint32_t n, co
             o[3] = make_float4(box[1][1].x, box[1][1].y, box[1][1].z, 0.0f);
         }
     }
-    if (i < n) {
-        const uint32_t* f = reinterpret_cast<const uint32_t*>(faces + i);
-        float4* o = atris + 3 * (size_t)i;
-        for (int k = 0; k < 3; ++k) {
-            const float4 v = *reinterpret_cast<const float4*>(verts + f[k]);
-            o[k] = make_float4(v.x, v.y, v.z, 0.0f);
-        }
-    }
+    if (i < n) storeTri(verts, faces, i, atris);
 }
 
 // 4-wide records (GeomScene::wnodes) of the LBVH: record i holds the
@@ -166,9 +165,15 @@ struct WideSlots {
 __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves,
                              uint32_t n, float4* __restrict__ wnodes) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i + 1 >= n) return;
     WideSlots w;
     w.clear();
+    if (n == 1 && i == 0) {  // a tree of one leaf: a record that holds it
+        const float4* p = reinterpret_cast<const float4*>(leaves);
+        w.put(0, p[0], p[1], leaves[0].objIdx | dev::kLeafRef);
+        w.store(wnodes);
+        return;
+    }
+    if (i + 1 >= n) return;
     const uint4 c = reinterpret_cast<const uint4*>(inodes + i)[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -202,9 +207,14 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
     const uint32_t numNodes = 2 * n - 1;
     if (i >= numNodes) return;
     const uint2 c = *reinterpret_cast<const uint2*>(bvh + 3 * (size_t)i + 2);
-    if (c.y == kEmpty || c.x >= numNodes || c.y >= numNodes) return;
     WideSlots w;
     w.clear();
+    if (n == 1 && c.y == kEmpty) {  // a tree of one leaf: a record that holds it
+        w.put(0, bvh[0], bvh[1], c.x | dev::kLeafRef);
+        w.store(wnodes);
+        return;
+    }
+    if (c.y == kEmpty || c.x >= numNodes || c.y >= numNodes) return;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const uint32_t ci = k ? c.y : c.x;
@@ -226,58 +236,39 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
     w.store(wnodes + 8 * (size_t)i);
 }
 
-// Ordered traversal, grid-stride over the rays with a fixed grid (waves per
-// CU x CUs). Each lane walks two rays at once, stepping them in turn, so one
-// ray's node fetch is in flight while the other's boxes and triangles are
-// tested (the walk is bound by dependent load latency). Each walker's stack
-// keeps kOrdLds / 2 slots in LDS ([slot][lane]) and the rest in its part of
-// `spill`.
+// Trace with the ordered traversal, grid-stride over the rays with a fixed
+// grid (waves per CU x CUs). Each lane walks two rays at once, stepping them in
+// turn, so one ray's node fetch is in flight while the other's boxes and
+// triangles are tested (the walk is bound by dependent load latency). Each
+// walker's stack keeps kOrdHalf slots in LDS ([slot][lane]) and the rest in
+// its part of `spill`.
 constexpr int kOrdLds = 32;
 constexpr int kOrdBlock = 128;
 constexpr int kOrdHalf = kOrdLds / 2;
 
-template <bool STATS, bool WIDE>
-__global__ __launch_bounds__(kOrdBlock) void k_trace_ordered(
-    const clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves, uint32_t n,
-    const clr_float3* __restrict__ verts, const clr_face* __restrict__ faces, const float* __restrict__ rays,
-    uint32_t numRays, uint32_t* __restrict__ hitFace, float* __restrict__ hitT, uint32_t* __restrict__ stats,
-    uint32_t* __restrict__ status, uint32_t* __restrict__ spill, const float4* __restrict__ anodes,
-    const float4* __restrict__ atris, const float4* __restrict__ bvh, const float4* __restrict__ wnodes) {
-    __shared__ uint32_t s_stack[kOrdLds * kOrdBlock];
-    const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
-    const uint32_t lanes = gridDim.x * kOrdBlock;
-    using S = dev::SpillStack<kOrdHalf>;
-    const S stk0{s_stack + threadIdx.x, kOrdBlock, spill + gid, lanes};
-    const S stk1{s_stack + kOrdHalf * kOrdBlock + threadIdx.x, kOrdBlock,
-                 spill + (size_t)(dev::kStackPairs - kOrdHalf) * lanes + gid, lanes};
-    const dev::GeomScene g{inodes, leaves, n, verts, faces, anodes, atris, bvh, wnodes};
-    using W = std::conditional_t<WIDE, dev::Wide<STATS, dev::NoAlpha, S, dev::kStackPairs>,
-                                 dev::Ordered<STATS, dev::NoAlpha, S, true>>;
-    W w0(g, stk0, dev::NoAlpha()), w1(g, stk1, dev::NoAlpha());
+// Walkers w0 and w1 over this lane's rays gid, gid + lanes, ...; done(w, r)
+// stores ray r's result.
+template <class W, class Done>
+__device__ __forceinline__ void traceTwo(W& w0, W& w1, const float* __restrict__ rays, uint32_t numRays, uint32_t gid,
+                                         uint32_t lanes, uint32_t* __restrict__ status, const Done& done) {
     const size_t R = numRays;
     bool over = false;
-    uint32_t next = gid, r0 = kEmpty, r1 = kEmpty;  // this lane's rays: gid, gid + lanes, ...
+    uint32_t next = gid, r0 = kEmpty, r1 = kEmpty;
     auto start = [&](W& w, uint32_t& r) {
         if (next < numRays) {
             r = next;
             next += lanes;
             const dev::V3 o = {rays[r], rays[R + r], rays[2 * R + r]};
             const dev::V3 d = {rays[3 * R + r], rays[4 * R + r], rays[5 * R + r]};
-            w.begin(o, d, rays[6 * R + r], false);
+            w.begin(o, d, rays[6 * R + r]);
         } else {
             r = kEmpty;
             w.done = true;
         }
     };
     auto finish = [&](const W& w, uint32_t r) {
-        const bool hit = w.best != kEmpty && !isinf(w.t);
-        hitFace[r] = hit ? w.best : kEmpty;
-        hitT[r] = w.t;
         if (w.over) over = true;
-        if constexpr (STATS) {
-            stats[2 * (size_t)r] = w.st.visits;
-            stats[2 * (size_t)r + 1] = w.st.tests;
-        }
+        done(w, r);
     };
     start(w0, r0);
     start(w1, r1);
@@ -300,6 +291,54 @@ __global__ __launch_bounds__(kOrdBlock) void k_trace_ordered(
     if (over) atomicOr(status, kStatusStackOverflow);
 }
 
+// With counts per ray: the walks whose visits and tests are defined.
+template <bool WIDE>
+__global__ __launch_bounds__(kOrdBlock) void k_trace_counts(
+    dev::GeomScene g, const float* __restrict__ rays, uint32_t numRays, uint32_t* __restrict__ hitFace,
+    float* __restrict__ hitT, uint32_t* __restrict__ stats, uint32_t* __restrict__ status,
+    uint32_t* __restrict__ spill) {
+    __shared__ uint32_t s_stack[kOrdLds * kOrdBlock];
+    const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
+    const uint32_t lanes = gridDim.x * kOrdBlock;
+    using S = dev::SpillStack<kOrdHalf>;
+    const S stk0{s_stack + threadIdx.x, kOrdBlock, spill + gid, lanes};
+    const S stk1{s_stack + kOrdHalf * kOrdBlock + threadIdx.x, kOrdBlock,
+                 spill + (size_t)(dev::kStackPairs - kOrdHalf) * lanes + gid, lanes};
+    using W = std::conditional_t<WIDE, dev::Wide<dev::NoAlpha, S, dev::kStackPairs>,
+                                 dev::Ordered<dev::NoAlpha, S, true>>;
+    W w0(g, stk0, dev::NoAlpha()), w1(g, stk1, dev::NoAlpha());
+    traceTwo(w0, w1, rays, numRays, gid, lanes, status, [&](const W& w, uint32_t r) {
+        const bool hit = w.best != kEmpty && !isinf(w.t);
+        hitFace[r] = hit ? w.best : kEmpty;
+        hitT[r] = w.t;
+        stats[2 * (size_t)r] = w.st.visits;
+        stats[2 * (size_t)r + 1] = w.st.tests;
+    });
+}
+
+// Without counts: WideWalk, whatever ordered walk the caller asked for (the
+// hit is the same).
+__global__ __launch_bounds__(kOrdBlock) void k_trace_wide(
+    dev::GeomScene g, const float* __restrict__ rays, uint32_t numRays, uint32_t* __restrict__ hitFace,
+    float* __restrict__ hitT, uint32_t* __restrict__ status, uint32_t* __restrict__ spill) {
+    constexpr int kPairs = kOrdHalf / 2;
+    __shared__ uint2 s_stack[2 * kPairs * kOrdBlock];
+    const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
+    const uint32_t lanes = gridDim.x * kOrdBlock;
+    using S = dev::PairStack<kPairs, dev::kStackPairs / 2>;
+    uint2* sp = reinterpret_cast<uint2*>(spill);
+    const S stk0{s_stack + threadIdx.x, kOrdBlock, sp + gid, lanes};
+    const S stk1{s_stack + kPairs * kOrdBlock + threadIdx.x, kOrdBlock, sp + (size_t)(S::CAP - kPairs) * lanes + gid,
+                 lanes};
+    using W = dev::WideWalk<dev::NoAlpha, S>;
+    W w0(g, stk0, dev::NoAlpha()), w1(g, stk1, dev::NoAlpha());
+    traceTwo(w0, w1, rays, numRays, gid, lanes, status, [&](const W& w, uint32_t r) {
+        const bool hit = w.best != kEmpty && !isinf(w.t);
+        hitFace[r] = hit ? w.best : kEmpty;
+        hitT[r] = w.t;
+    });
+}
+
 }  // namespace
 
 size_t accelNodeBytes(uint32_t n, bool midpoint) {
@@ -311,7 +350,6 @@ size_t accelWideBytes(uint32_t n, bool midpoint) { return 2 * accelNodeBytes(n, 
 
 void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
                      float4* wnodes, hipStream_t stream) {
-    if (n < 2) return;
     if (bvh)
         k_accel_wide_bvh<<<(2 * n - 1 + 255) / 256, 256, 0, stream>>>(reinterpret_cast<const float4*>(bvh), n,
                                                                        wnodes);
@@ -322,7 +360,7 @@ void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, 
 int buildAccel(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
                uint32_t n, const clr_float3* vertices, const clr_face* faces, const float4** anodes,
                const float4** atris, hipStream_t stream, const float4** wnodes) {
-    const size_t nodeBytes = accelNodeBytes(n, bvh != nullptr);
+    const size_t nodeBytes = anodes ? accelNodeBytes(n, bvh != nullptr) : 0;
     const size_t triBytes = ((size_t)n * 48 + 255) & ~size_t(255);
     const size_t need = nodeBytes + triBytes + (wnodes ? accelWideBytes(n, bvh != nullptr) : 0);
     if (ctx->accelBytes < need) {
@@ -338,10 +376,10 @@ int buildAccel(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* 
         }
         ctx->accelBytes = need;
     }
-    float4* an = static_cast<float4*>(ctx->accel);
+    float4* an = anodes ? static_cast<float4*>(ctx->accel) : nullptr;
     float4* at = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes);
     launchAccelBuild(inodes, leaves, bvh, n, vertices, faces, an, at, stream);
-    *anodes = an;
+    if (anodes) *anodes = an;
     *atris = at;
     if (wnodes) {
         float4* wn = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes + triBytes);
@@ -375,21 +413,21 @@ int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     const size_t lanes = (size_t)grid * kOrdBlock;
     rc = ensureTraceSpill(ctx, lanes * 2 * (dev::kStackPairs - kOrdHalf) * sizeof(uint32_t));
     if (rc) return rc;
+    const bool binary = stats && !wide;  // only the binary walk's counts need its records
     const float4 *anodes = nullptr, *atris = nullptr, *wnodes = nullptr;
-    rc = buildAccel(ctx, inodes, leaves, bvh, n, vertices, faces, &anodes, &atris, stream, wide ? &wnodes : nullptr);
+    rc = buildAccel(ctx, inodes, leaves, bvh, n, vertices, faces, binary ? &anodes : nullptr, &atris, stream,
+                    binary ? nullptr : &wnodes);
     if (rc) return rc;
-    const float4* b4 = reinterpret_cast<const float4*>(bvh);
-    auto launch = [&](auto kernel) {
-        kernel<<<grid, kOrdBlock, 0, stream>>>(inodes, leaves, n, vertices, faces, rays, numRays, hitFace, hitT, stats,
-                                               ctx->devStatus, ctx->traceSpill, anodes, atris, b4, wnodes);
-    };
-    if (wide) {
-        if (stats) launch(k_trace_ordered<true, true>);
-        else launch(k_trace_ordered<false, true>);
-    } else {
-        if (stats) launch(k_trace_ordered<true, false>);
-        else launch(k_trace_ordered<false, false>);
-    }
+    const dev::GeomScene g{inodes, leaves, n, vertices, faces, anodes, atris, reinterpret_cast<const float4*>(bvh),
+                           wnodes};
+    if (!stats)
+        k_trace_wide<<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, ctx->devStatus, ctx->traceSpill);
+    else if (wide)
+        k_trace_counts<true><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats, ctx->devStatus,
+                                                             ctx->traceSpill);
+    else
+        k_trace_counts<false><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats, ctx->devStatus,
+                                                              ctx->traceSpill);
     return hipCheck(ctx, hipGetLastError(), "trace launch");
 }
 

@@ -54,7 +54,7 @@ struct GeomScene {
     uint32_t n;
     const clr_float3* verts;
     const clr_face* faces;
-    const float4* anodes = nullptr;  // [n - 1][4] (LBVH) or [2n - 1][4] by node (midpoint BVH)
+    const float4* anodes = nullptr;  // [n - 1][4] (LBVH) or [2n - 1][4] by node (midpoint BVH); walks that count only
     const float4* atris = nullptr;   // [n][3]
     // CPU midpoint BVH (clr_bvh_node[2n - 1], 3 float4 each). When set, the
     // reference-order walks use it instead of inodes / leaves, and the
@@ -379,14 +379,15 @@ __device__ __forceinline__ float slabEnter(float4 mn, float4 mx, V3 o, V3 inv, f
     return e <= fminf(tmax, tBound) ? e : __builtin_nanf("");
 }
 
-// Moller-Trumbore on the packed triangle copy (same operations as triTest).
+// Moller-Trumbore on the packed triangle record {p0 | flag, p1 - p0, p2 - p0}
+// (same operations as triTest: the record holds the edges triTest forms).
+// `flag` is nonzero when the face has an alpha texture to look up.
 __device__ __forceinline__ bool triTestPacked(const float4* tris, V3 o, V3 d, uint32_t faceIdx, float& t,
-                                              float& b1Out, float& b2Out) {
+                                              float& b1Out, float& b2Out, uint32_t& flag) {
     const float4* tp = tris + 3 * (size_t)faceIdx;
     const float4 a = tp[0], b = tp[1], c = tp[2];
-    const V3 p0 = {a.x, a.y, a.z}, p1 = {b.x, b.y, b.z}, p2 = {c.x, c.y, c.z};
-    const V3 edge01 = p1 - p0;
-    const V3 edge02 = p2 - p0;
+    const V3 p0 = {a.x, a.y, a.z}, edge01 = {b.x, b.y, b.z}, edge02 = {c.x, c.y, c.z};
+    flag = __float_as_uint(a.w);
     const V3 p = cross(d, edge02);
     const float det = dot(edge01, p);
     if (det > -0.000001f && det < 0.000001f) return false;
@@ -405,14 +406,13 @@ __device__ __forceinline__ bool triTestPacked(const float4* tris, V3 o, V3 d, ui
     return true;
 }
 
-// Resumable ordered walk over the traversal layout: begin() sets up one ray,
+// Resumable counting walk over the binary traversal layout (callers that need
+// no counts use WideWalk): begin() sets up one ray, and
 // each step() either visits one internal node (both child boxes, its leaf
 // children's triangles nearer first, then enter the nearer internal child and
 // push the farther) or pops one candidate and re-tests its box against the
 // current t. Same decisions, hits and counts as a walk run to completion, so
 // callers can interleave rays (refill idle lanes) without changing results.
-// any (set by begin): stop at the first accepted triangle with a finite
-// distance (occlusion queries).
 // PAIRS (for stacks with a spill region of kStackPairs slots): the farther
 // child is pushed with its entry distance, and a visit that enters no child
 // pops at once, entering the first candidate whose entry is still <= t. That
@@ -421,39 +421,35 @@ __device__ __forceinline__ bool triTestPacked(const float4* tris, V3 o, V3 d, ui
 // visit / test counts are unchanged.
 constexpr int kStackPairs = 128;  // stack slots of a PAIRS walk: 64 (ref, entry) pairs
 
-template <bool STATS, class Alpha, class Stack, bool PAIRS = false>
+template <class Alpha, class Stack, bool PAIRS = false>
 struct Ordered {
-    GeomScene g;  // by value: rebind() switches scenes between rays
+    GeomScene g;
     const Stack& stack;
     Alpha alpha;
     V3 o, d, inv;
     float t, b1, b2;
     uint32_t best, node, steps;
     int depth;
-    bool done, over, any;
+    bool done, over;
     TraceStats st;
 
     __device__ __forceinline__ Ordered(const GeomScene& g_, const Stack& s_, const Alpha& a_)
         : g(g_), stack(s_), alpha(a_) {}
-    __device__ __forceinline__ void rebind(const GeomScene& g_, const Alpha& a_) {
-        g = g_;
-        alpha = a_;
-    }
 
     __device__ __forceinline__ void leaf(uint32_t face) {
-        if constexpr (STATS) ++st.tests;
+        ++st.tests;
         float tt = t, x1, x2;
-        if (!triTestPacked(g.atris, o, d, face, tt, x1, x2)) return;
+        uint32_t flag;
+        if (!triTestPacked(g.atris, o, d, face, tt, x1, x2, flag)) return;
         if (tt == t && face > best) return;
-        if (alpha.reject(face, x1, x2)) return;
+        if (flag && alpha.reject(face, x1, x2)) return;
         t = tt;
         best = face;
         b1 = x1;
         b2 = x2;
-        if (any && !isinf(tt)) done = true;
     }
 
-    __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax, bool anyHit = false) {
+    __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax) {
         o = o_;
         d = d_;
         inv = {safeInv(d.x), safeInv(d.y), safeInv(d.z)};
@@ -464,7 +460,6 @@ struct Ordered {
         depth = 0;
         done = false;
         over = false;
-        any = anyHit;
         steps = 0;
         st = {0u, 0u};
         if (g.n == 0) {
@@ -492,7 +487,7 @@ struct Ordered {
             return;
         }
         if (node != kNone) {
-            if constexpr (STATS) ++st.visits;
+            ++st.visits;
             const float4* np = g.anodes + 4 * (size_t)node;
             const float4 lo0 = np[0], hi0 = np[1], lo1 = np[2], hi1 = np[3];
             const uint32_t r0 = __float_as_uint(lo0.w), r1 = __float_as_uint(hi0.w);
@@ -504,8 +499,7 @@ struct Ordered {
                 const bool la = first1 ? l1 : l0, lb = first1 ? l0 : l1;
                 const float ea = first1 ? e1 : e0, eb = first1 ? e0 : e1;
                 if (la && ea <= t) leaf(ra & ~kLeafRef);
-                if (!done && lb && eb <= t) leaf(rb & ~kLeafRef);
-                if (done) return;
+                if (lb && eb <= t) leaf(rb & ~kLeafRef);
             }
             const bool go0 = !l0 && e0 <= t, go1 = !l1 && e1 <= t;
             if (go0 && go1) {
@@ -553,7 +547,9 @@ struct Ordered {
     }
 };
 
-// Ordered walk over the 4-wide records (GeomScene::wnodes): a visit loads
+// The counting walk over the 4-wide records (GeomScene::wnodes), whose
+// visits and tests are defined (clr_trace_closest_wide with counts; other
+// callers use WideWalk): a visit loads
 // one 128-byte record and tests up to four grandchildren boxes, so the chain
 // of dependent node loads is half the binary walk's. Leaf entries are tested
 // nearest first at the visit; internal entries within t continue with the
@@ -563,39 +559,35 @@ struct Ordered {
 // would test, and the accepted hit is the same (closest t, then the smaller
 // face index, alpha rejections as in the binary walk). CAP: stack slots (two
 // per entry); a push beyond them is dropped and flagged.
-template <bool STATS, class Alpha, class Stack, int CAP>
+template <class Alpha, class Stack, int CAP>
 struct Wide {
-    GeomScene g;  // by value: rebind() switches scenes between rays
+    GeomScene g;
     const Stack& stack;
     Alpha alpha;
     V3 o, d, inv;
     float t, b1, b2;
     uint32_t best, node, steps;
     int depth;
-    bool done, over, any;
+    bool done, over;
     TraceStats st;
 
     __device__ __forceinline__ Wide(const GeomScene& g_, const Stack& s_, const Alpha& a_)
         : g(g_), stack(s_), alpha(a_) {}
-    __device__ __forceinline__ void rebind(const GeomScene& g_, const Alpha& a_) {
-        g = g_;
-        alpha = a_;
-    }
 
     __device__ __forceinline__ void leaf(uint32_t face) {
-        if constexpr (STATS) ++st.tests;
+        ++st.tests;
         float tt = t, x1, x2;
-        if (!triTestPacked(g.atris, o, d, face, tt, x1, x2)) return;
+        uint32_t flag;
+        if (!triTestPacked(g.atris, o, d, face, tt, x1, x2, flag)) return;
         if (tt == t && face > best) return;
-        if (alpha.reject(face, x1, x2)) return;
+        if (flag && alpha.reject(face, x1, x2)) return;
         t = tt;
         best = face;
         b1 = x1;
         b2 = x2;
-        if (any && !isinf(tt)) done = true;
     }
 
-    __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax, bool anyHit = false) {
+    __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax) {
         o = o_;
         d = d_;
         inv = {safeInv(d.x), safeInv(d.y), safeInv(d.z)};
@@ -606,7 +598,6 @@ struct Wide {
         depth = 0;
         done = false;
         over = false;
-        any = anyHit;
         steps = 0;
         st = {0u, 0u};
         if (g.n == 0) {
@@ -630,7 +621,7 @@ struct Wide {
             over = true;
             return;
         }
-        if constexpr (STATS) ++st.visits;
+        ++st.visits;
         const float4* wp = g.wnodes + 8 * (size_t)node;
         const float4 lx = wp[0], ly = wp[1], lz = wp[2], hx = wp[3], hy = wp[4], hz = wp[5], rf = wp[6];
         float k[4] = {slabEnter(make_float4(lx.x, ly.x, lz.x, 0.0f), make_float4(hx.x, hy.x, hz.x, 0.0f), o, inv, t),
@@ -663,10 +654,7 @@ struct Wide {
         cx(1, 2);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (r[c] != kNone && (r[c] & kLeafRef) && k[c] <= t) {
-                leaf(r[c] & ~kLeafRef);
-                if (done) return;
-            }
+            if (r[c] != kNone && (r[c] & kLeafRef) && k[c] <= t) leaf(r[c] & ~kLeafRef);
         }
         uint32_t next = kNone;
         float enext = 0.0f;
@@ -705,36 +693,219 @@ struct Wide {
     }
 };
 
-// The 4-wide walk run to completion for one ray (as orderedHit).
-template <bool STATS, bool ANY, class Alpha = NoAlpha, class Stack = LdsStack, int CAP = kStackDepth>
-__device__ __forceinline__ uint32_t wideHit(const GeomScene& g, V3 o, V3 d, float& t, const Stack& stack,
-                                            TraceStats& st, float* b1Out = nullptr, float* b2Out = nullptr,
-                                            const Alpha& alpha = Alpha(), bool* overflow = nullptr) {
-    Wide<STATS, Alpha, Stack, CAP> w(g, stack, alpha);
-    w.begin(o, d, t, ANY);
+// Stack of (reference, entry distance) pairs: the first L pairs of a lane in
+// LDS ([pair][lane], one 8-byte access a pair, conflict-free at any mix of
+// depths), the others up to CAP in a per-lane global region.
+template <int L, int CAP_>
+struct PairStack {
+    static constexpr int CAP = CAP_;
+    uint2* lds;
+    int stride;
+    uint2* spill;
+    size_t spillStride;
+    __device__ __forceinline__ void put(int k, uint32_t ref, float entry) const {
+        const uint2 v = make_uint2(ref, __float_as_uint(entry));
+        if (L >= CAP || k < L) lds[k * stride] = v;
+        else spill[(size_t)(k - L) * spillStride] = v;
+    }
+    __device__ __forceinline__ uint2 get(int k) const {
+        return (L >= CAP || k < L) ? lds[k * stride] : spill[(size_t)(k - L) * spillStride];
+    }
+};
+
+// The walk over the 4-wide records that every renderer and every trace
+// without counts uses. It finds the hit of Ordered and Wide: the smallest
+// (t, face) over the accepted triangles, whatever boxes are entered on the
+// way, as long as none that holds an accepted triangle is passed over. That
+// leaves the box arithmetic free, and a visit is bound by its instructions
+// (few lanes are active, so every instruction counts in full):
+//   * near and far planes are loaded by the ray's direction signs (two planes
+//     an axis instead of four and a min and max each), and a plane's distance
+//     is one fma: t = plane * inv - o * inv. The cancellation error of that
+//     form, at most 2^-22 |o * inv|, is covered by moving the near planes'
+//     constant down and the far planes' up by 2^-21 |o * inv|; the relative
+//     pad of slabEnter (1 -+ 2^-16 on entry and exit) is one factor 1 - 2^-15
+//     on the entry. Every box that slabEnter admits is admitted; NaNs (from
+//     infinite products) are ignored by min / max and so admit.
+//   * leaf entries are tested in a loop over each lane's own leaves, so the
+//     triangle test runs as often as the lane with the most leaves has, not
+//     once for each of the four slots in which some lane has one;
+//   * internal entries are sorted as one word each (entry distance with its
+//     two lowest bits replaced by the slot: rounded down, so a pop never
+//     drops a candidate it should not).
+// begin() with `any` stops at the first accepted triangle of finite distance;
+// with a bound (tmax, bestFace) it accepts only triangles before it in (t,
+// face) order, so an any walk bounded by a light's own hit answers whether
+// that hit is the closest.
+// Stack: PairStack. Alpha: as in Ordered, asked only for flagged triangles.
+// Against the counting walk in the same kernels: 2^22 random rays on 2^24
+// triangles 8.72 -> 8.10 ms, 512x512 at 8 spp of the differentiation scene
+// 31.9 -> 26.3 ms (forward and adjoint), 640x360 at 16 spp of the showcase
+// scene on the wavefront renderer 24.3 -> 21.4 ms.
+template <class Alpha, class Stack>
+struct WideWalk {
+    const float4* wn;
+    const float4* tris;
+    uint32_t limit;  // more visits than this mean malformed records
+    const Stack& stack;
+    Alpha alpha;
+    V3 o, d, inv, cn, cf;  // near plane distance: plane * inv + cn; far: plane * inv + cf
+    uint32_t nx, ny, nz;   // float4 offset of the near planes in a record (far: 3, 5, 7 - it)
+    float t, b1, b2;
+    uint32_t best, node, steps;
+    int depth;
+    bool done, over, any;
+
+    __device__ __forceinline__ WideWalk(const GeomScene& g, const Stack& s_, const Alpha& a_)
+        : wn(g.wnodes), tris(g.atris), limit(2u * g.n + 2u), stack(s_), alpha(a_) {}
+    __device__ __forceinline__ void rebind(const GeomScene& g, const Alpha& a_) {
+        wn = g.wnodes;
+        tris = g.atris;
+        limit = 2u * g.n + 2u;
+        alpha = a_;
+    }
+
+    __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax, bool anyHit = false, uint32_t bestFace = kNone) {
+        o = o_;
+        d = d_;
+        auto recip = [](float v) { return __builtin_amdgcn_rcpf(fabsf(v) > 1e-20f ? v : copysignf(1e-20f, v)); };
+        inv = {recip(d.x), recip(d.y), recip(d.z)};
+        constexpr float kSlack = 1.0f / 2097152.0f;
+        const V3 oi = {o.x * inv.x, o.y * inv.y, o.z * inv.z};
+        cn = {-oi.x - fabsf(oi.x) * kSlack, -oi.y - fabsf(oi.y) * kSlack, -oi.z - fabsf(oi.z) * kSlack};
+        cf = {-oi.x + fabsf(oi.x) * kSlack, -oi.y + fabsf(oi.y) * kSlack, -oi.z + fabsf(oi.z) * kSlack};
+        nx = inv.x < 0.0f ? 3u : 0u;
+        ny = inv.y < 0.0f ? 4u : 1u;
+        nz = inv.z < 0.0f ? 5u : 2u;
+        t = tmax;
+        b1 = b2 = 0.0f;
+        best = bestFace;
+        node = 0;
+        steps = 0;
+        depth = 0;
+        done = false;
+        over = false;
+        any = anyHit;
+    }
+
+    __device__ __forceinline__ void leaf(uint32_t face) {
+        float tt = t, x1, x2;
+        uint32_t flag;
+        if (!triTestPacked(tris, o, d, face, tt, x1, x2, flag)) return;
+        if (tt == t && face >= best) return;
+        if (flag && alpha.reject(face, x1, x2)) return;
+        t = tt;
+        best = face;
+        b1 = x1;
+        b2 = x2;
+        if (any && !isinf(tt)) done = true;
+    }
+
+    static __device__ __forceinline__ uint32_t pick(const uint4& r, uint32_t slot) {
+        const uint32_t lo = (slot & 1u) ? r.y : r.x, hi = (slot & 1u) ? r.w : r.z;
+        return (slot & 2u) ? hi : lo;
+    }
+
+    __device__ __forceinline__ void step() {
+        if (++steps > limit) {
+            done = true;
+            over = true;
+            return;
+        }
+        const float4* wp = wn + 8 * (size_t)node;
+        const float4 ax = wp[nx], ay = wp[ny], az = wp[nz];
+        const float4 bx = wp[3u - nx], by = wp[5u - ny], bz = wp[7u - nz];
+        const uint4 r = reinterpret_cast<const uint4*>(wp)[6];
+        uint32_t leaves = 0;
+        auto entry = [&](float px, float py, float pz, float qx, float qy, float qz, uint32_t ref, uint32_t slot) {
+            const float tn = fmaxf(fmaxf(__builtin_fmaf(px, inv.x, cn.x), __builtin_fmaf(py, inv.y, cn.y)),
+                                   fmaxf(__builtin_fmaf(pz, inv.z, cn.z), 0.0f)) *
+                             (1.0f - 1.0f / 32768.0f);
+            const float tf = fminf(fminf(__builtin_fmaf(qx, inv.x, cf.x), __builtin_fmaf(qy, inv.y, cf.y)),
+                                   __builtin_fmaf(qz, inv.z, cf.z));
+            const bool pass = tn <= tf && tn <= t && ref != kNone;
+            const bool leafRef = (ref & kLeafRef) != 0;
+            if (pass && leafRef) leaves |= 1u << slot;
+            return pass && !leafRef ? ((__float_as_uint(tn) & ~3u) | slot) : 0xFFFFFFFFu;
+        };
+        uint32_t k0 = entry(ax.x, ay.x, az.x, bx.x, by.x, bz.x, r.x, 0u);
+        uint32_t k1 = entry(ax.y, ay.y, az.y, bx.y, by.y, bz.y, r.y, 1u);
+        uint32_t k2 = entry(ax.z, ay.z, az.z, bx.z, by.z, bz.z, r.z, 2u);
+        uint32_t k3 = entry(ax.w, ay.w, az.w, bx.w, by.w, bz.w, r.w, 3u);
+        while (leaves) {
+            const uint32_t slot = (uint32_t)__builtin_ctz(leaves);
+            leaves &= leaves - 1u;
+            leaf(pick(r, slot) & ~kLeafRef);
+            if (done) return;
+        }
+        auto cx = [](uint32_t& a, uint32_t& b) {
+            const uint32_t lo = min(a, b);
+            b = max(a, b);
+            a = lo;
+        };
+        cx(k0, k1);
+        cx(k2, k3);
+        cx(k0, k2);
+        cx(k1, k3);
+        cx(k1, k2);
+        // Entries beyond a hit of this visit's own leaves stay (sorted last,
+        // dropped at their pop); 0xFFFFFFFF is a NaN and fails every compare.
+        if (k1 != 0xFFFFFFFFu) {
+            if (k2 != 0xFFFFFFFFu) {
+                if (k3 != 0xFFFFFFFFu) push(pick(r, k3 & 3u), __uint_as_float(k3));
+                push(pick(r, k2 & 3u), __uint_as_float(k2));
+            }
+            push(pick(r, k1 & 3u), __uint_as_float(k1));
+        }
+        if (__uint_as_float(k0) <= t) {
+            node = pick(r, k0 & 3u);
+            return;
+        }
+        while (depth > 0) {
+            const uint2 c = stack.get(--depth);
+            if (__uint_as_float(c.y) <= t) {
+                node = c.x;
+                return;
+            }
+        }
+        done = true;
+    }
+
+    __device__ __forceinline__ void push(uint32_t ref, float e) {
+        if (depth < Stack::CAP) stack.put(depth++, ref, e);
+        else over = true;
+    }
+};
+
+// The walk run to completion for one ray. Returns the face (kNone when
+// nothing was accepted) and updates t, b1, b2.
+template <class Alpha, class Stack>
+__device__ __forceinline__ uint32_t wideHit(const GeomScene& g, V3 o, V3 d, float& t, const Stack& stack, float& b1,
+                                            float& b2, const Alpha& alpha, bool& overflow) {
+    WideWalk<Alpha, Stack> w(g, stack, alpha);
+    w.begin(o, d, t);
     while (!w.done) w.step();
     t = w.t;
-    if (b1Out) *b1Out = w.b1;
-    if (b2Out) *b2Out = w.b2;
-    if (overflow && w.over) *overflow = true;
-    if constexpr (STATS) st = w.st;
+    b1 = w.b1;
+    b2 = w.b2;
+    if (w.over) overflow = true;
     return w.best;
 }
 
-// The ordered walk run to completion for one ray. Returns the face (kNone
-// when nothing was accepted) and updates t, b1, b2.
-template <bool STATS, bool ANY, class Alpha = NoAlpha, class Stack = LdsStack, bool PAIRS = false>
+// The binary ordered walk run to completion for one ray. Returns the face
+// (kNone when nothing was accepted), updates t, b1, b2 and sets the counts.
+template <class Alpha, class Stack>
 __device__ __forceinline__ uint32_t orderedHit(const GeomScene& g, V3 o, V3 d, float& t, const Stack& stack,
-                                               TraceStats& st, float* b1Out = nullptr, float* b2Out = nullptr,
-                                               const Alpha& alpha = Alpha(), bool* overflow = nullptr) {
-    Ordered<STATS, Alpha, Stack, PAIRS> w(g, stack, alpha);
-    w.begin(o, d, t, ANY);
+                                               TraceStats& st, float& b1, float& b2, const Alpha& alpha,
+                                               bool& overflow) {
+    Ordered<Alpha, Stack> w(g, stack, alpha);
+    w.begin(o, d, t);
     while (!w.done) w.step();
     t = w.t;
-    if (b1Out) *b1Out = w.b1;
-    if (b2Out) *b2Out = w.b2;
-    if (overflow && w.over) *overflow = true;
-    if constexpr (STATS) st = w.st;
+    b1 = w.b1;
+    b2 = w.b2;
+    if (w.over) overflow = true;
+    st = w.st;
     return w.best;
 }
 

@@ -38,8 +38,6 @@
 
 namespace clr {
 
-int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, hipStream_t stream);
-
 namespace {
 
 using namespace dev;
@@ -318,7 +316,7 @@ __global__ void k_wf_init(WfArgs A, uint32_t chunk, uint32_t count, uint32_t spp
 // shadow kernels of this iteration append to.
 template <bool ORDERED, int LD, bool BATCH, int K = 1>
 __global__ __launch_bounds__(256) void k_wf_extend(WfArgs A, uint32_t in) {
-    extern __shared__ uint32_t s_stack[];
+    extern __shared__ __align__(8) uint32_t s_stack[];
     const WfBufs& B = A.B;
     const RScene S = A.S;
     const uint32_t chunk = B.counts[kCntChunk];
@@ -338,10 +336,14 @@ __global__ __launch_bounds__(256) void k_wf_extend(WfArgs A, uint32_t in) {
         // rays at once, stepping them in turn, so that one ray's node fetch
         // overlaps the other's tests; each walker has its own stack.
         const RScene* S0 = firstScene<BATCH>(A, S);
-        const SpillStack<LD> stk1{s_stack + LD * blockDim.x + threadIdx.x, (int)blockDim.x,
-                                  B.spill + (size_t)(kStackPairs - kMinLdsDepth) * lanes + gid, lanes};
-        using W = Wide<false, TexAlpha, SpillStack<LD>, kStackPairs>;
-        W w0(S0->g, stk, TexAlpha{S0}), w1(S0->g, stk1, TexAlpha{S0});
+        using PS = PairStack<LD / 2, kStackPairs / 2>;
+        uint2* const lds = reinterpret_cast<uint2*>(s_stack) + threadIdx.x;
+        uint2* const spill = reinterpret_cast<uint2*>(B.spill) + gid;
+        const PS stk0{lds, (int)blockDim.x, spill, lanes};
+        const PS stk1{lds + LD / 2 * blockDim.x, (int)blockDim.x,
+                      spill + (size_t)(kStackPairs - kMinLdsDepth) / 2 * lanes, lanes};
+        using W = WideWalk<TexAlpha, PS>;
+        W w0(S0->g, stk0, TexAlpha{S0}), w1(S0->g, stk1, TexAlpha{S0});
         WavePool pool(n);
         bool busy0 = false, busy1 = false;
         uint32_t j0 = 0, j1 = 0;
@@ -594,7 +596,7 @@ __global__ __launch_bounds__(256) void k_wf_shadow(WfArgs A, uint32_t in) {
     RScene S = A.S;
     if (!BATCH) finishScene(S);
     const uint32_t chunk = A.B.counts[kCntChunk];
-    extern __shared__ uint32_t s_stack[];
+    extern __shared__ __align__(8) uint32_t s_stack[];
     const WfBufs& B = A.B;
     const uint32_t out = in ^ 1u;
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -613,10 +615,14 @@ __global__ __launch_bounds__(256) void k_wf_shadow(WfArgs A, uint32_t in) {
         // K walkers per lane, as in k_wf_extend (a path slot has at most one
         // shadow ray per iteration, so the pixel updates never collide).
         const RScene* S0 = firstScene<BATCH>(A, S);
-        const SpillStack<LD> stk1{s_stack + LD * blockDim.x + threadIdx.x, (int)blockDim.x,
-                                  B.spill + (size_t)(kStackPairs - kMinLdsDepth) * lanes + gid, lanes};
-        using W = Wide<false, TexAlpha, SpillStack<LD>, kStackPairs>;
-        W w0(S0->g, stk, TexAlpha{S0}), w1(S0->g, stk1, TexAlpha{S0});
+        using PS = PairStack<LD / 2, kStackPairs / 2>;
+        uint2* const lds = reinterpret_cast<uint2*>(s_stack) + threadIdx.x;
+        uint2* const spill = reinterpret_cast<uint2*>(B.spill) + gid;
+        const PS stk0{lds, (int)blockDim.x, spill, lanes};
+        const PS stk1{lds + LD / 2 * blockDim.x, (int)blockDim.x,
+                      spill + (size_t)(kStackPairs - kMinLdsDepth) / 2 * lanes, lanes};
+        using W = WideWalk<TexAlpha, PS>;
+        W w0(S0->g, stk0, TexAlpha{S0}), w1(S0->g, stk1, TexAlpha{S0});
         WavePool pool(n);
         bool busy0 = false, busy1 = false;
         uint32_t i0 = 0, i1 = 0, target0 = kNone, target1 = kNone;
@@ -1077,7 +1083,7 @@ int renderWavefront(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_para
     WfState& w = *ctx->wf;
     WfArgs A;
     std::memset(&A, 0, sizeof(A));  // padding too: the graph cache compares the bytes
-    rc = prepareRenderScene(ctx, sd, A.S, stream);
+    rc = prepareRenderScene(ctx, sd, A.S, accelFor(rp), stream);
     if (rc) return rc;
     // Tile-major positions: whole 8x8 tiles, edge-tile positions outside the
     // image are skipped by k_wf_init.
@@ -1107,8 +1113,7 @@ int prepareBatchScenes(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t numSc
     size_t bytes = align(sizeof(RScene) * numScenes) + align(sizeof(int) * numScenes);
     for (uint32_t s = 0; s < numScenes; ++s) {
         const uint32_t n = scenes[s].numFaces;
-        bytes += accelNodeBytes(n, scenes[s].bvhNodes != nullptr) + accelWideBytes(n, scenes[s].bvhNodes != nullptr) +
-                 align(48ull * n) + align(4ull * n);
+        bytes += accelWideBytes(n, scenes[s].bvhNodes != nullptr) + align(48ull * n) + align(4ull * n);
     }
     if (ctx->batchBytes < bytes) {
         bool capturing = false;
@@ -1135,32 +1140,28 @@ int prepareBatchScenes(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t numSc
     int* envWords = c.take<int>(numScenes);
     std::vector<RScene> table(numScenes);
     // Per-scene arrays grouped by kind: every scene's 4-wide records, then
-    // every scene's triangle records, binary records and face-light words.
-    // The walks read the first two kinds of all scenes at once. Packed
-    // together, away from the binary records that the renderers' walk does
-    // not read, they span fewer pages: on the 256-scene batch the traversal
-    // kernels' L1 address-translation misses fell from 25 % to 3 % of
-    // requests, and the render took a third less time than with each scene's
-    // arrays side by side.
-    std::vector<float4*> wns(numScenes), ats(numScenes), ans(numScenes);
+    // every scene's triangle records and face-light words. The walks read the
+    // first two kinds of all scenes at once. Packed together they span fewer
+    // pages: on the 256-scene batch the traversal kernels' L1
+    // address-translation misses fell from 25 % to 3 % of requests, and the
+    // render took a third less time than with each scene's arrays side by side.
+    std::vector<float4*> wns(numScenes), ats(numScenes);
     std::vector<uint32_t*> fls(numScenes);
     for (uint32_t s = 0; s < numScenes; ++s)
         wns[s] = c.take<float4>(accelWideBytes(scenes[s].numFaces, scenes[s].bvhNodes != nullptr) / sizeof(float4));
     for (uint32_t s = 0; s < numScenes; ++s) ats[s] = c.take<float4>(3ull * scenes[s].numFaces);
-    for (uint32_t s = 0; s < numScenes; ++s)
-        ans[s] = c.take<float4>(accelNodeBytes(scenes[s].numFaces, scenes[s].bvhNodes != nullptr) / sizeof(float4));
     for (uint32_t s = 0; s < numScenes; ++s) fls[s] = c.take<uint32_t>(scenes[s].numFaces);
     for (uint32_t s = 0; s < numScenes; ++s) {
         const clr_scene_dev& sd = scenes[s];
         const uint32_t n = sd.numFaces;
-        float4 *an = ans[s], *wn = wns[s], *at = ats[s];
+        float4 *wn = wns[s], *at = ats[s];
         uint32_t* fl = fls[s];
-        launchAccelBuild(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, sd.vertices, sd.faces, an, at, stream);
+        launchAccelBuild(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, sd.vertices, sd.faces, nullptr, at, stream);
         launchAccelWide(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, wn, stream);
         launchFaceLights(sd.lights, sd.numLights, n, fl, envWords + s, stream);
         RScene& S = table[s];
         std::memset(&S, 0, sizeof(S));
-        S.g = GeomScene{sd.internalNodes, sd.leafNodes, n, sd.vertices, sd.faces, an, at,
+        S.g = GeomScene{sd.internalNodes, sd.leafNodes, n, sd.vertices, sd.faces, nullptr, at,
                         reinterpret_cast<const float4*>(sd.bvhNodes), wn};
         S.normals = sd.normals;
         S.tangents = sd.tangents;
