@@ -12,6 +12,7 @@ namespace clr {
 struct WfState;
 namespace dev {
 struct RScene;
+struct GeomScene;
 }
 }
 
@@ -154,11 +155,11 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
 
 // ---- rendering (render.hip, wavefront.hip) ----
 // The traversal layout a call needs: none (the reference walks read the
-// drop-in nodes), the binary records (the visualiser's counting walk), or the
-// 4-wide records (every other walk).
-enum class AccelKind { kNone, kBinary, kWide };
+// drop-in nodes), the binary or the 4-wide float records (the counting
+// walks), or the 4-wide byte records (every other walk).
+enum class AccelKind { kNone, kBinary, kWide, kBytes };
 inline AccelKind accelFor(const clr_render_params& rp) {
-    return (rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL) ? AccelKind::kNone : AccelKind::kWide;
+    return (rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL) ? AccelKind::kNone : AccelKind::kBytes;
 }
 int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, AccelKind kind, hipStream_t stream);
 int ensureRenderScratch(clr_ctx* ctx, uint32_t numFaces);
@@ -201,19 +202,17 @@ void launchAccelBuild(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves,
                       hipStream_t stream);
 // Bytes of the traversal layout's node array (256-B aligned).
 size_t accelNodeBytes(uint32_t n, bool midpoint);
-// The renderers' 4-wide records (128 B per node slot) and their build.
-size_t accelWideBytes(uint32_t n, bool midpoint);
-void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
-                     float4* wnodes, hipStream_t stream);
+// The 4-wide byte records (64 B per node slot) and their build.
+size_t accelByteBytes(uint32_t n, bool midpoint);
+void launchAccelBytes(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
+                      float4* qnodes, hipStream_t stream);
 // Face -> first light map and first environment light of one scene.
 void launchFaceLights(const clr_light_info* lights, uint32_t numLights, uint32_t numFaces, uint32_t* faceLight,
                       int* envLight, hipStream_t stream);
-// Builds the ordered traversal's layout from the drop-in nodes on `stream`
-// into context memory: the triangle records, with `anodes` the binary node
-// records, with `wnodes` the 4-wide records.
-int buildAccel(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
-               uint32_t n, const clr_float3* vertices, const clr_face* faces, const float4** anodes,
-               const float4** atris, hipStream_t stream, const float4** wnodes = nullptr);
+// Builds the traversal layout `kind` of the scene's geometry on `stream` into
+// context memory (the triangle records, and the node records of that kind)
+// and returns the geometry view with it.
+int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomScene& g, hipStream_t stream);
 int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
                  uint32_t n, const clr_float3* vertices, const clr_face* faces, const float* rays, uint32_t numRays,
                  uint32_t* hitFace, float* hitT, uint32_t* stats, hipStream_t stream, bool wide = false);

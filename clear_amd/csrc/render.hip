@@ -150,162 +150,257 @@ __device__ V3 tracePath(const RScene& S, uint32_t gx, uint32_t gy, uint32_t maxD
     return pix;
 }
 
-// All spp camera paths of pixel (gx, gy), summed: the same terms, in the same
-// order and from the same random numbers as spp calls of tracePath, so the
-// result is bit-identical. The two loops of those calls (samples, and bounces
-// within a path) are merged into one: a lane whose path ends starts its next
-// sample at once, and every pass of the loop traces exactly one ray per active
-// lane (camera, shadow or extension) at one call site. A wave then runs as
-// long as its lanes' longest sum of paths rather than the sum of its longest
-// paths, and its traversals keep their lanes busy.
-template <int WALK, class Stack>
-__device__ V3 tracePixel(const RScene& S, uint32_t gx, uint32_t gy, uint32_t spp, uint32_t maxDepth,
-                         uint32_t flags, Rng& rng, const Stack& stack) {
-    const bool noRR = (flags & CLR_RENDER_NO_RR) != 0;
-    V3 acc = v3z();
-    if (spp == 0) return acc;
-    uint32_t k = 0;
-    // path state
-    V3 pix, alpha, org, dir, vout = v3z();
-    float initY, dirPDF;
-    uint32_t sampledType, depth;
-    bool first, shadow;
-    SurfPt sp;
-    BSDF B;
-    EDF E;
-    clr_face F;
-    // pending light sample: while `shadow`, org and dir hold the shadow ray
-    // (dir = vinL); the extension ray's are not needed again after it
-    SurfPt lp;
-    bool atInf = false;
-    float lightPDF = 0.0f, dist2 = 0.0f;
-
-    auto startSample = [&]() {
-        float w;
-        cameraRay(S, gx, gy, rng, org, dir, w, dirPDF);
-        alpha = v3s(1.0f) * w;
-        initY = lum(alpha);
-        pix = v3z();
-        sampledType = 0;
-        depth = 0;
-        first = true;
-        shadow = false;
-    };
-    // The path ends; envTerm: it left the scene (tracePath's traceContinue).
-    auto finishSample = [&](bool envTerm) {
-        if (envTerm) {
-            vout = -dir;
-            const float theta = acosf(clampf(dir.y, -1.0f, 1.0f));
-            const float phi = fmodf(atan2f(-dir.x, dir.z) + 2.0f * kPiF, 2 * kPiF);
-            const float u = phi / (2.0f * kPiF), v = theta / kPiF;
-            edfEnv(S, u, v, E);
-            float mis = 1.0f;
-            if ((sampledType & kNonSingular) != 0 && depth > 0) {
-                const float lightPDF = areaPdfEnv(S, u, v) * 1.0f / absCosEDF(E, vout);
-                mis = emissionHitMis(flags, dirPDF, lightPDF);
-            }
-            pix += (mis * alpha) * evalLe(E, vout);
-        }
-        acc += pix;
-        if (++k < spp) startSample();
-    };
-    // BSDF sample at sp: the next extension ray, or the end of the path.
-    auto sampleBounce = [&]() {
-        const float bc = rng.uniform(), b0 = rng.uniform(), b1 = rng.uniform();
-        V3 nd = v3z();
-        const V3 f = sampleFs(B, vout, bc, b0, b1, nd, dirPDF, sampledType);
-        if ((f.x == 0.0f && f.y == 0.0f && f.z == 0.0f) || dirPDF == 0.0f) {
-            finishSample(false);
-            return;
-        }
-        alpha = alpha * (f * (fabsf(dot(B.N, nd)) / dirPDF));
-        dir = nd;
-        org = sp.p + dir * kRayEps;
-        ++depth;
-        shadow = false;
-    };
-
-    startSample();
-    while (k < spp) {
-        SurfPt hsp;
-        const bool hit = intersect<WALK>(S, org, dir, stack, hsp);
-        if (shadow) {
-            const V3 vinL = dir;
-            const bool visible = atInf ? !hit : (hit && hsp.face == lp.face);
-            // A zero or infinite light density (an environment sample at a
-            // pole, where sin(theta) = 0) contributes nothing.
-            if (visible && lightPDF > 0.0f && lightPDF < INFINITY) {
-                const V3 vinLrev = -vinL;
-                const float fsPDF = evalFsPdf(B, vout, vinL) * absCosEDF(E, vinL) / dist2;
-                const float mis = lightSampleMis(flags, lightPDF, fsPDF);
-                const float wgt = mis * absCosEDF(E, vinL) * fabsf(dot(B.N, vinL)) / dist2 / lightPDF;
-                const V3 term = wgt * ((alpha * evalLe(E, vinLrev)) * evalFs(B, vout, vinL));
-                pix += term;
-            }
-            sampleBounce();
-            continue;
-        }
-        if (!hit) {
-            finishSample(true);
-            continue;
-        }
-        sp = hsp;
-        F = S.g.faces[sp.face];
-        vout = -dir;
-        if (F.lightPtr != 0xFFFFu) {
-            edfArea(S, F.lightPtr, sp, sp.u, sp.v, E);
-            if (first) {
-                pix += alpha * evalLe(E, vout);
-            } else {
-                float mis = 1.0f;
-                if (sampledType & kNonSingular) {
-                    const V3 dd = sp.p - org;
-                    const float d2 = dd.x * dd.x + dd.y * dd.y + dd.z * dd.z;
-                    const float lightPDF = areaPdfOfFace(S, sp.face) * d2 / absCosEDF(E, vout);
-                    mis = emissionHitMis(flags, dirPDF, lightPDF);
-                }
-                pix += (mis * alpha) * evalLe(E, vout);
-            }
-        }
-        if (!first) {
-            if (depth >= maxDepth) {
-                finishSample(false);
-                continue;
-            }
-            if (!noRR) {
-                const float cp = fminf(lum(alpha) * (1.0f / initY), 1.0f);
-                if (rng.uniform() < cp) {
-                    alpha = alpha * (1.0f / cp);
-                    dirPDF *= cp;
-                } else {
-                    finishSample(false);
-                    continue;
-                }
-            }
-        }
-        first = false;
-        bsdfAlloc(S, F.matPtr, sp, B);
-        if (hasNonSpecular(B)) {
-            const float lu = rng.uniform(), l0 = rng.uniform(), l1 = rng.uniform();
-            // With BSDF samples alone the light sample is skipped (its numbers are drawn).
-            if (!(flags & CLR_RENDER_BSDF_SAMPLING_ONLY)) {
-                sampleLight(S, lu, l0, l1, lp, atInf, E, lightPDF);
-                V3 vinL = lp.p - sp.p;
-                dist2 = dot(vinL, vinL);
-                vinL = vinL * (1.0f / sqrtf(dist2));
-                if (atInf) {
-                    vinL = lp.p;
-                    dist2 = 1.0f;
-                }
-                org = sp.p + vinL * kRayEps;
-                dir = vinL;
-                shadow = true;
-                continue;
-            }
-        }
-        sampleBounce();
+// Pixels of an image as jobs of tracePixels: states advance, radiance adds up.
+struct ImageJob {
+    uint4* states;
+    float4* pixels;
+    uint32_t width;
+    __device__ __forceinline__ void load(uint32_t gx, uint32_t gy, Rng& rng) const {
+        const uint4 st = states[(size_t)gy * width + gx];
+        rng = {st.x, st.y, st.z, st.w};
     }
-    return acc;
+    __device__ __forceinline__ void store(uint32_t gx, uint32_t gy, const Rng& rng, V3 acc) const {
+        const size_t pi = (size_t)gy * width + gx;
+        states[pi] = make_uint4(rng.s0, rng.s1, rng.s2, rng.s3);
+        float4 p = pixels[pi];
+        p.x += acc.x;
+        p.y += acc.y;
+        p.z += acc.z;
+        pixels[pi] = p;
+    }
+    __device__ __forceinline__ bool unseen(V3 c) const { return c.x == 0.0f && c.y == 0.0f && c.z == 0.0f; }
+    __device__ __forceinline__ void emission(V3, uint32_t) const {}
+    __device__ __forceinline__ void lightSample(uint32_t, uint32_t, const BSDF&, V3, V3, const SurfPt&) const {}
+    __device__ __forceinline__ void lightSeen(V3, V3) const {}
+    __device__ __forceinline__ void bounce(uint32_t, const BSDF&, V3, V3, const SurfPt&, V3) const {}
+    __device__ __forceinline__ void finish(V3) const {}
+};
+
+// The megakernel's and the adjoint's schedule for the ordered traversal: a wave
+// traces the pixels that `src` hands to its lanes, each lane all samples of one
+// pixel after the other (the terms, their order and the random numbers of
+// tracePath, so images and states are bit-identical), and every lane one ray at
+// a time: a camera or extension ray, or a light sample's shadow ray. A lane
+// whose ray is finished waits until kServeMin lanes wait (or none walks); they
+// are then served together: shaded, given their next ray, next sample or next
+// pixel. Serving all lanes only when the last one has finished its ray keeps
+// lanes idle for as long as the longest walk (17.5 % of VALU lanes active);
+// serving each at once would run the shading code for a lane or two at a time.
+//
+// A vertex is shaded at once: its light sample's weighted contribution and its
+// BSDF sample are computed before the shadow ray is cast (their random numbers
+// come in that order), so across a walk a lane keeps two rays and a colour
+// instead of the BSDF and both surface points. A contribution of exactly zero
+// casts no shadow ray. A shadow ray only asks whether the light is seen: an
+// environment sample stops at the first hit, an area sample first tests the
+// light's own triangle and then stops at the first hit before it in (t, face)
+// order, the order in which the closest hit is defined.
+// JOB: loads and stores a pixel, and observes the path's radiance terms
+// (nothing for images, derivatives for the adjoint).
+constexpr uint32_t kServeMin = 56;
+
+template <class Job, class Stack, class Source>
+__device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint32_t maxDepth, uint32_t flags,
+                                            const Stack& stack, Job& job, Source& src) {
+    const bool noRR = (flags & CLR_RENDER_NO_RR) != 0;
+    WideWalk<TexAlpha, Stack> w(S.g, stack, TexAlpha{&S});
+    bool live = false;
+    uint32_t gx = 0, gy = 0, k = 0;
+    Rng rng{};
+    V3 acc = v3z();
+    // the path: its ray is the walk's (w.o, w.d) unless a shadow ray is cast
+    V3 pix = v3z(), alpha = v3z();
+    float initY = 0.0f, dirPDF = 0.0f;
+    uint32_t sampledType = 0, depth = 0;
+    bool first = true, over = false;
+    // while a shadow ray is cast: its contribution, the light's face (kNone:
+    // the environment), and the extension ray after it unless the path ends
+    bool shadow = false, ends = false;
+    uint32_t target = kNone;
+    V3 contrib = v3z(), nextOrg = v3z(), nextDir = v3z();
+
+    while (true) {
+        bool ray = false, newSample = false, anyRay = false;
+        V3 org = v3z(), dir = v3z();
+        float bound = INFINITY;
+        uint32_t boundFace = kNone;
+        if (live) {
+            over |= w.over();
+            bool end = false, left = false;  // the path ends; it left the scene
+            const bool hit = w.best != kNone && !isinf(w.t);
+            if (!w.done()) {
+                // still walking
+            } else if (shadow) {
+                shadow = false;
+                if (target == kNone ? !hit : w.best == target) {
+                    pix += contrib;
+                    job.lightSeen(contrib, pix);
+                }
+                if (ends) {
+                    end = true;
+                } else {
+                    org = nextOrg;
+                    dir = nextDir;
+                    ray = true;
+                }
+            } else if (!hit) {
+                end = left = true;
+            } else {
+                SurfPt sp;
+                hitParams(S, w.o, w.d, w.t, w.best, w.b1, w.b2, sp);
+                const clr_face F = S.g.faces[sp.face];
+                const V3 vout = -w.d;
+                EDF E;
+                if (F.lightPtr != 0xFFFFu) {
+                    edfArea(S, F.lightPtr, sp, sp.u, sp.v, E);
+                    V3 term;
+                    if (first) {
+                        term = alpha * evalLe(E, vout);
+                    } else {
+                        float mis = 1.0f;
+                        if (sampledType & kNonSingular) {
+                            const V3 dd = sp.p - w.o;
+                            const float d2 = dd.x * dd.x + dd.y * dd.y + dd.z * dd.z;
+                            const float lightPDF = areaPdfOfFace(S, sp.face) * d2 / absCosEDF(E, vout);
+                            mis = emissionHitMis(flags, dirPDF, lightPDF);
+                        }
+                        term = (mis * alpha) * evalLe(E, vout);
+                    }
+                    pix += term;
+                    job.emission(term, F.lightPtr);
+                }
+                if (!first) {
+                    if (depth >= maxDepth) {
+                        end = true;
+                    } else if (!noRR) {
+                        const float cp = fminf(lum(alpha) * (1.0f / initY), 1.0f);
+                        if (rng.uniform() < cp) {
+                            alpha = alpha * (1.0f / cp);
+                            dirPDF *= cp;
+                        } else {
+                            end = true;
+                        }
+                    }
+                }
+                first = false;
+                if (!end) {
+                    BSDF B;
+                    bsdfAlloc(S, F.matPtr, sp, B);
+                    if (hasNonSpecular(B)) {
+                        const float lu = rng.uniform(), l0 = rng.uniform(), l1 = rng.uniform();
+                        // With BSDF samples alone the light sample is skipped (its numbers are drawn).
+                        if (!(flags & CLR_RENDER_BSDF_SAMPLING_ONLY)) {
+                            SurfPt lp;
+                            bool atInf = false;
+                            float lightPDF;
+                            sampleLight(S, lu, l0, l1, lp, atInf, E, lightPDF);
+                            V3 vinL = lp.p - sp.p;
+                            float dist2 = dot(vinL, vinL);
+                            vinL = vinL * (1.0f / sqrtf(dist2));
+                            if (atInf) {
+                                vinL = lp.p;
+                                dist2 = 1.0f;
+                            }
+                            // A zero or infinite light density (an environment sample at a
+                            // pole, where sin(theta) = 0) contributes nothing.
+                            if (lightPDF > 0.0f && lightPDF < INFINITY) {
+                                const V3 vinLrev = -vinL;
+                                const float fsPDF = evalFsPdf(B, vout, vinL) * absCosEDF(E, vinL) / dist2;
+                                const float mis = lightSampleMis(flags, lightPDF, fsPDF);
+                                const float wgt = mis * absCosEDF(E, vinL) * fabsf(dot(B.N, vinL)) / dist2 / lightPDF;
+                                contrib = wgt * ((alpha * evalLe(E, vinLrev)) * evalFs(B, vout, vinL));
+                                org = sp.p + vinL * kRayEps;
+                                dir = vinL;
+                                target = atInf ? kNone : lp.face;
+                                shadow = !job.unseen(contrib);
+                                if (shadow && !atInf) {
+                                    float x1, x2;
+                                    uint32_t flag;
+                                    shadow = triTestPacked(S.g.atris, org, dir, lp.face, bound, x1, x2, flag) &&
+                                             !isinf(bound) && !(flag && TexAlpha{&S}.reject(lp.face, x1, x2));
+                                    boundFace = lp.face;
+                                }
+                                if (shadow)
+                                    job.lightSample(atInf ? 0xFFFFFFFFu : (uint32_t)S.g.faces[lp.face].lightPtr, F.matPtr,
+                                                    B, vout, vinL, sp);
+                            }
+                        }
+                    }
+                    const float bc = rng.uniform(), b0 = rng.uniform(), b1 = rng.uniform();
+                    V3 nd = v3z();
+                    const V3 f = sampleFs(B, vout, bc, b0, b1, nd, dirPDF, sampledType);
+                    ends = (f.x == 0.0f && f.y == 0.0f && f.z == 0.0f) || dirPDF == 0.0f;
+                    if (!ends) {
+                        job.bounce(F.matPtr, B, vout, nd, sp, pix);
+                        alpha = alpha * (f * (fabsf(dot(B.N, nd)) / dirPDF));
+                        nextDir = nd;
+                        nextOrg = sp.p + nd * kRayEps;
+                        ++depth;
+                    }
+                    if (shadow) {
+                        ray = anyRay = true;
+                    } else if (ends) {
+                        end = true;
+                    } else {
+                        org = nextOrg;
+                        dir = nextDir;
+                        bound = INFINITY;
+                        boundFace = kNone;
+                        ray = true;
+                    }
+                }
+            }
+            if (end) {
+                if (left) {
+                    const V3 vout = -w.d;
+                    const float theta = acosf(clampf(w.d.y, -1.0f, 1.0f));
+                    const float phi = fmodf(atan2f(-w.d.x, w.d.z) + 2.0f * kPiF, 2 * kPiF);
+                    const float u = phi / (2.0f * kPiF), v = theta / kPiF;
+                    EDF E;
+                    edfEnv(S, u, v, E);
+                    float mis = 1.0f;
+                    if ((sampledType & kNonSingular) != 0 && depth > 0) {
+                        const float lightPDF = areaPdfEnv(S, u, v) * 1.0f / absCosEDF(E, vout);
+                        mis = emissionHitMis(flags, dirPDF, lightPDF);
+                    }
+                    pix += (mis * alpha) * evalLe(E, vout);
+                }
+                acc += pix;
+                job.finish(pix);
+                if (++k < spp) {
+                    newSample = true;
+                } else {
+                    job.store(gx, gy, rng, acc);
+                    live = false;
+                }
+            }
+        }
+        if (src.take(!live, gx, gy)) {
+            job.load(gx, gy, rng);
+            acc = v3z();
+            k = 0;
+            live = newSample = true;
+        }
+        if (newSample) {
+            float wgt;
+            cameraRay(S, gx, gy, rng, org, dir, wgt, dirPDF);
+            alpha = v3s(1.0f) * wgt;
+            initY = lum(alpha);
+            pix = v3z();
+            sampledType = 0;
+            depth = 0;
+            first = true;
+            ray = true;
+        }
+        if (ray) w.begin(org, dir, bound, anyRay, boundFace);
+        if (__ballot(live) == 0) break;
+        // Walk until enough lanes wait. Every walk ends (its visits are
+        // bounded), so the loop does.
+        do {
+            if (!w.done()) w.step();
+        } while (__ballot(!w.done()) != 0 && __popcll(__ballot(live && w.done())) < (int)kServeMin);
+    }
+    if (over) atomicOr(S.status, kStatusStackOverflow);
 }
 
 // ---- path-replay adjoint ----------------------------------------------------
@@ -419,100 +514,148 @@ struct AdjHook {
     }
 };
 
+// AdjHook as a job of tracePixels, which shades a vertex before its light
+// sample is known to be seen: the sample's factors wait here, and the prefix
+// recorded at the vertex's bounce is completed when the sample counts.
+struct AdjJob : AdjHook {
+    const uint4* states;
+    const float4* dLdI;
+    uint32_t width;
+    float inv;  // 1 / spp
+    uint32_t lightM;  // parameter index + 1 of the waiting sample's material (0: none)
+    bool lightEm, recorded, finite;
+    V3 lightRho;
+    float lightDlog;
+
+    __device__ __forceinline__ void load(uint32_t gx, uint32_t gy, Rng& rng) {
+        const size_t pi = (size_t)gy * width + gx;
+        const uint4 st = states[pi];
+        rng = {st.x, st.y, st.z, st.w};
+        const float4 a = dLdI[pi];
+        adj = {a.x * inv, a.y * inv, a.z * inv};
+        finite = fabsf(adj.x) < INFINITY && fabsf(adj.y) < INFINITY && fabsf(adj.z) < INFINITY;
+    }
+    __device__ __forceinline__ void store(uint32_t, uint32_t, const Rng&, V3) {}
+    // A zero term's derivatives are zero unless the image gradient is not finite.
+    __device__ __forceinline__ bool unseen(V3 term) const {
+        return finite && term.x == 0.0f && term.y == 0.0f && term.z == 0.0f;
+    }
+    __device__ __forceinline__ void lightSample(uint32_t lightPtr, uint32_t matPtr, const BSDF& B, V3 vout, V3 vinL,
+                                                const SurfPt& sp) {
+        lightEm = lightPtr == lightProp;
+        lightM = param(matPtr, B);
+        recorded = false;
+        if (lightM) {
+            lightRho = B.c[0].R;
+            lightDlog = dlogSigma(matPtr, B, sp, vout, vinL);
+        }
+    }
+    __device__ __forceinline__ void lightSeen(V3 term, V3 pixSoFar) {
+        if (lightEm) addEmission(term);
+        if (lightM) {
+            addAlbedo(lightM - 1, term, lightRho);
+            atomicAdd(acc->sig + (lightM - 1), dot(adj, term) * lightDlog);
+        }
+        if (recorded) recPrefix[n - 1] = pixSoFar;
+    }
+    __device__ __forceinline__ void bounce(uint32_t matPtr, const BSDF& B, V3 vout, V3 vin, const SurfPt& sp,
+                                           V3 pixSoFar) {
+        const int before = n;
+        AdjHook::bounce(matPtr, B, vout, vin, sp, pixSoFar);
+        recorded = n != before;
+    }
+};
+
 }  // namespace dev
 
 namespace {
 
 constexpr int kTile = 8;  // 8x8 pixels per wave
 
-// Occupancy of the ordered megakernel, which waits on memory. The ordered
-// walk's stack keeps its first kMegaLds words per lane in LDS and the rest in
-// a per-lane global region, so LDS holds 20 waves per CU (8 KiB each) where
-// the whole stack in LDS (16 KiB) held 10, and the register budget is set for
-// five waves per SIMD (96 VGPRs, a few spilled). 16 spp of the 1080p outdoor
-// scene: 134.6 ms at 10 waves per CU, 109.9 at 12, 92.9 at 16, 89.5 at 20.
-// Only deep walks touch the spill. The reference walks keep their 64-entry
-// LDS stack (10 waves per CU).
+// Occupancy of the ordered megakernel: the walk's stack keeps its first
+// kMegaLds words per lane in LDS and the rest in a per-lane global region that
+// only deep walks touch, so LDS holds 20 waves per CU (8 KiB each) where the
+// whole stack in LDS (16 KiB) holds 10; the register budget is four waves per
+// SIMD. The reference walks keep their 64-entry LDS stack.
 constexpr int kMegaLds = 32;
-constexpr uint32_t kMegaWavesPerCU = 20;  // persistent grid
-// The merged sample/bounce loop keeps more state alive across its one trace
-// call: at four waves per SIMD (128 VGPRs) it beat five (96 VGPRs, more
-// spills): 1080p 341-345 -> 330-334 ms, the 256-scene batch 289-294 -> 284-286.
-// Three (168 VGPRs) took 378-381 and 325-326 ms.
-constexpr uint32_t kMegaMergedWavesPerCU = 16;
+constexpr uint32_t kMegaWavesPerCU = 16;
+constexpr uint32_t kReferenceWavesPerCU = 20;  // persistent grid of the reference walks
 // The adjoint's waves also hold 4 KiB of LDS gradient sums, so its stack
-// keeps 16 words in LDS (8 KiB per wave with the sums) and its register
-// budget is set for four waves per SIMD: 512x512, 32 spp, depth 5 of the
-// differentiation scene, 99 ms at 8 waves per CU (20 KiB of LDS each),
-// 100 ms at 13 (a 32-word stack), 68.6 ms at 16.
+// keeps 16 words in LDS (8 KiB per wave with the sums).
 constexpr uint32_t kAdjWavesPerCU = 16;
 constexpr int kAdjLds = 16;
+
+template <int LDS>
+using MegaStack = dev::PairStack<LDS / 2, dev::kStackDepth / 2>;
+template <int LDS>
+__device__ __forceinline__ MegaStack<LDS> megaStack(uint32_t* s_stack, uint32_t* spill) {
+    return {reinterpret_cast<uint2*>(s_stack) + threadIdx.x, 64,
+            reinterpret_cast<uint2*>(spill) + blockIdx.x * 64u + threadIdx.x, gridDim.x * 64u};
+}
 
 __global__ void k_mega_reset(uint32_t* counter) {
     if (threadIdx.x == 0) *counter = 0u;
 }
 
-// One 8x8 tile (tile index `tile` of an image tilesX tiles wide), all spp
-// samples of its pixels; states and pixels are the image's own arrays.
-template <int WALK, int LDS, bool MERGED>
-__device__ __forceinline__ void renderTile(const dev::RScene& S, uint32_t tile, uint32_t tilesX, uint32_t width,
-                                           uint32_t height, uint32_t spp, uint32_t maxDepth, uint32_t flags,
-                                           uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
-                                           uint32_t* __restrict__ spill, uint32_t* s_stack) {
-    const uint32_t lanes = gridDim.x * 64u;
-    const uint32_t lane = blockIdx.x * 64u + threadIdx.x;
-    const uint32_t gx = (tile % tilesX) * kTile + (threadIdx.x % kTile);
-    const uint32_t gy = (tile / tilesX) * kTile + (threadIdx.x / kTile);
-    if (gx >= width || gy >= height) return;
-    const size_t pi = (size_t)gy * width + gx;
-    uint4 st = reinterpret_cast<uint4*>(states)[pi];
-    dev::Rng rng{st.x, st.y, st.z, st.w};
-    dev::V3 acc = dev::v3z();
-    dev::NoHook hook;
-    // MERGED: the sample and bounce loops merged (tracePixel).
-    auto trace = [&](const auto& stk) {
-        if constexpr (MERGED)
-            acc = dev::tracePixel<WALK>(S, gx, gy, spp, maxDepth, flags, rng, stk);
-        else
-            for (uint32_t k = 0; k < spp; ++k) acc += dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook);
-    };
-    if constexpr (WALK == dev::kWalkOrdered)
-        trace(dev::PairStack<LDS / 2, dev::kStackDepth / 2>{reinterpret_cast<uint2*>(s_stack) + threadIdx.x, 64,
-                                                            reinterpret_cast<uint2*>(spill) + lane, lanes});
-    else
-        trace(dev::LdsStack{s_stack + threadIdx.x, 64});
-    reinterpret_cast<uint4*>(states)[pi] = make_uint4(rng.s0, rng.s1, rng.s2, rng.s3);
-    float4 p = reinterpret_cast<float4*>(pixels)[pi];
-    p.x += acc.x;
-    p.y += acc.y;
-    p.z += acc.z;
-    reinterpret_cast<float4*>(pixels)[pi] = p;
-}
-
-// The next tile of a persistent wave: lane 0 takes it from the counter.
+// The next tile of a persistent wave: lane 0 takes it from the counter
+// (zeroed by k_mega_reset on the same stream).
 __device__ __forceinline__ uint32_t nextTile(uint32_t* tileCounter) {
     uint32_t t = 0;
     if (threadIdx.x == 0) t = atomicAdd(tileCounter, 1u);
     return __builtin_amdgcn_readfirstlane(__shfl((int)t, 0));
 }
 
-// Persistent waves: each takes the next 8x8 tile from a device counter
-// (zeroed by k_mega_reset on the same stream) until the image is done, so
-// the spill region is sized by the grid, not by the image.
-// LDS: stack words per lane kept in LDS (the ordered walk spills the rest;
-// the reference walks need all kStackDepth).
-template <int WALK, int LDS, bool MERGED>
-__device__ __forceinline__ void renderTiles(const dev::RScene& scene, uint32_t width, uint32_t height, uint32_t spp,
-                                            uint32_t maxDepth, uint32_t flags, uint32_t* __restrict__ states,
-                                            clr_float3* __restrict__ pixels, uint32_t* __restrict__ tileCounter,
-                                            uint32_t* __restrict__ spill, uint32_t* s_stack) {
+// Pixels for tracePixels from 8x8 tiles that the wave takes from a device
+// counter: tiles [first, end) of one image, whose first tile is number
+// `first` of the counter's. A tile beyond `end` ends the source and stays in
+// `tile` for the caller (the next image of a batch, or past the last one).
+struct TileSource {
+    uint32_t* counter;
+    uint32_t width, height, tilesX, first, end;
+    uint32_t tile;      // current tile
+    uint32_t next = 0;  // its next position, 0..64
+    bool open = true;
+    // Every lane calls it; returns true in wanting lanes that got a pixel.
+    __device__ __forceinline__ bool take(bool want, uint32_t& gx, uint32_t& gy) {
+        bool got = false;
+        while (open) {
+            const uint64_t idle = __ballot(want && !got);
+            if (idle == 0) break;
+            if (next >= 64u) {
+                tile = nextTile(counter);
+                next = 0;
+                if (tile >= end) open = false;
+                continue;
+            }
+            const uint32_t pos = next + (uint32_t)__popcll(idle & ((1ull << __lane_id()) - 1ull));
+            if (want && !got && pos < 64u) {
+                const uint32_t t = tile - first;
+                const uint32_t x = (t % tilesX) * kTile + pos % kTile, y = (t / tilesX) * kTile + pos / kTile;
+                if (x < width && y < height) {
+                    gx = x;
+                    gy = y;
+                    got = true;
+                }
+            }
+            next += (uint32_t)__popcll(idle);
+        }
+        return got;
+    }
+};
+
+// One image by persistent waves.
+template <int LDS, class Job>
+__device__ __forceinline__ void renderImage(const dev::RScene& scene, uint32_t width, uint32_t height, uint32_t spp,
+                                            uint32_t maxDepth, uint32_t flags, Job& job, uint32_t* tileCounter,
+                                            uint32_t* spill, uint32_t* s_stack) {
     dev::RScene S = scene;  // resolved copy; the kernel argument itself stays read-only
     dev::finishScene(S);
     const uint32_t tilesX = (width + kTile - 1) / kTile;
-    const uint32_t tiles = tilesX * ((height + kTile - 1) / kTile);
-    for (uint32_t tile = nextTile(tileCounter); tile < tiles; tile = nextTile(tileCounter))
-        renderTile<WALK, LDS, MERGED>(S, tile, tilesX, width, height, spp, maxDepth, flags, states, pixels, spill,
-                                      s_stack);
+    TileSource src{tileCounter, width, height, tilesX, 0u, tilesX * ((height + kTile - 1) / kTile),
+                   nextTile(tileCounter)};
+    src.open = src.tile < src.end;
+    const MegaStack<LDS> stk = megaStack<LDS>(s_stack, spill);
+    dev::tracePixels(S, spp, maxDepth, flags, stk, job, src);
 }
 
 // A batch of equally sized images: the tiles of all scenes share one
@@ -520,74 +663,97 @@ __device__ __forceinline__ void renderTiles(const dev::RScene& scene, uint32_t w
 // whose states and pixels start at scene * width * height. Consecutive tiles
 // stay in one scene, so the waves resident at a time walk a few scenes'
 // arrays. The table's entries have their blob headers resolved.
-template <int WALK, int LDS, bool MERGED>
-__device__ __forceinline__ void renderBatchTiles(const dev::RScene* __restrict__ table, uint32_t numScenes,
-                                                 uint32_t width, uint32_t height, uint32_t spp, uint32_t maxDepth,
-                                                 uint32_t flags, uint32_t* __restrict__ states,
-                                                 clr_float3* __restrict__ pixels, uint32_t* __restrict__ tileCounter,
-                                                 uint32_t* __restrict__ spill, uint32_t* s_stack) {
+template <int LDS>
+__device__ __forceinline__ void renderBatch(const dev::RScene* __restrict__ table, uint32_t numScenes, uint32_t width,
+                                            uint32_t height, uint32_t spp, uint32_t maxDepth, uint32_t flags,
+                                            uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
+                                            uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill,
+                                            uint32_t* s_stack) {
     const uint32_t tilesX = (width + kTile - 1) / kTile;
     const uint32_t tilesPerScene = tilesX * ((height + kTile - 1) / kTile);
     const uint32_t tiles = tilesPerScene * numScenes;
     const size_t npix = (size_t)width * height;
-    for (uint32_t tile = nextTile(tileCounter); tile < tiles; tile = nextTile(tileCounter)) {
+    const MegaStack<LDS> stk = megaStack<LDS>(s_stack, spill);
+    uint32_t tile = nextTile(tileCounter);
+    while (tile < tiles) {
         const uint32_t s = tile / tilesPerScene;
         const dev::RScene S = table[s];
-        renderTile<WALK, LDS, MERGED>(S, tile - s * tilesPerScene, tilesX, width, height, spp, maxDepth, flags,
-                                      states + 4 * npix * s, pixels + npix * s, spill, s_stack);
+        dev::ImageJob job{reinterpret_cast<uint4*>(states) + npix * s, reinterpret_cast<float4*>(pixels) + npix * s,
+                          width};
+        TileSource src{tileCounter, width, height, tilesX, s * tilesPerScene, (s + 1) * tilesPerScene, tile};
+        dev::tracePixels(S, spp, maxDepth, flags, stk, job, src);
+        tile = src.tile;
     }
 }
 
-// Large images: five waves per SIMD (four with MERGED). MERGED: the ordered walk's merged
-// sample and bounce loop (tracePixel), used when Russian roulette is on.
-// Without it paths run to the bounce cap unless they leave the scene, little
-// imbalance is left to recover, and the per-sample loop needs fewer registers
-// (the 512x512 differentiation scene without roulette: 56 ms per-sample
-// against 61 ms merged).
-template <int WALK, bool MERGED>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MERGED ? 4 : 5))) void k_render_mega(
+// The ordered traversal, large images.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_render_mega(
     dev::RScene scene, uint32_t width, uint32_t height, uint32_t spp, uint32_t maxDepth, uint32_t flags,
     uint32_t* __restrict__ states, clr_float3* __restrict__ pixels, uint32_t* __restrict__ tileCounter,
     uint32_t* __restrict__ spill) {
-    constexpr int kLds = WALK == dev::kWalkOrdered ? kMegaLds : dev::kStackDepth;
-    __shared__ __align__(8) uint32_t s_stack[kLds * 64];
-    renderTiles<WALK, kLds, MERGED>(scene, width, height, spp, maxDepth, flags, states, pixels, tileCounter, spill,
-                                    s_stack);
+    __shared__ __align__(8) uint32_t s_stack[kMegaLds * 64];
+    dev::ImageJob job{reinterpret_cast<uint4*>(states), reinterpret_cast<float4*>(pixels), width};
+    renderImage<kMegaLds>(scene, width, height, spp, maxDepth, flags, job, tileCounter, spill, s_stack);
 }
 
 // Images of at most kMegaFewTiles tiles per CU cannot fill many waves per
 // CU, so their waves keep the whole stack in LDS and all the registers they
 // want (no spills).
 constexpr uint32_t kMegaFewTiles = 4;
-template <int WALK, bool MERGED>
 __global__ __launch_bounds__(64) void k_render_mega_few(dev::RScene scene, uint32_t width, uint32_t height,
                                                         uint32_t spp, uint32_t maxDepth, uint32_t flags,
                                                         uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
                                                         uint32_t* __restrict__ tileCounter,
                                                         uint32_t* __restrict__ spill) {
     __shared__ __align__(8) uint32_t s_stack[dev::kStackDepth * 64];
-    renderTiles<WALK, dev::kStackDepth, MERGED>(scene, width, height, spp, maxDepth, flags, states, pixels,
-                                                tileCounter, spill, s_stack);
+    dev::ImageJob job{reinterpret_cast<uint4*>(states), reinterpret_cast<float4*>(pixels), width};
+    renderImage<dev::kStackDepth>(scene, width, height, spp, maxDepth, flags, job, tileCounter, spill, s_stack);
 }
 
 // Batches: the same two shapes.
-template <bool MERGED>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MERGED ? 4 : 5))) void k_render_mega_batch(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_render_mega_batch(
     const dev::RScene* __restrict__ table, uint32_t numScenes, uint32_t width, uint32_t height, uint32_t spp,
     uint32_t maxDepth, uint32_t flags, uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
     uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill) {
     __shared__ __align__(8) uint32_t s_stack[kMegaLds * 64];
-    renderBatchTiles<dev::kWalkOrdered, kMegaLds, MERGED>(table, numScenes, width, height, spp, maxDepth, flags,
-                                                          states, pixels, tileCounter, spill, s_stack);
+    renderBatch<kMegaLds>(table, numScenes, width, height, spp, maxDepth, flags, states, pixels, tileCounter, spill,
+                          s_stack);
 }
-template <bool MERGED>
 __global__ __launch_bounds__(64) void k_render_mega_batch_few(
     const dev::RScene* __restrict__ table, uint32_t numScenes, uint32_t width, uint32_t height, uint32_t spp,
     uint32_t maxDepth, uint32_t flags, uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,
     uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill) {
     __shared__ __align__(8) uint32_t s_stack[dev::kStackDepth * 64];
-    renderBatchTiles<dev::kWalkOrdered, dev::kStackDepth, MERGED>(table, numScenes, width, height, spp, maxDepth,
-                                                                  flags, states, pixels, tileCounter, spill, s_stack);
+    renderBatch<dev::kStackDepth>(table, numScenes, width, height, spp, maxDepth, flags, states, pixels, tileCounter,
+                                  spill, s_stack);
+}
+
+// The reference's walks (WALK: over the LBVH or the CPU midpoint BVH), one
+// 8x8 tile at a time, each lane all samples of its pixel.
+template <int WALK>
+__global__ __launch_bounds__(64) void k_render_reference(dev::RScene scene, uint32_t width, uint32_t height,
+                                                         uint32_t spp, uint32_t maxDepth, uint32_t flags,
+                                                         uint32_t* __restrict__ states,
+                                                         clr_float3* __restrict__ pixels,
+                                                         uint32_t* __restrict__ tileCounter) {
+    __shared__ uint32_t s_stack[dev::kStackDepth * 64];
+    dev::RScene S = scene;
+    dev::finishScene(S);
+    const dev::LdsStack stk{s_stack + threadIdx.x, 64};
+    const dev::ImageJob job{reinterpret_cast<uint4*>(states), reinterpret_cast<float4*>(pixels), width};
+    const uint32_t tilesX = (width + kTile - 1) / kTile;
+    const uint32_t tiles = tilesX * ((height + kTile - 1) / kTile);
+    dev::NoHook hook;
+    for (uint32_t tile = nextTile(tileCounter); tile < tiles; tile = nextTile(tileCounter)) {
+        const uint32_t gx = (tile % tilesX) * kTile + (threadIdx.x % kTile);
+        const uint32_t gy = (tile / tilesX) * kTile + (threadIdx.x / kTile);
+        if (gx >= width || gy >= height) continue;
+        dev::Rng rng;
+        job.load(gx, gy, rng);
+        dev::V3 acc = dev::v3z();
+        for (uint32_t k = 0; k < spp; ++k) acc += dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook);
+        job.store(gx, gy, rng, acc);
+    }
 }
 
 // bvh_visualizer (bvh_visualizer.cl:25-84): one ray through each pixel
@@ -640,10 +806,10 @@ __global__ __launch_bounds__(64) void k_bvh_visualizer(dev::RScene scene, uint32
     reinterpret_cast<float4*>(pixels)[pi] = p;
 }
 
-// Adjoint of k_render_mega: the same pixels, samples and random states, each
-// sample replayed with the adjoint hook. Persistent waves take tiles from the
-// same kind of counter, with a split stack, and sum their gradients in LDS
-// over all their tiles; the sums go to global memory once per wave.
+// Adjoint of a render: the same pixels, samples and random states, each
+// sample replayed with the adjoint's job (reference walks: hook). Persistent
+// waves sum their gradients in LDS over all their tiles; the sums go to
+// global memory once per wave.
 template <int WALK>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_render_adjoint(
     dev::RScene scene, uint32_t width, uint32_t height, uint32_t spp, uint32_t maxDepth, uint32_t flags,
@@ -664,31 +830,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const uint8_t* e = S.mat + ((lightProp + 1u + 3u) & ~3u);
         M = dev::evalColor(S.tex + dev::ld<uint32_t>(e + 4), 0.0f, 0.0f);
     }
-    const uint32_t tilesX = (width + kTile - 1) / kTile;
-    const uint32_t tiles = tilesX * ((height + kTile - 1) / kTile);
-    const uint32_t lanes = gridDim.x * 64u;
-    const uint32_t lane = blockIdx.x * 64u + threadIdx.x;
-    auto nextTile = [&]() {
-        uint32_t t = 0;
-        if (threadIdx.x == 0) t = atomicAdd(tileCounter, 1u);
-        return (uint32_t)__shfl((int)t, 0);
-    };
-    const float inv = 1.0f / (float)spp;
-    for (uint32_t tile = nextTile(); tile < tiles; tile = nextTile()) {
-        const uint32_t gx = (tile % tilesX) * kTile + (threadIdx.x % kTile);
-        const uint32_t gy = (tile / tilesX) * kTile + (threadIdx.x / kTile);
-        if (gx >= width || gy >= height) continue;
-        const size_t pi = (size_t)gy * width + gx;
-        const uint4 st = reinterpret_cast<const uint4*>(states)[pi];
-        dev::Rng rng{st.x, st.y, st.z, st.w};
-        const float4 a = dLdI[pi];
-        dev::AdjHook hook{S, table, lightProp, M, {a.x * inv, a.y * inv, a.z * inv}, &s_acc, 0};
-        if constexpr (WALK == dev::kWalkOrdered) {
-            const dev::PairStack<kLds / 2, dev::kStackDepth / 2> stk{reinterpret_cast<uint2*>(s_stack) + threadIdx.x, 64,
-                                                                     reinterpret_cast<uint2*>(spill) + lane, lanes};
-            for (uint32_t k = 0; k < spp; ++k) hook.finish(dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook));
-        } else {
-            const dev::LdsStack stk{s_stack + threadIdx.x, 64};
+    dev::AdjJob job{{S, table, lightProp, M, dev::v3z(), &s_acc, 0}, reinterpret_cast<const uint4*>(states), dLdI,
+                    width, 1.0f / (float)spp};
+    if constexpr (WALK == dev::kWalkOrdered) {
+        renderImage<kLds>(scene, width, height, spp, maxDepth, flags, job, tileCounter, spill, s_stack);
+    } else {
+        const uint32_t tilesX = (width + kTile - 1) / kTile;
+        const uint32_t tiles = tilesX * ((height + kTile - 1) / kTile);
+        const dev::LdsStack stk{s_stack + threadIdx.x, 64};
+        for (uint32_t tile = nextTile(tileCounter); tile < tiles; tile = nextTile(tileCounter)) {
+            const uint32_t gx = (tile % tilesX) * kTile + (threadIdx.x % kTile);
+            const uint32_t gy = (tile / tilesX) * kTile + (threadIdx.x / kTile);
+            if (gx >= width || gy >= height) continue;
+            dev::Rng rng;
+            job.load(gx, gy, rng);
+            dev::AdjHook& hook = job;
             for (uint32_t k = 0; k < spp; ++k) hook.finish(dev::tracePath<WALK>(S, gx, gy, maxDepth, flags, rng, stk, hook));
         }
     }
@@ -778,15 +934,8 @@ int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, Ac
     if (sd.numLights)
         k_face_lights_fill<<<(sd.numLights + 255) / 256, 256, 0, stream>>>(sd.lights, sd.numLights,
                                                                            sd.numFaces, faceLight, envLight);
-    const float4 *anodes = nullptr, *atris = nullptr, *wnodes = nullptr;
-    if (kind != AccelKind::kNone) {
-        rc = buildAccel(ctx, sd.internalNodes, sd.leafNodes, sd.bvhNodes, sd.numFaces, sd.vertices, sd.faces,
-                        kind == AccelKind::kBinary ? &anodes : nullptr, &atris, stream,
-                        kind == AccelKind::kWide ? &wnodes : nullptr);
-        if (rc) return rc;
-    }
-    S.g = dev::GeomScene{sd.internalNodes, sd.leafNodes, sd.numFaces, sd.vertices, sd.faces, anodes, atris,
-                         reinterpret_cast<const float4*>(sd.bvhNodes), wnodes};
+    rc = buildAccel(ctx, sd, kind, S.g, stream);
+    if (rc) return rc;
     S.normals = sd.normals;
     S.tangents = sd.tangents;
     S.uvs = sd.uvs;
@@ -814,27 +963,28 @@ int renderMegakernel(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_par
     int cus = 0;
     rc = hipCheck(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
     if (rc) return rc;
-    const bool merged = !(flags & CLR_RENDER_NO_RR) && !(flags & CLR_RENDER_REFERENCE_TRAVERSAL);
+    const bool reference = (flags & CLR_RENDER_REFERENCE_TRAVERSAL) != 0;
     const uint32_t grid =
-        std::max(1u, std::min(tiles, (uint32_t)cus * (merged ? kMegaMergedWavesPerCU : kMegaWavesPerCU)));
-    rc = ensureTraceSpill(ctx, (size_t)grid * 64 * (dev::kStackDepth - kMegaLds) * sizeof(uint32_t));
-    if (rc) return rc;
+        std::max(1u, std::min(tiles, (uint32_t)cus * (reference ? kReferenceWavesPerCU : kMegaWavesPerCU)));
     uint32_t* counter = ctx->devStatus + kWordMegaTiles;
+    if (!reference) {
+        rc = ensureTraceSpill(ctx, (size_t)grid * 64 * (dev::kStackDepth - kMegaLds) * sizeof(uint32_t));
+        if (rc) return rc;
+    }
     k_mega_reset<<<1, 64, 0, stream>>>(counter);
-    auto launch = [&](auto kernel) {
-        kernel<<<grid, 64, 0, stream>>>(S, rp.width, rp.height, rp.samplesPerPixel, rp.maxDepth, flags, states, pixels,
-                                        counter, ctx->traceSpill);
-    };
-    const bool few = tiles <= (uint32_t)cus * kMegaFewTiles;
-    if (!(rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL)) {
-        if (few)
-            launch(merged ? k_render_mega_few<dev::kWalkOrdered, true> : k_render_mega_few<dev::kWalkOrdered, false>);
-        else
-            launch(merged ? k_render_mega<dev::kWalkOrdered, true> : k_render_mega<dev::kWalkOrdered, false>);
-    } else if (sd.bvhNodes)
-        launch(k_render_mega<dev::kWalkMidpoint, false>);
-    else
-        launch(k_render_mega<dev::kWalkLbvh, false>);
+    if (!reference) {
+        auto launch = [&](auto kernel) {
+            kernel<<<grid, 64, 0, stream>>>(S, rp.width, rp.height, rp.samplesPerPixel, rp.maxDepth, flags, states,
+                                            pixels, counter, ctx->traceSpill);
+        };
+        launch(tiles <= (uint32_t)cus * kMegaFewTiles ? k_render_mega_few : k_render_mega);
+    } else {
+        auto launch = [&](auto kernel) {
+            kernel<<<grid, 64, 0, stream>>>(S, rp.width, rp.height, rp.samplesPerPixel, rp.maxDepth, flags, states,
+                                            pixels, counter);
+        };
+        launch(sd.bvhNodes ? k_render_reference<dev::kWalkMidpoint> : k_render_reference<dev::kWalkLbvh>);
+    }
     return hipCheck(ctx, hipGetLastError(), "render launch");
 }
 
@@ -844,9 +994,7 @@ int renderMegakernelBatch(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t nu
     int rc = hipCheck(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
     if (rc) return rc;
     const uint64_t tiles = (uint64_t)((rp.width + kTile - 1) / kTile) * ((rp.height + kTile - 1) / kTile) * numScenes;
-    const bool merged = !(rp.flags & CLR_RENDER_NO_RR);
-    const uint32_t grid = (uint32_t)std::max<uint64_t>(
-        1, std::min<uint64_t>(tiles, (uint64_t)cus * (merged ? kMegaMergedWavesPerCU : kMegaWavesPerCU)));
+    const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(tiles, (uint64_t)cus * kMegaWavesPerCU));
     const size_t spillBytes = (size_t)grid * 64 * (dev::kStackDepth - kMegaLds) * sizeof(uint32_t);
     if (ctx->traceSpillBytes < spillBytes) {
         bool capturing = false;
@@ -868,10 +1016,7 @@ int renderMegakernelBatch(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t nu
         kernel<<<grid, 64, 0, stream>>>(table, numScenes, rp.width, rp.height, rp.samplesPerPixel, rp.maxDepth,
                                         rp.flags, states, pixels, counter, ctx->traceSpill);
     };
-    if (tiles <= (uint64_t)cus * kMegaFewTiles)
-        launch(merged ? k_render_mega_batch_few<true> : k_render_mega_batch_few<false>);
-    else
-        launch(merged ? k_render_mega_batch<true> : k_render_mega_batch<false>);
+    launch(tiles <= (uint64_t)cus * kMegaFewTiles ? k_render_mega_batch_few : k_render_mega_batch);
     return hipCheck(ctx, hipGetLastError(), "batch render launch");
 }
 

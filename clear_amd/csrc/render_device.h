@@ -331,18 +331,24 @@ __device__ void hitParams(const RScene& S, V3 org, V3 dir, float t, uint32_t fac
 }
 
 // Alpha rejection through the face's alpha texture (bvh_traversal.cl:94-105).
+// Not inlined: the walks ask rarely, and the texture lookup inside their loop
+// cost every visit registers and mask arithmetic.
+__device__ __attribute__((noinline)) bool alphaReject(const clr_face* faces, const float* uvs, const uint8_t* tex,
+                                                      uint32_t face, float b1, float b2) {
+    const clr_face& f = faces[face];
+    if (f.uv0 == kNone || f.alphaTexPtr == kNone) return false;
+    const float b0 = 1.0f - b1 - b2;
+    const float2 a = reinterpret_cast<const float2*>(uvs)[f.uv0];
+    const float2 b = reinterpret_cast<const float2*>(uvs)[f.uv1];
+    const float2 c = reinterpret_cast<const float2*>(uvs)[f.uv2];
+    const float u = b0 * a.x + b1 * b.x + b2 * c.x;
+    const float v = b0 * a.y + b1 * b.y + b2 * c.y;
+    return evalAlpha(tex + f.alphaTexPtr, u, v) == 0.0f;
+}
 struct TexAlpha {
     const RScene* S;
     __device__ __forceinline__ bool reject(uint32_t face, float b1, float b2) const {
-        const clr_face& f = S->g.faces[face];
-        if (f.uv0 == kNone || f.alphaTexPtr == kNone) return false;
-        const float b0 = 1.0f - b1 - b2;
-        const float2 a = reinterpret_cast<const float2*>(S->uvs)[f.uv0];
-        const float2 b = reinterpret_cast<const float2*>(S->uvs)[f.uv1];
-        const float2 c = reinterpret_cast<const float2*>(S->uvs)[f.uv2];
-        const float u = b0 * a.x + b1 * b.x + b2 * c.x;
-        const float v = b0 * a.y + b1 * b.y + b2 * c.y;
-        return evalAlpha(S->tex + f.alphaTexPtr, u, v) == 0.0f;
+        return alphaReject(S->g.faces, S->uvs, S->tex, face, b1, b2);
     }
 };
 

@@ -38,7 +38,8 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_closest(
     dev::V3 o = {rays[r], rays[R + r], rays[2 * R + r]};
     dev::V3 d = {rays[3 * R + r], rays[4 * R + r], rays[5 * R + r]};
     float t = rays[6 * R + r];
-    dev::GeomScene g{inodes, leaves, n, verts, faces, nullptr, nullptr, bvh};
+    dev::GeomScene g{inodes, leaves, n, verts, faces};
+    g.bvh = bvh;
     dev::TraceStats st{0u, 0u};
     bool over = false;
     uint32_t best = dev::closestHit<STATS>(g, o, d, t, dev::LdsStack{s_stack + threadIdx.x, kTraceBlock},
@@ -160,17 +161,74 @@ struct WideSlots {
                            __uint_as_float(ref[3]));
         o[7] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
+    // The 64-byte form (GeomScene::qnodes). Per axis the grid starts at the
+    // lowest plane and its step is the smallest power of two that reaches the
+    // highest plane in 255 steps; planes round outwards, and a box whose
+    // plane is not ordered against the grid's ends (NaN) takes the end.
+    __device__ __forceinline__ void storeBytes(float4* o) const {
+        float org[3], scale[3];
+        uint32_t qlo[3], qhi[3];
+        for (int a = 0; a < 3; ++a) {
+            float l = INFINITY, h = -INFINITY;
+            bool finite = true;
+            for (int c = 0; c < 4; ++c)
+                if (ref[c] != dev::kNone) {
+                    l = fminf(l, lo[a][c]);
+                    h = fmaxf(h, hi[a][c]);
+                    finite &= fabsf(lo[a][c]) < INFINITY && fabsf(hi[a][c]) < INFINITY;
+                }
+            const float ext = h - l;
+            finite &= ext < 1e38f;
+            qlo[a] = qhi[a] = 0;
+            if (!finite) {
+                org[a] = 0.0f;
+                scale[a] = INFINITY;
+                qhi[a] = 0xFFFFFFFFu;
+                continue;
+            }
+            // 2^e with 255 * 2^e >= ext: the exponent of ext / 255 rounded up.
+            const uint32_t bits = __float_as_uint(ext * (1.0f / 254.5f));
+            const uint32_t e = max((bits + 0x007FFFFFu) >> 23, 1u);
+            const float s = __uint_as_float(e << 23), inv = __uint_as_float(min(254u - e, 254u) << 23);
+            org[a] = l;
+            scale[a] = s;
+            for (int c = 0; c < 4; ++c) {
+                if (ref[c] == dev::kNone) {
+                    qlo[a] |= 255u << (8 * c);
+                    continue;
+                }
+                float fl = floorf((lo[a][c] - l) * inv), fh = ceilf((hi[a][c] - l) * inv);
+                if (l + fl * s > lo[a][c]) fl -= 1.0f;
+                if (l + fh * s < hi[a][c]) fh += 1.0f;
+                const uint32_t ql = fl >= 0.0f && fl <= 255.0f ? (uint32_t)fl : 0u;
+                const uint32_t qh = fh >= 0.0f && fh <= 255.0f ? (uint32_t)fh : 255u;
+                qlo[a] |= ql << (8 * c);
+                qhi[a] |= qh << (8 * c);
+            }
+        }
+        uint4* u = reinterpret_cast<uint4*>(o);
+        o[0] = make_float4(org[0], org[1], org[2], scale[0]);
+        u[1] = make_uint4(qlo[0], qhi[0], qlo[1], qhi[1]);
+        u[2] = make_uint4(qlo[2], qhi[2], __float_as_uint(scale[1]), __float_as_uint(scale[2]));
+        u[3] = make_uint4(ref[0], ref[1], ref[2], ref[3]);
+    }
+    template <bool BYTES>
+    __device__ __forceinline__ void put(float4* records, size_t i) const {
+        if constexpr (BYTES) storeBytes(records + 4 * i);
+        else store(records + 8 * i);
+    }
 };
 
+template <bool BYTES>
 __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves,
-                             uint32_t n, float4* __restrict__ wnodes) {
+                             uint32_t n, float4* __restrict__ records) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     WideSlots w;
     w.clear();
     if (n == 1 && i == 0) {  // a tree of one leaf: a record that holds it
         const float4* p = reinterpret_cast<const float4*>(leaves);
         w.put(0, p[0], p[1], leaves[0].objIdx | dev::kLeafRef);
-        w.store(wnodes);
+        w.put<BYTES>(records, 0);
         return;
     }
     if (i + 1 >= n) return;
@@ -197,12 +255,13 @@ __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const cl
             w.put(2 * k + m, p[0], p[1], gl ? (leaves[gi].objIdx | dev::kLeafRef) : gi);
         }
     }
-    w.store(wnodes + 8 * (size_t)i);
+    w.put<BYTES>(records, i);
 }
 
 // The same records for a CPU midpoint BVH, by node number (leaf node slots
 // stay unused).
-__global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, float4* __restrict__ wnodes) {
+template <bool BYTES>
+__global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, float4* __restrict__ records) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t numNodes = 2 * n - 1;
     if (i >= numNodes) return;
@@ -211,7 +270,7 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
     w.clear();
     if (n == 1 && c.y == kEmpty) {  // a tree of one leaf: a record that holds it
         w.put(0, bvh[0], bvh[1], c.x | dev::kLeafRef);
-        w.store(wnodes);
+        w.put<BYTES>(records, 0);
         return;
     }
     if (c.y == kEmpty || c.x >= numNodes || c.y >= numNodes) return;
@@ -233,7 +292,7 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
             w.put(2 * k + m, q[0], q[1], gc.y == kEmpty ? (gc.x | dev::kLeafRef) : gi);
         }
     }
-    w.store(wnodes + 8 * (size_t)i);
+    w.put<BYTES>(records, i);
 }
 
 // Trace with the ordered traversal, grid-stride over the rays with a fixed
@@ -263,26 +322,25 @@ __device__ __forceinline__ void traceTwo(W& w0, W& w1, const float* __restrict__
             w.begin(o, d, rays[6 * R + r]);
         } else {
             r = kEmpty;
-            w.done = true;
         }
     };
     auto finish = [&](const W& w, uint32_t r) {
-        if (w.over) over = true;
+        if (w.over()) over = true;
         done(w, r);
     };
     start(w0, r0);
     start(w1, r1);
     while (r0 != kEmpty || r1 != kEmpty) {
         if (r0 != kEmpty) {
-            if (!w0.done) w0.step();
-            if (w0.done) {
+            if (!w0.done()) w0.step();
+            if (w0.done()) {
                 finish(w0, r0);
                 start(w0, r0);
             }
         }
         if (r1 != kEmpty) {
-            if (!w1.done) w1.step();
-            if (w1.done) {
+            if (!w1.done()) w1.step();
+            if (w1.done()) {
                 finish(w1, r1);
                 start(w1, r1);
             }
@@ -322,14 +380,14 @@ __global__ __launch_bounds__(kOrdBlock) void k_trace_wide(
     dev::GeomScene g, const float* __restrict__ rays, uint32_t numRays, uint32_t* __restrict__ hitFace,
     float* __restrict__ hitT, uint32_t* __restrict__ status, uint32_t* __restrict__ spill) {
     constexpr int kPairs = kOrdHalf / 2;
+    using S = dev::PairStack<kPairs, dev::kStackPairs / 2>;
     __shared__ uint2 s_stack[2 * kPairs * kOrdBlock];
     const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
     const uint32_t lanes = gridDim.x * kOrdBlock;
-    using S = dev::PairStack<kPairs, dev::kStackPairs / 2>;
     uint2* sp = reinterpret_cast<uint2*>(spill);
     const S stk0{s_stack + threadIdx.x, kOrdBlock, sp + gid, lanes};
-    const S stk1{s_stack + kPairs * kOrdBlock + threadIdx.x, kOrdBlock, sp + (size_t)(S::CAP - kPairs) * lanes + gid,
-                 lanes};
+    const S stk1{s_stack + kPairs * kOrdBlock + threadIdx.x, kOrdBlock,
+                 sp + (size_t)(S::CAP - kPairs) * lanes + gid, lanes};
     using W = dev::WideWalk<dev::NoAlpha, S>;
     W w0(g, stk0, dev::NoAlpha()), w1(g, stk1, dev::NoAlpha());
     traceTwo(w0, w1, rays, numRays, gid, lanes, status, [&](const W& w, uint32_t r) {
@@ -347,22 +405,35 @@ size_t accelNodeBytes(uint32_t n, bool midpoint) {
 }
 
 size_t accelWideBytes(uint32_t n, bool midpoint) { return 2 * accelNodeBytes(n, midpoint); }
+size_t accelByteBytes(uint32_t n, bool midpoint) { return accelNodeBytes(n, midpoint); }
 
-void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
-                     float4* wnodes, hipStream_t stream) {
+namespace {
+template <bool BYTES>
+void launchWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
+                float4* records, hipStream_t stream) {
     if (bvh)
-        k_accel_wide_bvh<<<(2 * n - 1 + 255) / 256, 256, 0, stream>>>(reinterpret_cast<const float4*>(bvh), n,
-                                                                       wnodes);
+        k_accel_wide_bvh<BYTES><<<(2 * n - 1 + 255) / 256, 256, 0, stream>>>(reinterpret_cast<const float4*>(bvh), n,
+                                                                             records);
     else
-        k_accel_wide<<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, wnodes);
+        k_accel_wide<BYTES><<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, records);
+}
+}  // namespace
+
+void launchAccelBytes(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
+                      float4* qnodes, hipStream_t stream) {
+    launchWide<true>(inodes, leaves, bvh, n, qnodes, stream);
 }
 
-int buildAccel(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
-               uint32_t n, const clr_float3* vertices, const clr_face* faces, const float4** anodes,
-               const float4** atris, hipStream_t stream, const float4** wnodes) {
-    const size_t nodeBytes = anodes ? accelNodeBytes(n, bvh != nullptr) : 0;
-    const size_t triBytes = ((size_t)n * 48 + 255) & ~size_t(255);
-    const size_t need = nodeBytes + triBytes + (wnodes ? accelWideBytes(n, bvh != nullptr) : 0);
+int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomScene& g, hipStream_t stream) {
+    const uint32_t n = sd.numFaces;
+    const bool midpoint = sd.bvhNodes != nullptr;
+    g = dev::GeomScene{sd.internalNodes, sd.leafNodes, n, sd.vertices, sd.faces};
+    g.bvh = reinterpret_cast<const float4*>(sd.bvhNodes);
+    if (kind == AccelKind::kNone) return CLR_OK;
+    const size_t nodeBytes = kind == AccelKind::kBinary ? accelNodeBytes(n, midpoint)
+                             : kind == AccelKind::kWide ? accelWideBytes(n, midpoint)
+                                                        : accelByteBytes(n, midpoint);
+    const size_t need = nodeBytes + (((size_t)n * 48 + 255) & ~size_t(255));
     if (ctx->accelBytes < need) {
         int rc = hipCheck(ctx, hipDeviceSynchronize(), "accel regrow sync");
         if (rc) return rc;
@@ -376,15 +447,19 @@ int buildAccel(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* 
         }
         ctx->accelBytes = need;
     }
-    float4* an = anodes ? static_cast<float4*>(ctx->accel) : nullptr;
-    float4* at = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes);
-    launchAccelBuild(inodes, leaves, bvh, n, vertices, faces, an, at, stream);
-    if (anodes) *anodes = an;
-    *atris = at;
-    if (wnodes) {
-        float4* wn = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes + triBytes);
-        launchAccelWide(inodes, leaves, bvh, n, wn, stream);
-        *wnodes = wn;
+    float4* nodes = static_cast<float4*>(ctx->accel);
+    float4* tris = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes);
+    launchAccelBuild(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, sd.vertices, sd.faces,
+                     kind == AccelKind::kBinary ? nodes : nullptr, tris, stream);
+    g.atris = tris;
+    if (kind == AccelKind::kBinary) {
+        g.anodes = nodes;
+    } else if (kind == AccelKind::kWide) {
+        g.wnodes = nodes;
+        launchWide<false>(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, nodes, stream);
+    } else {
+        g.qnodes = nodes;
+        launchWide<true>(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, nodes, stream);
     }
     return hipCheck(ctx, hipGetLastError(), "traversal layout launch");
 }
@@ -413,13 +488,16 @@ int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     const size_t lanes = (size_t)grid * kOrdBlock;
     rc = ensureTraceSpill(ctx, lanes * 2 * (dev::kStackPairs - kOrdHalf) * sizeof(uint32_t));
     if (rc) return rc;
-    const bool binary = stats && !wide;  // only the binary walk's counts need its records
-    const float4 *anodes = nullptr, *atris = nullptr, *wnodes = nullptr;
-    rc = buildAccel(ctx, inodes, leaves, bvh, n, vertices, faces, binary ? &anodes : nullptr, &atris, stream,
-                    binary ? nullptr : &wnodes);
+    clr_scene_dev sd{};
+    sd.vertices = vertices;
+    sd.faces = faces;
+    sd.internalNodes = inodes;
+    sd.leafNodes = leaves;
+    sd.numFaces = n;
+    sd.bvhNodes = bvh;
+    dev::GeomScene g;
+    rc = buildAccel(ctx, sd, !stats ? AccelKind::kBytes : wide ? AccelKind::kWide : AccelKind::kBinary, g, stream);
     if (rc) return rc;
-    const dev::GeomScene g{inodes, leaves, n, vertices, faces, anodes, atris, reinterpret_cast<const float4*>(bvh),
-                           wnodes};
     if (!stats)
         k_trace_wide<<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, ctx->devStatus, ctx->traceSpill);
     else if (wide)

@@ -60,13 +60,21 @@ struct GeomScene {
     // reference-order walks use it instead of inodes / leaves, and the
     // traversal layout is indexed by its node numbers.
     const float4* bvh = nullptr;
-    // 4-wide records for the renderers' walk ([slots][8], slots as anodes):
+    // 4-wide records of the counting 4-wide walk ([slots][8], slots as anodes):
     // record i holds the up to four grandchildren of internal node i (the
     // children of each internal child, a leaf child itself), as SoA
     // float4s: lo.x, lo.y, lo.z, hi.x, hi.y, hi.z of slots 0..3, then the
     // four references (face | kLeafRef, node, or kNone for an empty slot
     // with an empty box). Unused when null.
     const float4* wnodes = nullptr;
+    // The same records in 64 bytes for WideWalk ([slots][4]): child boxes as
+    // bytes on the record's own grid. float4s: origin.xyz, scale.x | bytes of
+    // lo.x, hi.x, lo.y, hi.y of slots 0..3 | bytes of lo.z, hi.z, then
+    // scale.y, scale.z | the four references. A plane is origin + byte *
+    // scale, rounded outwards (scale a power of two); an axis on which some
+    // box is not finite has scale infinity and bytes 0 and 255, which every
+    // ray passes.
+    const float4* qnodes = nullptr;
 };
 constexpr uint32_t kLeafRef = 0x80000000u;
 static_assert(sizeof(clr_lbvh_inode) == 48 && sizeof(clr_lbvh_leaf) == 48 && sizeof(clr_bvh_node) == 48,
@@ -430,8 +438,10 @@ struct Ordered {
     float t, b1, b2;
     uint32_t best, node, steps;
     int depth;
-    bool done, over;
+    bool ended, overflowed;
     TraceStats st;
+    __device__ __forceinline__ bool done() const { return ended; }
+    __device__ __forceinline__ bool over() const { return overflowed; }
 
     __device__ __forceinline__ Ordered(const GeomScene& g_, const Stack& s_, const Alpha& a_)
         : g(g_), stack(s_), alpha(a_) {}
@@ -458,23 +468,23 @@ struct Ordered {
         best = kNone;
         node = kNone;
         depth = 0;
-        done = false;
-        over = false;
+        ended = false;
+        overflowed = false;
         steps = 0;
         st = {0u, 0u};
         if (g.n == 0) {
-            done = true;
+            ended = true;
         } else if (g.n == 1) {
             // The single leaf: LBVH leaf 0 (objIdx) or the midpoint root leaf
             // (children[0]); both hold the box in their first 32 bytes and
             // the face at byte 32.
             const float4* lp = g.bvh ? g.bvh : reinterpret_cast<const float4*>(g.leaves);
             if (slabEnter(lp[0], lp[1], o, inv, t) <= t) leaf(reinterpret_cast<const uint32_t*>(lp + 2)[0]);
-            done = true;
+            ended = true;
         } else {
             const float4* np = g.bvh ? g.bvh : reinterpret_cast<const float4*>(g.inodes);
             if (slabEnter(np[0], np[1], o, inv, t) <= t) node = 0;
-            else done = true;
+            else ended = true;
         }
     }
 
@@ -482,8 +492,8 @@ struct Ordered {
         // A tree visits each node at most once and pops at most as often as
         // it pushes: more than 2n steps means malformed nodes; stop and flag.
         if (++steps > 2u * g.n + 2u) {
-            done = true;
-            over = true;
+            ended = true;
+            overflowed = true;
             return;
         }
         if (node != kNone) {
@@ -509,11 +519,11 @@ struct Ordered {
                         stack.put(depth + 1, __float_as_uint(first1 ? e0 : e1));
                         depth += 2;
                     } else {
-                        over = true;
+                        overflowed = true;
                     }
                 } else {
                     if (depth < kStackDepth) stack.put(depth++, first1 ? r0 : r1);
-                    else over = true;
+                    else overflowed = true;
                 }
                 node = first1 ? r1 : r0;
             } else if (go0 || go1) {
@@ -530,12 +540,12 @@ struct Ordered {
                         }
                     }
                 }
-                if (node == kNone && depth == 0) done = true;
+                if (node == kNone && depth == 0) ended = true;
             }
             return;
         }
         if constexpr (PAIRS) {  // not reached: PAIRS visits pop inline
-            done = true;
+            ended = true;
             return;
         }
         // The candidate's own box: first 32 bytes of its 48-byte record (LBVH
@@ -543,7 +553,7 @@ struct Ordered {
         const uint32_t cand = stack.get(--depth);
         const float4* cp = (g.bvh ? g.bvh : reinterpret_cast<const float4*>(g.inodes)) + 3 * (size_t)cand;
         if (slabEnter(cp[0], cp[1], o, inv, t) <= t) node = cand;
-        else if (depth == 0) done = true;
+        else if (depth == 0) ended = true;
     }
 };
 
@@ -568,8 +578,10 @@ struct Wide {
     float t, b1, b2;
     uint32_t best, node, steps;
     int depth;
-    bool done, over;
+    bool ended, overflowed;
     TraceStats st;
+    __device__ __forceinline__ bool done() const { return ended; }
+    __device__ __forceinline__ bool over() const { return overflowed; }
 
     __device__ __forceinline__ Wide(const GeomScene& g_, const Stack& s_, const Alpha& a_)
         : g(g_), stack(s_), alpha(a_) {}
@@ -596,20 +608,20 @@ struct Wide {
         best = kNone;
         node = kNone;
         depth = 0;
-        done = false;
-        over = false;
+        ended = false;
+        overflowed = false;
         steps = 0;
         st = {0u, 0u};
         if (g.n == 0) {
-            done = true;
+            ended = true;
         } else if (g.n == 1) {
             const float4* lp = g.bvh ? g.bvh : reinterpret_cast<const float4*>(g.leaves);
             if (slabEnter(lp[0], lp[1], o, inv, t) <= t) leaf(reinterpret_cast<const uint32_t*>(lp + 2)[0]);
-            done = true;
+            ended = true;
         } else {
             const float4* np = g.bvh ? g.bvh : reinterpret_cast<const float4*>(g.inodes);
             if (slabEnter(np[0], np[1], o, inv, t) <= t) node = 0;
-            else done = true;
+            else ended = true;
         }
     }
 
@@ -617,8 +629,8 @@ struct Wide {
         // Each node is visited at most once: more than 2n steps means
         // malformed records; stop and flag.
         if (++steps > 2u * g.n + 2u) {
-            done = true;
-            over = true;
+            ended = true;
+            overflowed = true;
             return;
         }
         ++st.visits;
@@ -679,7 +691,7 @@ struct Wide {
                 return;
             }
         }
-        done = true;
+        ended = true;
     }
 
     __device__ __forceinline__ void push(uint32_t ref, float entry) {
@@ -688,7 +700,7 @@ struct Wide {
             stack.put(depth + 1, __float_as_uint(entry));
             depth += 2;
         } else {
-            over = true;
+            overflowed = true;
         }
     }
 };
@@ -698,18 +710,29 @@ struct Wide {
 // depths), the others up to CAP in a per-lane global region.
 template <int L, int CAP_>
 struct PairStack {
-    static constexpr int CAP = CAP_;
+    static constexpr int CAP = CAP_, kInLds = L;
     uint2* lds;
     int stride;
     uint2* spill;
     size_t spillStride;
+    // Kept apart so that no access is made through a pointer that may be
+    // either (a flat access: it takes the memory path also for LDS).
     __device__ __forceinline__ void put(int k, uint32_t ref, float entry) const {
-        const uint2 v = make_uint2(ref, __float_as_uint(entry));
-        if (L >= CAP || k < L) lds[k * stride] = v;
-        else spill[(size_t)(k - L) * spillStride] = v;
+        if (L >= CAP || k < L)
+            lds[k * stride] = make_uint2(ref, __float_as_uint(entry));
+        else
+            __builtin_nontemporal_store((uint64_t)__float_as_uint(entry) << 32 | ref, global(k));
     }
     __device__ __forceinline__ uint2 get(int k) const {
-        return (L >= CAP || k < L) ? lds[k * stride] : spill[(size_t)(k - L) * spillStride];
+        uint2 v = lds[(L >= CAP ? k : min(k, L - 1)) * stride];
+        if (L < CAP && k >= L) {
+            const uint64_t g = __builtin_nontemporal_load(global(k));
+            v = make_uint2((uint32_t)g, (uint32_t)(g >> 32));
+        }
+        return v;
+    }
+    __device__ __forceinline__ uint64_t* global(int k) const {
+        return reinterpret_cast<uint64_t*>(spill + (size_t)(k - L) * spillStride);
     }
 };
 
@@ -719,14 +742,18 @@ struct PairStack {
 // way, as long as none that holds an accepted triangle is passed over. That
 // leaves the box arithmetic free, and a visit is bound by its instructions
 // (few lanes are active, so every instruction counts in full):
-//   * near and far planes are loaded by the ray's direction signs (two planes
+//   * a record is 64 bytes (GeomScene::qnodes): four 16-byte loads from half a
+//     cache line where the float planes took seven from a whole one; the
+//     walks wait on L2, and the records of a scene take half of it;
+//   * near and far planes are chosen by the ray's direction signs (two planes
 //     an axis instead of four and a min and max each), and a plane's distance
-//     is one fma: t = plane * inv - o * inv. The cancellation error of that
-//     form, at most 2^-22 |o * inv|, is covered by moving the near planes'
-//     constant down and the far planes' up by 2^-21 |o * inv|; the relative
-//     pad of slabEnter (1 -+ 2^-16 on entry and exit) is one factor 1 - 2^-15
-//     on the entry. Every box that slabEnter admits is admitted; NaNs (from
-//     infinite products) are ignored by min / max and so admit.
+//     is one fma: t = byte * (scale * inv) + (origin * inv - o * inv). The
+//     cancellation error of that form, a few 2^-24 |o * inv| (or of t), is
+//     covered by moving the near planes' constant down and the far planes'
+//     up by 2^-21 |o * inv|; the relative pad of slabEnter (1 -+ 2^-16 on entry
+//     and exit) is one factor 1 - 2^-15 on the entry. Every box that
+//     slabEnter admits is admitted; NaNs (from infinite products) are ignored
+//     by min / max and so admit.
 //   * leaf entries are tested in a loop over each lane's own leaves, so the
 //     triangle test runs as often as the lane with the most leaves has, not
 //     once for each of the four slots in which some lane has one;
@@ -744,26 +771,28 @@ struct PairStack {
 // scene on the wavefront renderer 24.3 -> 21.4 ms.
 template <class Alpha, class Stack>
 struct WideWalk {
-    const float4* wn;
+    const float4* qn;
     const float4* tris;
     uint32_t limit;  // more visits than this mean malformed records
     const Stack& stack;
     Alpha alpha;
     V3 o, d, inv, cn, cf;  // near plane distance: plane * inv + cn; far: plane * inv + cf
-    uint32_t nx, ny, nz;   // float4 offset of the near planes in a record (far: 3, 5, 7 - it)
     float t, b1, b2;
-    uint32_t best, node, steps;
+    uint32_t best, bound, node, left;  // node: kNone when the walk has ended
     int depth;
-    bool done, over, any;
+    uint32_t mode;  // kAny, kOver
+    static constexpr uint32_t kAny = 1u, kOver = 2u;
 
     __device__ __forceinline__ WideWalk(const GeomScene& g, const Stack& s_, const Alpha& a_)
-        : wn(g.wnodes), tris(g.atris), limit(2u * g.n + 2u), stack(s_), alpha(a_) {}
+        : qn(g.qnodes), tris(g.atris), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
     __device__ __forceinline__ void rebind(const GeomScene& g, const Alpha& a_) {
-        wn = g.wnodes;
+        qn = g.qnodes;
         tris = g.atris;
         limit = 2u * g.n + 2u;
         alpha = a_;
     }
+    __device__ __forceinline__ bool done() const { return node == kNone; }
+    __device__ __forceinline__ bool over() const { return (mode & kOver) != 0; }
 
     __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax, bool anyHit = false, uint32_t bestFace = kNone) {
         o = o_;
@@ -774,31 +803,38 @@ struct WideWalk {
         const V3 oi = {o.x * inv.x, o.y * inv.y, o.z * inv.z};
         cn = {-oi.x - fabsf(oi.x) * kSlack, -oi.y - fabsf(oi.y) * kSlack, -oi.z - fabsf(oi.z) * kSlack};
         cf = {-oi.x + fabsf(oi.x) * kSlack, -oi.y + fabsf(oi.y) * kSlack, -oi.z + fabsf(oi.z) * kSlack};
-        nx = inv.x < 0.0f ? 3u : 0u;
-        ny = inv.y < 0.0f ? 4u : 1u;
-        nz = inv.z < 0.0f ? 5u : 2u;
         t = tmax;
         b1 = b2 = 0.0f;
-        best = bestFace;
-        node = 0;
-        steps = 0;
+        best = bound = bestFace;
+        node = tmax >= 0.0f ? 0u : kNone;  // no t >= 0 lies before a negative or NaN bound
+        left = limit;
         depth = 0;
-        done = false;
-        over = false;
-        any = anyHit;
+        mode = anyHit ? kAny : 0u;
     }
 
+    // The reference's triangle test (triTestPacked) without branches on the
+    // way: with a handful of lanes in it, some lane passes each early exit.
     __device__ __forceinline__ void leaf(uint32_t face) {
-        float tt = t, x1, x2;
-        uint32_t flag;
-        if (!triTestPacked(tris, o, d, face, tt, x1, x2, flag)) return;
-        if (tt == t && face >= best) return;
-        if (flag && alpha.reject(face, x1, x2)) return;
+        const float4* tp = tris + 3 * (size_t)face;
+        const float4 a = tp[0], b = tp[1], c = tp[2];
+        const V3 p0 = {a.x, a.y, a.z}, edge01 = {b.x, b.y, b.z}, edge02 = {c.x, c.y, c.z};
+        const V3 p = cross(d, edge02);
+        const float det = dot(edge01, p);
+        const float invDet = 1.0f / det;
+        const V3 dd = o - p0;
+        const float u = dot(dd, p) * invDet;
+        const V3 q = cross(dd, edge01);
+        const float v = dot(d, q) * invDet;
+        const float tt = dot(edge02, q) * invDet;
+        const uint32_t miss = (uint32_t)(det > -0.000001f && det < 0.000001f) | (uint32_t)(u < 0.0f) |
+                              (uint32_t)(u > 1.0f) | (uint32_t)(v < 0.0f) | (uint32_t)(u + v > 1.0f) |
+                              (uint32_t)(tt < 0.0f) | (uint32_t)(tt > t) | (uint32_t)(tt == t && face >= best);
+        if (miss) return;
+        if (__float_as_uint(a.w) && alpha.reject(face, u, v)) return;
         t = tt;
         best = face;
-        b1 = x1;
-        b2 = x2;
-        if (any && !isinf(tt)) done = true;
+        b1 = u;
+        b2 = v;
     }
 
     static __device__ __forceinline__ uint32_t pick(const uint4& r, uint32_t slot) {
@@ -806,37 +842,39 @@ struct WideWalk {
         return (slot & 2u) ? hi : lo;
     }
 
+    // Visits `node`.
     __device__ __forceinline__ void step() {
-        if (++steps > limit) {
-            done = true;
-            over = true;
-            return;
-        }
-        const float4* wp = wn + 8 * (size_t)node;
-        const float4 ax = wp[nx], ay = wp[ny], az = wp[nz];
-        const float4 bx = wp[3u - nx], by = wp[5u - ny], bz = wp[7u - nz];
-        const uint4 r = reinterpret_cast<const uint4*>(wp)[6];
+        const float4* qp = qn + 4 * (size_t)node;
+        const float4 q0 = qp[0];
+        const uint4 q1 = reinterpret_cast<const uint4*>(qp)[1], q2 = reinterpret_cast<const uint4*>(qp)[2];
+        const uint4 r = reinterpret_cast<const uint4*>(qp)[3];
+        const bool sx = inv.x < 0.0f, sy = inv.y < 0.0f, sz = inv.z < 0.0f;
+        const uint32_t nx = sx ? q1.y : q1.x, fx = sx ? q1.x : q1.y;
+        const uint32_t ny = sy ? q1.w : q1.z, fy = sy ? q1.z : q1.w;
+        const uint32_t nz = sz ? q2.y : q2.x, fz = sz ? q2.x : q2.y;
+        const float kx = q0.w * inv.x, ky = __uint_as_float(q2.z) * inv.y, kz = __uint_as_float(q2.w) * inv.z;
+        const float nbx = __builtin_fmaf(q0.x, inv.x, cn.x), fbx = __builtin_fmaf(q0.x, inv.x, cf.x);
+        const float nby = __builtin_fmaf(q0.y, inv.y, cn.y), fby = __builtin_fmaf(q0.y, inv.y, cf.y);
+        const float nbz = __builtin_fmaf(q0.z, inv.z, cn.z), fbz = __builtin_fmaf(q0.z, inv.z, cf.z);
         uint32_t leaves = 0;
-        auto entry = [&](float px, float py, float pz, float qx, float qy, float qz, uint32_t ref, uint32_t slot) {
-            const float tn = fmaxf(fmaxf(__builtin_fmaf(px, inv.x, cn.x), __builtin_fmaf(py, inv.y, cn.y)),
-                                   fmaxf(__builtin_fmaf(pz, inv.z, cn.z), 0.0f)) *
+        auto entry = [&](uint32_t slot, uint32_t ref) {
+            auto byte = [&](uint32_t v) { return (float)((v >> (8u * slot)) & 0xFFu); };
+            const float tn = fmaxf(fmaxf(__builtin_fmaf(byte(nx), kx, nbx), __builtin_fmaf(byte(ny), ky, nby)),
+                                   fmaxf(__builtin_fmaf(byte(nz), kz, nbz), 0.0f)) *
                              (1.0f - 1.0f / 32768.0f);
-            const float tf = fminf(fminf(__builtin_fmaf(qx, inv.x, cf.x), __builtin_fmaf(qy, inv.y, cf.y)),
-                                   __builtin_fmaf(qz, inv.z, cf.z));
-            const bool pass = tn <= tf && tn <= t && ref != kNone;
-            const bool leafRef = (ref & kLeafRef) != 0;
-            if (pass && leafRef) leaves |= 1u << slot;
-            return pass && !leafRef ? ((__float_as_uint(tn) & ~3u) | slot) : 0xFFFFFFFFu;
+            const float tf = fminf(fminf(__builtin_fmaf(byte(fx), kx, fbx), __builtin_fmaf(byte(fy), ky, fby)),
+                                   fminf(__builtin_fmaf(byte(fz), kz, fbz), t));
+            const bool pass = tn <= tf;
+            const uint32_t isLeaf = (uint32_t)((int32_t)ref >> 31);  // all ones; empty slots too, skipped below
+            leaves |= (pass ? 1u << slot : 0u) & isLeaf;
+            return (pass ? ((__float_as_uint(tn) & ~3u) | slot) : 0xFFFFFFFFu) | isLeaf;
         };
-        uint32_t k0 = entry(ax.x, ay.x, az.x, bx.x, by.x, bz.x, r.x, 0u);
-        uint32_t k1 = entry(ax.y, ay.y, az.y, bx.y, by.y, bz.y, r.y, 1u);
-        uint32_t k2 = entry(ax.z, ay.z, az.z, bx.z, by.z, bz.z, r.z, 2u);
-        uint32_t k3 = entry(ax.w, ay.w, az.w, bx.w, by.w, bz.w, r.w, 3u);
+        uint32_t k0 = entry(0u, r.x), k1 = entry(1u, r.y), k2 = entry(2u, r.z), k3 = entry(3u, r.w);
         while (leaves) {
             const uint32_t slot = (uint32_t)__builtin_ctz(leaves);
             leaves &= leaves - 1u;
-            leaf(pick(r, slot) & ~kLeafRef);
-            if (done) return;
+            const uint32_t ref = pick(r, slot);
+            if (ref != kNone) leaf(ref & ~kLeafRef);
         }
         auto cx = [](uint32_t& a, uint32_t& b) {
             const uint32_t lo = min(a, b);
@@ -848,32 +886,51 @@ struct WideWalk {
         cx(k0, k2);
         cx(k1, k3);
         cx(k1, k2);
-        // Entries beyond a hit of this visit's own leaves stay (sorted last,
-        // dropped at their pop); 0xFFFFFFFF is a NaN and fails every compare.
-        if (k1 != 0xFFFFFFFFu) {
-            if (k2 != 0xFFFFFFFFu) {
-                if (k3 != 0xFFFFFFFFu) push(pick(r, k3 & 3u), __uint_as_float(k3));
-                push(pick(r, k2 & 3u), __uint_as_float(k2));
+        // Push all but the nearest, farthest first. Entries beyond a hit of
+        // this visit's own leaves stay (their pop drops them); 0xFFFFFFFF is a
+        // NaN and fails every compare.
+        const int more = (int)(k1 != 0xFFFFFFFFu) + (int)(k2 != 0xFFFFFFFFu) + (int)(k3 != 0xFFFFFFFFu);
+        // Unless some lane's stack nears its global part, three stores without
+        // branches: what is not pushed goes to the free slot above the top.
+        const bool deep = __ballot(depth + 3 > Stack::kInLds) != 0;
+        if (!deep) {
+            auto put = [&](uint32_t k, int j) {
+                const int at = depth + more - (k != 0xFFFFFFFFu ? j + 1 : 0);
+                stack.lds[at * stack.stride] = make_uint2(pick(r, k & 3u), k);
+            };
+            if (__ballot(k3 != 0xFFFFFFFFu)) put(k3, 2);
+            if (__ballot(k2 != 0xFFFFFFFFu)) put(k2, 1);
+            put(k1, 0);
+            depth += more;
+        } else {
+            if (k3 != 0xFFFFFFFFu) push(pick(r, k3 & 3u), __uint_as_float(k3));
+            if (k2 != 0xFFFFFFFFu) push(pick(r, k2 & 3u), __uint_as_float(k2));
+            if (k1 != 0xFFFFFFFFu) push(pick(r, k1 & 3u), __uint_as_float(k1));
+        }
+        const bool go = __uint_as_float(k0) <= t;
+        node = go ? pick(r, k0 & 3u) : kNone;
+        if (!go) {
+            while (depth > 0) {
+                const uint2 e = stack.get(--depth);
+                if (__uint_as_float(e.y) <= t) {
+                    node = e.x;
+                    break;
+                }
             }
-            push(pick(r, k1 & 3u), __uint_as_float(k1));
         }
-        if (__uint_as_float(k0) <= t) {
-            node = pick(r, k0 & 3u);
-            return;
+        // An any walk ends at its first hit of finite distance, every walk at
+        // a NaN distance (nothing compares with it) or with its visits used up.
+        const bool stop = ((mode & kAny) && best != bound && !isinf(t)) || t != t;
+        if (--left == 0u) {
+            mode |= kOver;
+            node = kNone;
         }
-        while (depth > 0) {
-            const uint2 c = stack.get(--depth);
-            if (__uint_as_float(c.y) <= t) {
-                node = c.x;
-                return;
-            }
-        }
-        done = true;
+        if (stop) node = kNone;
     }
 
     __device__ __forceinline__ void push(uint32_t ref, float e) {
         if (depth < Stack::CAP) stack.put(depth++, ref, e);
-        else over = true;
+        else mode |= kOver;
     }
 };
 
@@ -884,11 +941,11 @@ __device__ __forceinline__ uint32_t wideHit(const GeomScene& g, V3 o, V3 d, floa
                                             float& b2, const Alpha& alpha, bool& overflow) {
     WideWalk<Alpha, Stack> w(g, stack, alpha);
     w.begin(o, d, t);
-    while (!w.done) w.step();
+    while (!w.done()) w.step();
     t = w.t;
     b1 = w.b1;
     b2 = w.b2;
-    if (w.over) overflow = true;
+    if (w.over()) overflow = true;
     return w.best;
 }
 
@@ -900,11 +957,11 @@ __device__ __forceinline__ uint32_t orderedHit(const GeomScene& g, V3 o, V3 d, f
                                                bool& overflow) {
     Ordered<Alpha, Stack> w(g, stack, alpha);
     w.begin(o, d, t);
-    while (!w.done) w.step();
+    while (!w.done()) w.step();
     t = w.t;
     b1 = w.b1;
     b2 = w.b2;
-    if (w.over) overflow = true;
+    if (w.over()) overflow = true;
     st = w.st;
     return w.best;
 }
