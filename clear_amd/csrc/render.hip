@@ -28,7 +28,7 @@ struct NoHook {
 // CLR_RENDER_* word (NO_RR disables Russian roulette, the bounce cap still
 // applies; the SAMPLING_ONLY bits select one strategy).
 template <int WALK, class Stack, class Hook = NoHook>
-__device__ V3 tracePath(const RScene& S, uint32_t gx, uint32_t gy, uint32_t maxDepth, uint32_t flags, Rng& rng,
+__device__ __forceinline__ V3 tracePath(const RScene& S, uint32_t gx, uint32_t gy, uint32_t maxDepth, uint32_t flags, Rng& rng,
                         const Stack& stack, Hook& hook) {
     const bool noRR = (flags & CLR_RENDER_NO_RR) != 0;
     V3 pix = v3z();
@@ -203,7 +203,7 @@ template <class Job, class Stack, class Source>
 __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint32_t maxDepth, uint32_t flags,
                                             const Stack& stack, Job& job, Source& src) {
     const bool noRR = (flags & CLR_RENDER_NO_RR) != 0;
-    WideWalk<TexAlpha, Stack> w(S.g, stack, TexAlpha{&S});
+    WideWalk<RareAlpha, Stack> w(S.g, stack, RareAlpha{&S});
     bool live = false;
     uint32_t gx = 0, gy = 0, k = 0;
     Rng rng{};
@@ -317,7 +317,7 @@ __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint3
                                     float x1, x2;
                                     uint32_t flag;
                                     shadow = triTestPacked(S.g.atris, org, dir, lp.face, bound, x1, x2, flag) &&
-                                             !isinf(bound) && !(flag && TexAlpha{&S}.reject(lp.face, x1, x2));
+                                             !isinf(bound) && !(flag && RareAlpha{&S}.reject(lp.face, x1, x2));
                                     boundFace = lp.face;
                                 }
                                 if (shadow)
@@ -428,6 +428,12 @@ struct AdjAcc {
     float sig[kMaxDiffMaterials];
     float em[3];
 };
+// The block's gradient sums (named here rather than passed by pointer, so that
+// the atomics on them are LDS instructions).
+__device__ __forceinline__ AdjAcc& adjAcc() {
+    __shared__ AdjAcc s_acc;
+    return s_acc;
+}
 
 // Oren-Nayar angular factor X of f = rho / pi * (A + B X) (same terms as fx).
 __device__ __forceinline__ float orenNayarX(V3 wo, V3 wi) {
@@ -450,7 +456,6 @@ struct AdjHook {
     const uint16_t* table;  // matPtr -> parameter index + 1 (0: not differentiable)
     uint32_t lightProp;     // lightPtr of the differentiable emitter
     V3 M, adj;              // its emission; dLoss/dpixel / spp
-    AdjAcc* acc;            // block accumulators (LDS)
     int n;
     uint32_t recM[kMaxAdjVertices];
     V3 recPrefix[kMaxAdjVertices], recRho[kMaxAdjVertices];
@@ -458,14 +463,14 @@ struct AdjHook {
 
     __device__ __forceinline__ uint32_t param(uint32_t matPtr, const BSDF& B) const {
         if (B.n != 1 || B.c[0].id != 0u) return 0u;
-        return table[matPtr & 0xFFFFu];
+        return asGlobal(table)[matPtr & 0xFFFFu];
     }
     __device__ __forceinline__ float dlogSigma(uint32_t matPtr, const BSDF& B, const SurfPt& sp, V3 vout,
                                                V3 vin) const {
         const BxDF& f = B.c[0];
         if (f.a == 1.0f) return 0.0f;  // sigma = 0: f = rho / pi
-        const uint8_t* e = S.mat + ((matPtr + 8u + 3u) & ~3u);
-        const float sigma = evalFloat(S.tex + ld<uint32_t>(e + 8), sp.u, sp.v);
+        const uint8_t* e = asGlobal(S.mat) + ((matPtr + 8u + 3u) & ~3u);
+        const float sigma = evalFloat(asGlobal(S.tex) + ld<uint32_t>(e + 8), sp.u, sp.v);
         const V3 wo = toLocal(B.S, B.T, B.N, vout), wi = toLocal(B.S, B.T, B.N, vin);
         const float X = orenNayarX(wo, wi);
         const float s2 = sigma * sigma, qa = s2 + 0.33f, qb = s2 + 0.09f;
@@ -473,14 +478,14 @@ struct AdjHook {
         return (dA + dB * X) / (f.a + f.b * X);
     }
     __device__ __forceinline__ void addAlbedo(uint32_t m, V3 term, V3 rho) const {
-        if (rho.x != 0.0f) atomicAdd(acc->alb + 3 * m + 0, adj.x * term.x / rho.x);
-        if (rho.y != 0.0f) atomicAdd(acc->alb + 3 * m + 1, adj.y * term.y / rho.y);
-        if (rho.z != 0.0f) atomicAdd(acc->alb + 3 * m + 2, adj.z * term.z / rho.z);
+        if (rho.x != 0.0f) atomicAdd(adjAcc().alb + 3 * m + 0, adj.x * term.x / rho.x);
+        if (rho.y != 0.0f) atomicAdd(adjAcc().alb + 3 * m + 1, adj.y * term.y / rho.y);
+        if (rho.z != 0.0f) atomicAdd(adjAcc().alb + 3 * m + 2, adj.z * term.z / rho.z);
     }
     __device__ __forceinline__ void addEmission(V3 term) const {
-        if (M.x != 0.0f) atomicAdd(acc->em + 0, adj.x * term.x / M.x);
-        if (M.y != 0.0f) atomicAdd(acc->em + 1, adj.y * term.y / M.y);
-        if (M.z != 0.0f) atomicAdd(acc->em + 2, adj.z * term.z / M.z);
+        if (M.x != 0.0f) atomicAdd(adjAcc().em + 0, adj.x * term.x / M.x);
+        if (M.y != 0.0f) atomicAdd(adjAcc().em + 1, adj.y * term.y / M.y);
+        if (M.z != 0.0f) atomicAdd(adjAcc().em + 2, adj.z * term.z / M.z);
     }
     __device__ __forceinline__ void emission(V3 term, uint32_t lightPtr) {
         if (lightPtr == lightProp) addEmission(term);
@@ -491,7 +496,7 @@ struct AdjHook {
         const uint32_t m = param(matPtr, B);
         if (m) {
             addAlbedo(m - 1, term, B.c[0].R);
-            atomicAdd(acc->sig + (m - 1), dot(adj, term) * dlogSigma(matPtr, B, sp, vout, vinL));
+            atomicAdd(adjAcc().sig + (m - 1), dot(adj, term) * dlogSigma(matPtr, B, sp, vout, vinL));
         }
     }
     __device__ __forceinline__ void bounce(uint32_t matPtr, const BSDF& B, V3 vout, V3 vin, const SurfPt& sp,
@@ -508,7 +513,7 @@ struct AdjHook {
         for (int k = 0; k < n; ++k) {
             const V3 after = L - recPrefix[k];
             addAlbedo(recM[k], after, recRho[k]);
-            atomicAdd(acc->sig + recM[k], dot(adj, after) * recDlog[k]);
+            atomicAdd(adjAcc().sig + recM[k], dot(adj, after) * recDlog[k]);
         }
         n = 0;
     }
@@ -554,7 +559,7 @@ struct AdjJob : AdjHook {
         if (lightEm) addEmission(term);
         if (lightM) {
             addAlbedo(lightM - 1, term, lightRho);
-            atomicAdd(acc->sig + (lightM - 1), dot(adj, term) * lightDlog);
+            atomicAdd(adjAcc().sig + (lightM - 1), dot(adj, term) * lightDlog);
         }
         if (recorded) recPrefix[n - 1] = pixSoFar;
     }
@@ -677,7 +682,7 @@ __device__ __forceinline__ void renderBatch(const dev::RScene* __restrict__ tabl
     uint32_t tile = nextTile(tileCounter);
     while (tile < tiles) {
         const uint32_t s = tile / tilesPerScene;
-        const dev::RScene S = table[s];
+        const dev::RScene S = dev::tableScene(table, s);
         dev::ImageJob job{reinterpret_cast<uint4*>(states) + npix * s, reinterpret_cast<float4*>(pixels) + npix * s,
                           width};
         TileSource src{tileCounter, width, height, tilesX, s * tilesPerScene, (s + 1) * tilesPerScene, tile};
@@ -818,7 +823,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     uint32_t* __restrict__ tileCounter, uint32_t* __restrict__ spill) {
     constexpr int kLds = WALK == dev::kWalkOrdered ? kAdjLds : dev::kStackDepth;
     __shared__ __align__(8) uint32_t s_stack[kLds * 64];
-    __shared__ dev::AdjAcc s_acc;
+    dev::AdjAcc& s_acc = dev::adjAcc();
     for (uint32_t i = threadIdx.x; i < dev::kMaxDiffMaterials * 3; i += 64) s_acc.alb[i] = 0.0f;
     for (uint32_t i = threadIdx.x; i < dev::kMaxDiffMaterials; i += 64) s_acc.sig[i] = 0.0f;
     if (threadIdx.x < 3) s_acc.em[threadIdx.x] = 0.0f;
@@ -830,7 +835,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const uint8_t* e = S.mat + ((lightProp + 1u + 3u) & ~3u);
         M = dev::evalColor(S.tex + dev::ld<uint32_t>(e + 4), 0.0f, 0.0f);
     }
-    dev::AdjJob job{{S, table, lightProp, M, dev::v3z(), &s_acc, 0}, reinterpret_cast<const uint4*>(states), dLdI,
+    dev::AdjJob job{{S, table, lightProp, M, dev::v3z(), 0}, reinterpret_cast<const uint4*>(states), dLdI,
                     width, 1.0f / (float)spp};
     if constexpr (WALK == dev::kWalkOrdered) {
         renderImage<kLds>(scene, width, height, spp, maxDepth, flags, job, tileCounter, spill, s_stack);

@@ -46,6 +46,32 @@ struct RScene {
     uint32_t* status;          // device status word (stack overflow flag)
 };
 
+// A scene read from a table in memory (see asGlobal).
+__device__ __forceinline__ RScene tableScene(const RScene* table, uint32_t i) {
+    RScene S = table[i];
+    S.g.inodes = asGlobal(S.g.inodes);
+    S.g.leaves = asGlobal(S.g.leaves);
+    S.g.verts = asGlobal(S.g.verts);
+    S.g.faces = asGlobal(S.g.faces);
+    S.g.atris = asGlobal(S.g.atris);
+    S.g.bvh = asGlobal(S.g.bvh);
+    S.g.qnodes = asGlobal(S.g.qnodes);
+    S.normals = asGlobal(S.normals);
+    S.tangents = asGlobal(S.tangents);
+    S.uvs = asGlobal(S.uvs);
+    S.lights = asGlobal(S.lights);
+    S.mat = asGlobal(S.mat);
+    S.tex = asGlobal(S.tex);
+    S.oth = asGlobal(S.oth);
+    S.camera = asGlobal(S.camera);
+    S.envLP = asGlobal(S.envLP);
+    S.lightDist = asGlobal(S.lightDist);
+    S.faceLight = asGlobal(S.faceLight);
+    S.envLightPtr = asGlobal(S.envLightPtr);
+    S.status = asGlobal(S.status);
+    return S;
+}
+
 template <typename T>
 __device__ __forceinline__ T ld(const uint8_t* p) {
     return *reinterpret_cast<const T*>(p);
@@ -155,7 +181,7 @@ __device__ __forceinline__ uint32_t checkerIdx(float u, float v) {
     const uint32_t b = v * 2 > 0 ? (uint32_t)(v * 2) : 0u;
     return (a + b) % 2u;
 }
-__device__ V3 evalColor(const uint8_t* t, float u, float v) {
+__device__ __forceinline__ V3 evalColor(const uint8_t* t, float u, float v) {
     const uint8_t type = t[0];
     if (type == 0) return ld3(t + 16);
     if (type == 4) {
@@ -196,7 +222,7 @@ __device__ V3 evalColor(const uint8_t* t, float u, float v) {
     }
     return v3z();
 }
-__device__ float evalFloat(const uint8_t* t, float u, float v) {
+__device__ __forceinline__ float evalFloat(const uint8_t* t, float u, float v) {
     const uint8_t type = t[0];
     if (type == 6) return ld<float>(t + 4);
     if (type == 7) {
@@ -206,7 +232,7 @@ __device__ float evalFloat(const uint8_t* t, float u, float v) {
     if (type == 8) return t[1] == 0 ? ld<float>(t + 4 + 4 * checkerIdx(u, v)) : 0.0f;
     return 0.0f;
 }
-__device__ float evalAlpha(const uint8_t* t, float u, float v) {
+__device__ __forceinline__ float evalAlpha(const uint8_t* t, float u, float v) {
     const uint8_t type = t[0];
     if (type == 2 || type == 5) {
         const uint32_t w = ld<uint32_t>(t + 4), h = ld<uint32_t>(t + 8);
@@ -293,7 +319,7 @@ struct SurfPt {
 
 // calcHitpointParameters (bvh_traversal.cl:110-158) from the accepted
 // triangle's barycentrics.
-__device__ void hitParams(const RScene& S, V3 org, V3 dir, float t, uint32_t face, float b1i, float b2i,
+__device__ __forceinline__ void hitParams(const RScene& S, V3 org, V3 dir, float t, uint32_t face, float b1i, float b2i,
                           SurfPt& sp) {
     const clr_face& f = S.g.faces[face];
     const V3 p0 = loadV3(S.g.verts, f.p0), p1 = loadV3(S.g.verts, f.p1), p2 = loadV3(S.g.verts, f.p2);
@@ -331,10 +357,8 @@ __device__ void hitParams(const RScene& S, V3 org, V3 dir, float t, uint32_t fac
 }
 
 // Alpha rejection through the face's alpha texture (bvh_traversal.cl:94-105).
-// Not inlined: the walks ask rarely, and the texture lookup inside their loop
-// cost every visit registers and mask arithmetic.
-__device__ __attribute__((noinline)) bool alphaReject(const clr_face* faces, const float* uvs, const uint8_t* tex,
-                                                      uint32_t face, float b1, float b2) {
+__device__ __forceinline__ bool alphaReject(const clr_face* faces, const float* uvs, const uint8_t* tex, uint32_t face,
+                                            float b1, float b2) {
     const clr_face& f = faces[face];
     if (f.uv0 == kNone || f.alphaTexPtr == kNone) return false;
     const float b0 = 1.0f - b1 - b2;
@@ -349,6 +373,19 @@ struct TexAlpha {
     const RScene* S;
     __device__ __forceinline__ bool reject(uint32_t face, float b1, float b2) const {
         return alphaReject(S->g.faces, S->uvs, S->tex, face, b1, b2);
+    }
+};
+// The same out of line, for WideWalk: it asks only for triangles with an alpha
+// texture, and the lookup inside its loop cost every visit registers and mask
+// arithmetic.
+__device__ __attribute__((noinline)) bool alphaRejectCall(const clr_face* faces, const float* uvs, const uint8_t* tex,
+                                                          uint32_t face, float b1, float b2) {
+    return alphaReject(asGlobal(faces), asGlobal(uvs), asGlobal(tex), face, b1, b2);
+}
+struct RareAlpha {
+    const RScene* S;
+    __device__ __forceinline__ bool reject(uint32_t face, float b1, float b2) const {
+        return alphaRejectCall(S->g.faces, S->uvs, S->tex, face, b1, b2);
     }
 };
 
@@ -366,7 +403,7 @@ __device__ __forceinline__ bool intersect(const RScene& S, V3 org, V3 dir, const
     bool over = false;
     uint32_t face;
     if constexpr (WALK == kWalkOrdered)  // over the 4-wide records (every render builds them)
-        face = wideHit(S.g, org, dir, t, stack, b1, b2, TexAlpha{&S}, over);
+        face = wideHit(S.g, org, dir, t, stack, b1, b2, RareAlpha{&S}, over);
     else if constexpr (WALK == kWalkMidpoint)
         face = bvhWalk<false, false>(S.g, org, dir, t, stack, st, &b1, &b2, TexAlpha{&S}, &over);
     else
@@ -459,7 +496,7 @@ __device__ __forceinline__ void bxPut(BSDF& B, int i, const BxDF& f) {
 }
 
 template <bool REG = false>
-__device__ void bsdfAlloc(const RScene& S, uint32_t off, const SurfPt& sp, BSDF& B) {
+__device__ __forceinline__ void bsdfAlloc(const RScene& S, uint32_t off, const SurfPt& sp, BSDF& B) {
     const uint8_t* m = S.mat + off;
     B.n = m[0];
     B.N = sp.sN;
@@ -543,7 +580,8 @@ __device__ void bsdfAlloc(const RScene& S, uint32_t off, const SurfPt& sp, BSDF&
     }
 }
 
-__device__ V3 fresnel(const uint8_t* fr, float cosi) {
+__device__ __forceinline__ V3 fresnel(const uint8_t* record, float cosi) {
+    const uint8_t* fr = asGlobal(record);
     const uint8_t type = fr[0];
     if (type == 0) return v3s(1.0f);
     if (type == 1) {
@@ -611,7 +649,7 @@ __device__ __forceinline__ V3 halfPlusZ(V3 wo, V3 wi) {
     return h.z < 0.0f ? -h : h;
 }
 
-__device__ V3 fx(const BxDF f, const uint8_t* oth, V3 wo, V3 wi) {
+__device__ __forceinline__ V3 fx(const BxDF f, const uint8_t* oth, V3 wo, V3 wi) {
     if (wi.z * wo.z <= 0.0f) return v3z();
     switch (f.id) {
         case 0: {
@@ -656,7 +694,7 @@ __device__ V3 fx(const BxDF f, const uint8_t* oth, V3 wo, V3 wi) {
     }
 }
 
-__device__ float fxPdf(const BxDF& f, V3 wo, V3 wi) {
+__device__ __forceinline__ float fxPdf(const BxDF& f, V3 wo, V3 wi) {
     switch (f.id) {
         case 0:
         case 5:
@@ -685,7 +723,7 @@ __device__ float fxPdf(const BxDF& f, V3 wo, V3 wi) {
     }
 }
 
-__device__ V3 sampleFx(const BxDF& f, const uint8_t* oth, V3 wo, float u0, float u1, V3& wi, float& pdf) {
+__device__ __forceinline__ V3 sampleFx(const BxDF& f, const uint8_t* oth, V3 wo, float u0, float u1, V3& wi, float& pdf) {
     switch (f.id) {
         case 0:
         case 5:
@@ -797,7 +835,7 @@ __device__ __forceinline__ bool hasNonSpecular(const BSDF& B) {
 }
 
 template <bool REG = false>
-__device__ V3 sampleFs(const BSDF& B, V3 vout, float uc, float u0, float u1, V3& vin, float& pdf,
+__device__ __forceinline__ V3 sampleFs(const BSDF& B, V3 vout, float uc, float u0, float u1, V3& vin, float& pdf,
                        uint32_t& sampledType) {
     const V3 wo = toLocal(B.S, B.T, B.N, vout);
     const uint32_t which = randUInt(uc, (uint32_t)B.n);
@@ -828,7 +866,7 @@ __device__ V3 sampleFs(const BSDF& B, V3 vout, float uc, float u0, float u1, V3&
     return ret;
 }
 template <bool REG = false>
-__device__ V3 evalFs(const BSDF& B, V3 vout, V3 vin) {
+__device__ __forceinline__ V3 evalFs(const BSDF& B, V3 vout, V3 vin) {
     const V3 wo = toLocal(B.S, B.T, B.N, vout), wi = toLocal(B.S, B.T, B.N, vin);
     const uint32_t flags = dot(vin, B.NG) * dot(vout, B.NG) > 0 ? (kAll & ~kTrans) : (kAll & ~kRefl);
     V3 r = v3z();
@@ -839,7 +877,7 @@ __device__ V3 evalFs(const BSDF& B, V3 vout, V3 vin) {
     return r;
 }
 template <bool REG = false>
-__device__ float evalFsPdf(const BSDF& B, V3 vout, V3 vin) {
+__device__ __forceinline__ float evalFsPdf(const BSDF& B, V3 vout, V3 vin) {
     const V3 wo = toLocal(B.S, B.T, B.N, vout), wi = toLocal(B.S, B.T, B.N, vin);
     float p = 0.0f;
     for (int i = 0; i < B.n; ++i) {
@@ -857,7 +895,7 @@ struct EDF {
            // apart from the one-sided cosine test of area emitters)
     V3 N, S, T, NG;
 };
-__device__ void edfArea(const RScene& Sc, uint32_t off, const SurfPt& lp, float u, float v, EDF& E) {
+__device__ __forceinline__ void edfArea(const RScene& Sc, uint32_t off, const SurfPt& lp, float u, float v, EDF& E) {
     const uint8_t* info = Sc.mat + off;
     E.env = false;
     E.n = info[0];
@@ -875,7 +913,7 @@ __device__ void edfArea(const RScene& Sc, uint32_t off, const SurfPt& lp, float 
         p += 8;
     }
 }
-__device__ void edfEnv(const RScene& Sc, float u, float v, EDF& E) {
+__device__ __forceinline__ void edfEnv(const RScene& Sc, float u, float v, EDF& E) {
     E.env = true;
     E.n = Sc.envLP[0];
     E.L = v3z();
@@ -900,7 +938,7 @@ __device__ __forceinline__ float absCosEDF(const EDF& E, V3 v) { return E.env ? 
 
 // Light sample (light.cl:138-245). Returns the light point in `lp` (face or
 // kNone for the environment) and multiplies areaPDF in.
-__device__ void sampleLight(const RScene& Sc, float ul, float u0, float u1, SurfPt& lp, bool& atInf, EDF& E,
+__device__ __forceinline__ void sampleLight(const RScene& Sc, float ul, float u0, float u1, SurfPt& lp, bool& atInf, EDF& E,
                             float& areaPDF) {
     const uint32_t li = sampleDiscrete(Sc.lightDist, ul, areaPDF);
     const clr_light_info L = Sc.lights[li];
@@ -962,7 +1000,7 @@ __device__ void sampleLight(const RScene& Sc, float ul, float u0, float u1, Surf
 }
 
 // getAreaPDF (light.cl:247-292).
-__device__ float areaPdfOfFace(const RScene& Sc, uint32_t face) {
+__device__ __forceinline__ float areaPdfOfFace(const RScene& Sc, uint32_t face) {
     const uint32_t li = Sc.faceLight[face];
     if (li == kNone) return 0.0f;
     const clr_face& f = Sc.g.faces[face];
@@ -970,7 +1008,7 @@ __device__ float areaPdfOfFace(const RScene& Sc, uint32_t face) {
     const V3 ng = cross(p1 - p0, p2 - p0);
     return 1.0f / (0.5f * length3(ng)) * probDiscrete(Sc.lightDist, li);
 }
-__device__ float areaPdfEnv(const RScene& Sc, float u, float v) {
+__device__ __forceinline__ float areaPdfEnv(const RScene& Sc, float u, float v) {
     float areaPDF = 0.0f;
     const uint32_t num = Sc.envLP[0];
     uint32_t p = (uint32_t)(Sc.envLP - Sc.mat) + 1;

@@ -41,6 +41,14 @@ __device__ __forceinline__ V3 loadV3(const clr_float3* p, uint32_t i) {
     return {v.x, v.y, v.z};
 }
 
+// A pointer read from memory is generic to the compiler, and every access
+// through it a flat one, which takes longer and waits for LDS too. All scene
+// pointers are to global memory.
+template <class T>
+__device__ __forceinline__ T* asGlobal(T* p) {
+    return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<uintptr_t>(p);
+}
+
 // Traversal layout derived from the drop-in nodes for the ordered walk:
 // per internal node i, 4 x float4 = {min of child 0 | ref0, max of child 0 |
 // ref1, min of child 1, max of child 1} (refs in the .w lanes as bits: an
@@ -163,12 +171,15 @@ struct SpillStack {
     int stride;
     uint32_t* spill;
     size_t spillStride;
+    // Two separate accesses, never one through a pointer that may be either.
     __device__ __forceinline__ void put(int k, uint32_t v) const {
         if (k < L) lds[k * stride] = v;
-        else spill[(size_t)(k - L) * spillStride] = v;
+        else __builtin_nontemporal_store(v, spill + (size_t)(k - L) * spillStride);
     }
     __device__ __forceinline__ uint32_t get(int k) const {
-        return k < L ? lds[k * stride] : spill[(size_t)(k - L) * spillStride];
+        uint32_t v = lds[min(k, L - 1) * stride];
+        if (k >= L) v = __builtin_nontemporal_load(spill + (size_t)(k - L) * spillStride);
+        return v;
     }
 };
 
@@ -768,7 +779,11 @@ struct PairStack {
 // Against the counting walk in the same kernels: 2^22 random rays on 2^24
 // triangles 8.72 -> 8.10 ms, 512x512 at 8 spp of the differentiation scene
 // 31.9 -> 26.3 ms (forward and adjoint), 640x360 at 16 spp of the showcase
-// scene on the wavefront renderer 24.3 -> 21.4 ms.
+// scene on the wavefront renderer 24.3 -> 21.4 ms (with float records). Byte
+// records, the branch-free leaf test, the stack without flat accesses and the
+// alpha lookup out of line: the random rays 9.99 -> 8.33 ms (2.79 -> 1.85 ->
+// 1.2 ms of it building records), 1080p at 32 spp on the megakernel 124 ->
+// 107 ms.
 template <class Alpha, class Stack>
 struct WideWalk {
     const float4* qn;
@@ -784,10 +799,10 @@ struct WideWalk {
     static constexpr uint32_t kAny = 1u, kOver = 2u;
 
     __device__ __forceinline__ WideWalk(const GeomScene& g, const Stack& s_, const Alpha& a_)
-        : qn(g.qnodes), tris(g.atris), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
+        : qn(asGlobal(g.qnodes)), tris(asGlobal(g.atris)), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
     __device__ __forceinline__ void rebind(const GeomScene& g, const Alpha& a_) {
-        qn = g.qnodes;
-        tris = g.atris;
+        qn = asGlobal(g.qnodes);
+        tris = asGlobal(g.atris);
         limit = 2u * g.n + 2u;
         alpha = a_;
     }

@@ -93,7 +93,7 @@ __device__ __forceinline__ void slotScene(const WfArgs& A, uint32_t v, RScene& S
         const uint32_t sc = v / A.posPerScene;
         vLocal = v - sc * A.posPerScene;
         pixBase = sc * A.width * A.height;
-        S = A.table[sc];
+        S = tableScene(A.table, sc);
     } else {
         vLocal = v;
         pixBase = 0;
@@ -342,15 +342,15 @@ __global__ __launch_bounds__(256) void k_wf_extend(WfArgs A, uint32_t in) {
         const PS stk0{lds, (int)blockDim.x, spill, lanes};
         const PS stk1{lds + LD / 2 * blockDim.x, (int)blockDim.x,
                       spill + (size_t)(kStackPairs - kMinLdsDepth) / 2 * lanes, lanes};
-        using W = WideWalk<TexAlpha, PS>;
-        W w0(S0->g, stk0, TexAlpha{S0}), w1(S0->g, stk1, TexAlpha{S0});
+        using W = WideWalk<RareAlpha, PS>;
+        W w0(S0->g, stk0, RareAlpha{S0}), w1(S0->g, stk1, RareAlpha{S0});
         WavePool pool(n);
         bool busy0 = false, busy1 = false;
         uint32_t j0 = 0, j1 = 0;
         auto start = [&](W& w, uint32_t j) {
             if constexpr (BATCH) {
                 const RScene* Sp = A.table + (chunk + B.rqSlot[in][j]) / A.posPerScene;
-                w.rebind(Sp->g, TexAlpha{Sp});
+                w.rebind(Sp->g, RareAlpha{Sp});
             }
             w.begin(xyz(B.rqOrg[in][j]), xyz(B.rqDir[in][j]), INFINITY);
         };
@@ -621,15 +621,15 @@ __global__ __launch_bounds__(256) void k_wf_shadow(WfArgs A, uint32_t in) {
         const PS stk0{lds, (int)blockDim.x, spill, lanes};
         const PS stk1{lds + LD / 2 * blockDim.x, (int)blockDim.x,
                       spill + (size_t)(kStackPairs - kMinLdsDepth) / 2 * lanes, lanes};
-        using W = WideWalk<TexAlpha, PS>;
-        W w0(S0->g, stk0, TexAlpha{S0}), w1(S0->g, stk1, TexAlpha{S0});
+        using W = WideWalk<RareAlpha, PS>;
+        W w0(S0->g, stk0, RareAlpha{S0}), w1(S0->g, stk1, RareAlpha{S0});
         WavePool pool(n);
         bool busy0 = false, busy1 = false;
         uint32_t i0 = 0, i1 = 0, target0 = kNone, target1 = kNone;
         auto start = [&](W& w, uint32_t i, uint32_t& target) {
             if constexpr (BATCH) {
                 const RScene* Sp = A.table + (chunk + B.sqSlot[i]) / A.posPerScene;
-                w.rebind(Sp->g, TexAlpha{Sp});
+                w.rebind(Sp->g, RareAlpha{Sp});
             }
             const float4 o4 = B.sqOrg[i];
             target = __float_as_uint(o4.w);
