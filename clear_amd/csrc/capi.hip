@@ -47,26 +47,6 @@ int ensurePool(clr_ctx* ctx, size_t bytes) {
     return CLR_OK;
 }
 
-int ensureExchange(clr_ctx* ctx, size_t nodes) {
-    if (nodes == 0) nodes = 1;
-    if (ctx->xchgNodes >= nodes) return CLR_OK;
-    int rc = hipCheck(ctx, hipDeviceSynchronize(), "exchange regrow sync");
-    if (rc) return rc;
-    const size_t want = nodes + nodes / 8;
-    if (ctx->xchg) (void)hipFree(ctx->xchg);
-    ctx->xchg = nullptr;
-    ctx->xchgNodes = 0;
-    hipError_t e = hipMalloc(&ctx->xchg, want * 6 * sizeof(uint64_t));
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->xchg = nullptr;
-        return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "hierarchy exchange buffer");
-    }
-    ctx->xchgNodes = want;
-    fillZero(reinterpret_cast<uint32_t*>(ctx->xchg), ctx->xchgNodes * 12, nullptr);
-    return hipCheck(ctx, hipDeviceSynchronize(), "exchange clear");
-}
-
 int ensureRenderScratch(clr_ctx* ctx, uint32_t numFaces) {
     if (!ctx->renderWords) {
         hipError_t e = hipMalloc(&ctx->renderWords, 64 * sizeof(uint32_t));
@@ -167,7 +147,7 @@ int clr_create(clr_ctx** out, int device) {
         (void)hipGetLastError();
         ctx->numCUs = 0;
     }
-    // The status and build-epoch words exist from the start, so no entry
+    // The status words exist from the start, so no entry
     // point allocates them while a caller's stream is being captured.
     if (ensureStatus(ctx) != CLR_OK) {
         clr_destroy(ctx);
@@ -186,7 +166,6 @@ int clr_destroy(clr_ctx* ctx) {
         DeviceScope ds(ctx->device);
         (void)hipDeviceSynchronize();
         if (ctx->pool) (void)hipFree(ctx->pool);
-        if (ctx->xchg) (void)hipFree(ctx->xchg);
         if (ctx->devStatus) (void)hipFree(ctx->devStatus);
         if (ctx->faceLight) (void)hipFree(ctx->faceLight);
         if (ctx->renderWords) (void)hipFree(ctx->renderWords);
@@ -325,8 +304,7 @@ int clr_lbvh_reserve(clr_ctx* ctx, uint32_t maxFaces, uint32_t numBitsPerDim) {
         return fail(ctx, CLR_ERR_UNSUPPORTED, "reserve size out of range");
     DeviceScope ds(ctx->device);
     if (ds.err != hipSuccess) return hipCheck(ctx, ds.err, "set device");
-    const int rc = ensurePool(ctx, lbvhScratchBytes(maxFaces, numBitsPerDim));
-    return rc ? rc : ensureExchange(ctx, maxFaces);
+    return ensurePool(ctx, lbvhScratchBytes(maxFaces, numBitsPerDim));
 }
 
 int clr_lbvh_reserve_segmented(clr_ctx* ctx, uint32_t maxTris, uint32_t numSegments, uint32_t numBitsPerDim) {
@@ -336,8 +314,7 @@ int clr_lbvh_reserve_segmented(clr_ctx* ctx, uint32_t maxTris, uint32_t numSegme
         return fail(ctx, CLR_ERR_UNSUPPORTED, "reserve size out of range");
     DeviceScope ds(ctx->device);
     if (ds.err != hipSuccess) return hipCheck(ctx, ds.err, "set device");
-    const int rc = ensurePool(ctx, lbvhSegScratchBytes(maxTris, numSegments, numBitsPerDim));
-    return rc ? rc : ensureExchange(ctx, maxTris);
+    return ensurePool(ctx, lbvhSegScratchBytes(maxTris, numSegments, numBitsPerDim));
 }
 
 int clr_lbvh_build_segmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffsets,

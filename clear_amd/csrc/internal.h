@@ -31,16 +31,9 @@ struct clr_ctx {
     bool profiling = false;
     hipEvent_t events[kMaxProfiledBuilds][kStageEvents] = {};
     int profiledBuilds = 0;
-    // Box hand-off buffer of the bottom-up hierarchy pass: six 64-bit words
-    // (float bits | build epoch) per internal node. Only ever written with
-    // epoch-tagged words, zeroed when (re)allocated and when the epoch wraps,
-    // so a stale word can never carry the current epoch.
-    uint64_t* xchg = nullptr;
-    size_t xchgNodes = 0;
     // 64 device words, allocated by clr_create: word kWordStatus holds the
     // device-side failure flags (bounded spin exceeded, stack overflow), read
-    // back by clr_device_status; word kWordEpoch the LBVH build epoch, which
-    // the build's kernels advance and read on the build's stream.
+    // back by clr_device_status.
     uint32_t* devStatus = nullptr;
     // Render scratch: face -> first light index, and 64 small device words
     // (word 0: first light at infinity).
@@ -81,21 +74,16 @@ int ensurePool(clr_ctx* ctx, size_t bytes);
 
 // Bits of the device status word.
 constexpr uint32_t kStatusLookbackSpin = 1u << 0;
-constexpr uint32_t kStatusExchangeSpin = 1u << 1;
 constexpr uint32_t kStatusStackOverflow = 1u << 2;
 constexpr uint32_t kStatusHierarchy = 1u << 3;
 constexpr uint32_t kStatusSegments = 1u << 4;
 // Upper bound on any device-side wait loop (iterations of one atomic load).
 constexpr uint32_t kSpinLimit = 1u << 22;
 
-// Grows the box hand-off buffer to `nodes` entries (synchronous when it has
-// to reallocate; the new buffer is zeroed).
-int ensureExchange(clr_ctx* ctx, size_t nodes);
 // Allocates the device status words if clr_create has not (synchronous).
 int ensureStatus(clr_ctx* ctx);
 // Indices into clr_ctx::devStatus.
 constexpr uint32_t kWordStatus = 0;
-constexpr uint32_t kWordEpoch = 1;
 constexpr uint32_t kWordMegaTiles = 2;  // next 8x8 tile of a megakernel render
 
 // Bump allocator over the pool (256-B aligned sub-buffers).

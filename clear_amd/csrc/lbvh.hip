@@ -17,13 +17,12 @@
 //   onesweep    one launch per 8-bit digit: stable LSD pass with wave64
 //               ballot ranking and decoupled look-back (the reference spends
 //               numBitsPerDim passes of 8 launches on 3-bit digits)
-//   hierarchy   one bottom-up pass that derives the Karras 2012 binary radix
-//               tree (node numbering of constructBinaryRadixTree,
-//               lbvh_construction.cl:342-410) and the refit boxes
-//               (calcNodeAABBs, :415-492) together: each leaf climbs, the
-//               second arrival at a parent merges fmin/fmax(left, right) and
-//               continues; release/acquire on the arrival word orders the box
-//               writes (the reference's atomic_inc has no fence).
+//   hierarchy   derives the Karras 2012 binary radix tree (node numbering of
+//               constructBinaryRadixTree, lbvh_construction.cl:342-410) and
+//               the refit boxes (calcNodeAABBs, :415-492) together: inside a
+//               block of leaves each leaf climbs and the second arrival at a
+//               parent merges fmin/fmax(left, right); the few nodes that
+//               cross blocks are then found and boxed directly, each on its own
 //
 // A node covering sorted range [l, r] is the left child of its parent when the
 // common prefix across its right boundary, delta(r, r+1), exceeds the one
@@ -142,29 +141,13 @@ __device__ __forceinline__ float waveMax(float v) {
 
 // ---------------------------------------------------------------- init ----
 // Clears `count` words (histograms, look-back words) and sets the scene box
-// to empty. With `epochWord`: when the build epoch is about to wrap to 0
-// (every 2^32 - 1 builds) it also clears the hierarchy's exchange words, so
-// that no word left by an earlier build carries the next epoch. No kernel
-// writes the epoch word while this one runs, so every block reads one value.
-__global__ __launch_bounds__(kBlock) void k_init(uint32_t* words, size_t count, uint32_t* sceneOrd,
-                                                 const uint32_t* epochWord = nullptr,
-                                                 uint32_t* xchgWords = nullptr, size_t xchgCount = 0) {
+// to empty.
+__global__ __launch_bounds__(kBlock) void k_init(uint32_t* words, size_t count, uint32_t* sceneOrd) {
     size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
     size_t stride = (size_t)gridDim.x * kBlock;
     for (size_t j = i; j < count; j += stride) words[j] = 0u;
-    if (epochWord && *epochWord == 0xFFFFFFFFu)
-        for (size_t j = i; j < xchgCount; j += stride) xchgWords[j] = 0u;
     if (sceneOrd && blockIdx.x == 0 && threadIdx.x < 6)
         sceneOrd[threadIdx.x] = threadIdx.x < 3 ? ordOf(INFINITY) : ordOf(-INFINITY);
-}
-
-// The build epoch tags the hierarchy's box hand-off words. It lives in device
-// memory and advances once per build on the build's own stream (in the
-// kernel after k_init), never 0, so a build replayed from a captured graph
-// still gets a fresh epoch.
-__device__ __forceinline__ void advanceEpoch(uint32_t* epochWord) {
-    const uint32_t e = *epochWord;
-    *epochWord = e == 0xFFFFFFFFu ? 1u : e + 1u;
 }
 
 // -------------------------------------------------------------- bounds ----
@@ -181,9 +164,7 @@ __global__ __launch_bounds__(kBlock) void k_bounds(const float* __restrict__ tri
                                                    float4* __restrict__ boxesOut,
                                                    float* __restrict__ cx, float* __restrict__ cy,
                                                    float* __restrict__ cz,
-                                                   uint32_t* __restrict__ sceneOrd,
-                                                   uint32_t* __restrict__ epochWord) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) advanceEpoch(epochWord);
+                                                   uint32_t* __restrict__ sceneOrd) {
     float lo[3] = {INFINITY, INFINITY, INFINITY};
     float hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
@@ -342,16 +323,6 @@ __global__ __launch_bounds__(kBlock) void k_morton(const float* __restrict__ cx,
 }
 
 // ------------------------------------------------------------ onesweep ----
-__device__ __forceinline__ void writeLeaf(clr_lbvh_leaf* leaves, uint32_t i, const Box& b,
-                                          uint32_t obj) {
-    uint4* o = reinterpret_cast<uint4*>(leaves + i);
-    o[0] = make_uint4(__float_as_uint(b.lo[0]), __float_as_uint(b.lo[1]),
-                      __float_as_uint(b.lo[2]), 0u);
-    o[1] = make_uint4(__float_as_uint(b.hi[0]), __float_as_uint(b.hi[1]),
-                      __float_as_uint(b.hi[2]), 0u);
-    o[2] = make_uint4(obj, 0u, 0u, 0u);
-}
-
 // One stable LSD pass on the 8-bit digit at `shift`. FIRST generates the
 // payload (original index) instead of reading it.
 template <typename KeyT, bool FIRST>
@@ -532,18 +503,6 @@ __device__ __forceinline__ int clzKey<uint64_t>(uint64_t v) {
     return __clzll((long long)v);
 }
 
-// delta(x, x+1) over extended keys (key, sorted position); the reference's
-// _numCommonBits (lbvh_construction.cl:322-332) for adjacent positions.
-// `base` is the first sorted position of x's scene (0 for a single build):
-// equal keys fall back to the scene-local positions, so a scene built inside a
-// segmented build gets the tree it gets alone.
-template <typename KeyT>
-__device__ __forceinline__ int deltaAdj(const KeyT* __restrict__ k, uint32_t x, int keyBits, uint32_t base = 0) {
-    const KeyT a = k[x], b = k[x + 1];
-    if (a != b) return clzKey<KeyT>(a ^ b) - (int)(8 * sizeof(KeyT)) + keyBits;
-    return keyBits + __clz((int)((x - base) ^ (x + 1u - base)));
-}
-
 // Segment view of a segmented build: per sorted position its scene, per scene
 // its first position (segOff[s]) and end (segOff[s + 1]). Scenes keep their
 // input ranges through the sort (scene id is the key's top digit), so a
@@ -554,23 +513,13 @@ struct SegView {
     const uint32_t* valid;  // 0: the scene offsets were rejected, nothing is built
 };
 
-// delta(x, x+1), -1 outside [0, n) and, in a segmented build, across scenes.
-template <typename KeyT, bool SEG>
-__device__ __forceinline__ int deltaAt(const KeyT* __restrict__ k, int64_t x, uint32_t n, int keyBits,
-                                       const SegView& sv) {
-    if (x < 0 || x + 1 >= (int64_t)n) return -1;
-    if constexpr (SEG) {
-        const uint32_t s = sv.segOf[x];
-        if (sv.segOf[x + 1] != s) return -1;
-        return deltaAdj<KeyT>(k, (uint32_t)x, keyBits, sv.segOff[s]);
-    } else {
-        return deltaAdj<KeyT>(k, (uint32_t)x, keyBits);
-    }
-}
-
-// deltaAt with unconditional loads (an index outside [0, n - 1) reads
-// position 0 and the result is -1), so that a thread's loads for several x
-// can be in flight together.
+// delta(x, x+1) over extended keys (key, sorted position); the reference's
+// _numCommonBits (lbvh_construction.cl:322-332) for adjacent positions. Equal
+// keys fall back to the scene-local positions, so a scene built inside a
+// segmented build gets the tree it gets alone. -1 outside [0, n) and, in a
+// segmented build, across scenes. The loads are unconditional (an index outside
+// [0, n - 1) reads position 0 and the result is -1), so that a thread's loads
+// for several x can be in flight together.
 template <typename KeyT, bool SEG>
 __device__ __forceinline__ int deltaAtLoaded(const KeyT* __restrict__ k, int64_t x, uint32_t n, int keyBits,
                                              const SegView& sv) {
@@ -603,106 +552,87 @@ __device__ __forceinline__ void writeNode(clr_lbvh_inode* nodes, uint32_t idx, c
     o[2] = make_uint4(flags, split - base, split + 1u - base, 0u);
 }
 
-__device__ __forceinline__ Box leafBox(const clr_lbvh_leaf* leaves, uint32_t i) {
-    const float4* p = reinterpret_cast<const float4*>(leaves + i);
-    const float4 a = p[0], b = p[1];
-    Box r;
-    r.lo[0] = a.x; r.lo[1] = a.y; r.lo[2] = a.z;
-    r.hi[0] = b.x; r.hi[1] = b.y; r.hi[2] = b.z;
-    return r;
-}
-
-// Box hand-off between the two children of a node. Every internal node
-// publishes its box before it arrives at its parent, as six 64-bit words
-// (float bits | epoch) written with relaxed agent-scope atomics (plain sc1
-// stores on gfx950; an acq_rel exchange would instead write back and
-// invalidate the whole per-XCD L2 at every step). The second arrival polls the
-// sibling's words until they carry this build's epoch: the sibling issued its
-// stores before its own arrival, which this thread has already observed, so
-// the wait ends; kSpinLimit only guards against a bug.
-__device__ __forceinline__ void publishBox(uint64_t* slot, const Box& b, uint32_t epoch) {
-    const uint64_t tag = (uint64_t)epoch << 32;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        __hip_atomic_store(slot + k, tag | __float_as_uint(b.lo[k]), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(slot + 3 + k, tag | __float_as_uint(b.hi[k]), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-__device__ __forceinline__ Box awaitBox(const uint64_t* slot, uint32_t epoch,
-                                        uint32_t* devStatus) {
-    uint64_t w[6];
-    // All six words in flight at once; re-poll only while some are stale.
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-        w[k] = __hip_atomic_load(slot + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t spins = 0;
-    while (true) {
-        bool fresh = true;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) fresh &= (uint32_t)(w[k] >> 32) == epoch;
-        if (fresh) break;
-        if (++spins >= kSpinLimit) {
-            atomicOr(devStatus, kStatusExchangeSpin);
-            break;
-        }
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-            if ((uint32_t)(w[k] >> 32) != epoch)
-                w[k] = __hip_atomic_load(slot + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    Box b;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        b.lo[k] = __uint_as_float((uint32_t)w[k]);
-        b.hi[k] = __uint_as_float((uint32_t)w[3 + k]);
-    }
-    return b;
-}
-
 // Bottom-up topology + refit in two phases.
 //
-// Phase 1 (k_hier_local): block b owns leaves [bs, be) (kLocalLeaves per
-// block, kHierThreads threads) and completes every node whose range lies
-// inside them. Arrival slots for splits bs..be-2, boxes and boundary deltas
-// live in LDS. The climb runs in synchronous steps over a queue of climbers
-// (a climber holds a completed node [l, r]; at first every leaf): in a step
-// each climber finds its parent (split r if delta(r) > delta(l-1), else l-1),
-// exchanges its far end into the parent's slot, and the second arrival
-// completes the parent (box = left child's box joined with the right's),
-// writes its record at its index (r if the parent is itself a left child,
-// else l; the root of the range at 0) and enqueues it. The queue is compacted
-// every step, so lanes are spent on live climbs only (a lane per leaf would
-// keep each wave stepping as long as its longest chain). Boxes: slot k holds
-// leaf k's box until internal node k is completed (leaf k lies inside node k
-// and was joined into its parent before). A climb whose parent splits at a
-// block boundary (bs-1 or be-1) stops and leaves a pending record (at most two
-// per block); after the last step the block writes the global arrival words
-// of every slot it did not complete: the far end of the one child that
-// arrived (publishing that child's box) or empty, and empty for the split
-// between it and the next block. Those are all the words phase 2 reads, so no
-// earlier pass clears them.
-// Phase 2 (k_hier_global): one thread per pending record continues with the
-// global epoch-tagged protocol. Only nodes whose range crosses a block
-// boundary (a small fraction) are finished there.
+// Phase 1 (k_hier_local): block b owns leaves [bs, be) (`B` per block, T
+// threads) and completes every node whose range lies inside them. Arrival slots
+// for splits bs..be-2, boxes and boundary deltas live in LDS. The climb runs in
+// synchronous steps over a queue of climbers (a climber holds a completed node
+// [l, r]; at first every leaf): in a step each climber finds its parent (split r
+// if delta(r) > delta(l-1), else l-1), exchanges its far end into the parent's
+// slot, and the second arrival completes the parent (box = left child's box
+// joined with the right's), whose record goes to its index (r if the parent is
+// itself a left child, else l; the root of the range at 0) and which is enqueued.
+// The queue is compacted every step, so lanes are spent on live climbs only (a
+// lane per leaf would keep each wave stepping as long as its longest chain).
+// Boxes: slot k holds leaf k's box until internal node k is completed (leaf k
+// lies inside node k and was joined into its parent before). A climb whose
+// parent splits at a block boundary (bs-1 or be-1) stops.
+//
+// What is left are the block's open splits: the boundaries x in [bs, be-1]
+// whose node reaches beyond the block (be-1 always does). They are few (their
+// deltas fall strictly towards the block's smallest and rise strictly after
+// it) and the stretches between them are finished subtrees. The block writes
+// the list of them (position, delta), with the union of the block's leaves up
+// to each and after each, and the block's own union and smallest delta.
+//
+// Phase 2 (k_hier_global): the node with split x covers (y, z], where y and z are
+// the nearest boundaries left and right of x with a smaller delta (of the keys
+// under one prefix, the one boundary of the smallest delta is the split). A lane
+// per open split finds y and z in its own block's list, or as the nearest block
+// with a smaller delta and the entry in that block's list, and unites the part
+// of the first block, the blocks between and the part of the last one.
+// Searching and uniting over blocks go through groups of 64 (k_hier_levels),
+// so a node costs a few dependent loads wherever its ends lie. The chain of
+// exchanges that climbed these nodes one above the other (up to 31 levels of two
+// device-wide round trips) took 118 us at 2^24 triangles, 88 at 3.1 M and 48 at
+// 35 k; k_hier_global takes 36, 20 and 12 us, a launch of k_hier_levels 5.
+// Boxes are united left to right throughout. omin / omax keep the left operand
+// on ties and skip NaNs, so they are associative (not commutative) and the box of
+// a range does not depend on how its leaves are grouped.
 constexpr int kLocalLeaves = 1024;
 constexpr int kHierThreads = 256;
-constexpr int kHierPer = kLocalLeaves / kHierThreads;
-static_assert(kLocalLeaves % kHierThreads == 0 && kLocalLeaves <= 65536, "hierarchy block shape");
 constexpr uint32_t kDone = 0xFFFFFFFEu;
-constexpr uint32_t kAuxFlagShift = 10;  // log2(kLocalLeaves)
+constexpr uint32_t kAuxFlagShift = 10;
 constexpr uint32_t kAuxEmpty = 0xFFFFu;
-static_assert((1u << kAuxFlagShift) == (uint32_t)kLocalLeaves, "completed-node record layout");
+static_assert((1u << kAuxFlagShift) >= (uint32_t)kLocalLeaves, "completed-node record layout");
+// Smaller blocks where there are few: shorter climbs, more CUs. Build times with
+// 256 / 1024 leaves per block (us, 60-bit keys): 106 / 111 at 10^4 triangles, 136 /
+// 143 at 70,000, 159 / 167 at 2^17, 238 / 241 at 2^19, 314 / 307 at 2^20 (more
+// entries cross blocks). One block needs no second phase (1000 triangles: 84 / 82).
+constexpr int kSmallLeaves = 256;
+constexpr uint32_t kSmallBuild = 1u << 19;  // up to this many triangles, beyond one block's
+inline uint32_t localLeavesFor(uint32_t n) {
+    return n > (uint32_t)kLocalLeaves && n <= kSmallBuild ? kSmallLeaves : kLocalLeaves;
+}
 
-struct Pending {
-    uint32_t valid, l, r, split, internal;  // split: unused (a pending node is never a root)
-    int dl, dr;
-    float box[6];
-    uint32_t pad[3];
+// Entries of a block's list: at most one open split per delta value on either
+// side of the smallest (deltas are below keyBits + 32 <= 95), the first and last
+// scene boundary, and be - 1.
+constexpr uint32_t kOpenCap = 256;
+constexpr int kMaxLevels = 5;  // blocks in groups of 64: 2^30 leaves make 2^20 blocks, 4 levels
+struct BoxRec {  // 32 bytes
+    float4 a;    // lo.xyz, hi.x
+    float4 b;    // hi.yz
 };
-static_assert(sizeof(Pending) == 64, "pending record layout");
+// Level 0: blocks; level k: groups of 64 of level k - 1.
+struct Level {
+    uint8_t* minDelta;  // smallest delta + 1 of the item's boundaries
+    BoxRec* box;        // its union
+    BoxRec* before;     // all but the top level: union of its group up to it,
+    BoxRec* after;      //   from it on,
+    BoxRec* span;       //   and of the kSpan items from it on (to the group's end at most)
+    uint32_t count;
+};
+constexpr int kSpan = 8;
+struct HierLists {
+    uint32_t* count;    // [blocks]
+    uint32_t* entries;  // [blocks][kOpenCap]: position in the block | (delta + 1) << 16
+    uint8_t* deltas;    // [blocks][kOpenCap]: delta + 1
+    float* unions;      // [blocks][kOpenCap][12]: leaves up to the split, leaves after it
+    Level level[kMaxLevels];
+    int levels;
+};
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup g runs on
 // XCD g % 8). This numbering gives each XCD one contiguous range of blocks,
@@ -719,16 +649,15 @@ __device__ __forceinline__ uint32_t xcdContiguous(uint32_t g, uint32_t G) {
 // segOff[s] - s + local, children and leaf object indices are scene-local.
 // A range [l, r] is a scene's root exactly when delta(l-1) and delta(r) are
 // both -1.
-template <bool SOUP, typename KeyT, bool SEG = false>
+template <bool SOUP, typename KeyT, int B, bool SEG = false>
 __global__ __launch_bounds__(kHierThreads) void k_hier_local(
     PrimSrc src, const KeyT* __restrict__ skeys, const uint32_t* __restrict__ sidx, uint32_t n,
-    int keyBits, uint32_t* __restrict__ otherEnd, uint64_t* __restrict__ xchg, const uint32_t* __restrict__ epochWord,
-    clr_lbvh_inode* __restrict__ inodes, clr_lbvh_leaf* __restrict__ leaves,
-    Pending* __restrict__ pend, uint32_t* __restrict__ devStatus, SegView sv = SegView{nullptr, nullptr, nullptr}) {
+    int keyBits, clr_lbvh_inode* __restrict__ inodes, clr_lbvh_leaf* __restrict__ leaves, HierLists lists,
+    uint32_t* __restrict__ devStatus, SegView sv = SegView{nullptr, nullptr, nullptr}) {
     if constexpr (SEG)
         if (*sv.valid == 0u) return;
-    const uint32_t epoch = *epochWord;
-    constexpr int B = kLocalLeaves;
+    constexpr int kHierPer = B / kHierThreads;
+    static_assert(B % kHierThreads == 0 && B <= kLocalLeaves, "hierarchy block shape");
     __shared__ uint32_t s_other[B];
     __shared__ float s_box[6][B];
     // Deltas fit in 8 bits (at most keyBits + 31 <= 95) and completed-node
@@ -803,7 +732,6 @@ __global__ __launch_bounds__(kHierThreads) void k_hier_local(
         for (int k = 0; k < kHierPer; ++k) s_delta[(uint32_t)k * kHierThreads + t] = dv[k];
         if (t == 0) s_delta[B] = dv[kHierPer];
     }
-    if (t < 2) pend[2 * blk + t].valid = 0u;
     if (t < 3) s_qc[t] = 0u;
     __syncthreads();
     // Leaf records [bs, be) as consecutive 16-B parts (whole lines per store).
@@ -847,15 +775,7 @@ __global__ __launch_bounds__(kHierThreads) void k_hier_local(
                 const bool isLeft = dr > dl;
                 const uint32_t ps = isLeft ? R : L - 1u;  // the parent's split
                 const uint32_t self = isLeft ? r : l;     // this node's box slot
-                if (ps < bs || ps + 1u >= be) {
-                    // Split on a block boundary: hand the climb to phase 2.
-                    Pending& P = pend[2 * blk + (isLeft ? 1 : 0)];
-                    P.l = L; P.r = R; P.split = 0u; P.internal = l != r ? 1u : 0u;
-                    P.dl = dl; P.dr = dr;
-#pragma unroll
-                    for (int k = 0; k < 6; ++k) P.box[k] = s_box[k][self];
-                    P.valid = 1u;
-                } else {
+                if (ps >= bs && ps + 1u < be) {  // else the split is on a block boundary: phase 2
                     const uint32_t other =
                         __hip_atomic_exchange(&s_other[ps - bs], isLeft ? L : R, __ATOMIC_ACQ_REL,
                                               __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -907,30 +827,100 @@ __global__ __launch_bounds__(kHierThreads) void k_hier_local(
         __syncthreads();
         cnt = *qcount;
     }
-    // The loop ends with a barrier. Export the arrival words of phase 2: the
-    // slots where exactly one child arrived (phase 2 brings the other) hold
-    // that child's far end, the slots where neither did are empty, and so is
-    // the split between this block and the next. Completed slots are never
-    // reached again.
-    if (t == 0 && be < n) otherEnd[be - 1] = kEmpty;
+    // The loop ends with a barrier. The block's list of open splits, in order
+    // (s_q is free now): the slots that were not completed, and be - 1. In a
+    // segmented build only the first and the last scene boundary count.
+    if constexpr (SEG) {
+        __syncthreads();  // every thread has read the last count
+        if (t == 0) {
+            s_qc[0] = (uint32_t)B;
+            s_qc[1] = 0u;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kHierPer; ++k) {
+            const uint32_t j = (uint32_t)k * kHierThreads + t;
+            if (j < nl && s_delta[j + 1] == -1) {
+                atomicMin(&s_qc[0], j);
+                atomicMax(&s_qc[1], j);
+            }
+        }
+        __syncthreads();
+    }
+    bool open[kHierPer];
+    uint64_t openMask[kHierPer];
+    const uint32_t wave = t >> 6;
+    uint32_t* s_cnt = s_q[1];  // [kHierPer][waves], then the list's subtree slots
 #pragma unroll
     for (int k = 0; k < kHierPer; ++k) {
         const uint32_t j = (uint32_t)k * kHierThreads + t;
-        if (bs + j + 1 < be) {
-            const uint32_t v = s_other[j];
-            if (v != kDone) otherEnd[bs + j] = v;
-            if (v != kEmpty && v != kDone) {
-                const uint32_t ps = bs + j;
-                const bool leftArrived = v <= ps;
-                const uint32_t idx = leftArrived ? ps : ps + 1u;
-                const bool isLeaf = leftArrived ? (v == ps) : (v == ps + 1u);
-                if (!isLeaf) {
-                    const uint64_t tag = (uint64_t)epoch << 32;
-                    uint64_t* slot = xchg + 6 * (size_t)idx;
+        open[k] = j + 1 == nl;
+        if (j + 1 < nl && s_other[j] != kDone) open[k] = !SEG || s_delta[j + 1] != -1 || j == s_qc[0] || j == s_qc[1];
+        openMask[k] = __ballot(open[k]);
+        if (lane == 0) s_cnt[k * (kHierThreads / 64) + wave] = (uint32_t)__popcll(openMask[k]);
+    }
+    __syncthreads();
+    uint32_t m = 0;
+    {
+        uint32_t before[kHierPer];
 #pragma unroll
-                    for (int c = 0; c < 6; ++c) slot[c] = tag | __float_as_uint(s_box[c][idx - bs]);
-                }
+        for (int k = 0; k < kHierPer; ++k)
+            for (uint32_t w = 0; w < kHierThreads / 64; ++w) {
+                if (w == wave) before[k] = m;
+                m += s_cnt[k * (kHierThreads / 64) + w];
             }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kHierPer; ++k) {
+            const uint32_t at = before[k] + (uint32_t)__popcll(openMask[k] & ltMask);
+            if (open[k] && at < kOpenCap) s_q[0][at] = (uint32_t)k * kHierThreads + t;
+        }
+        if (m > kOpenCap) {  // not with sorted keys
+            m = kOpenCap;
+            if (t == 0) atomicOr(devStatus, kStatusHierarchy);
+        }
+    }
+    __syncthreads();
+    // Slot of the subtree that ends at each entry, then the unions up to (wave
+    // 0) and after each entry (wave 1), a thread per box component.
+    for (uint32_t k = t; k < m; k += kHierThreads) {
+        const uint32_t a = k ? s_q[0][k - 1] + 1u : 0u, e = s_q[0][k];
+        const uint32_t d = (uint32_t)(s_delta[e + 1] + 1);
+        s_cnt[k] = s_delta[e + 1] > s_delta[a] ? e : a;
+        lists.entries[(size_t)blk * kOpenCap + k] = e | d << 16;
+        lists.deltas[(size_t)blk * kOpenCap + k] = (uint8_t)d;
+    }
+    __syncthreads();
+    if (t < 6) {
+        float* out = lists.unions + (size_t)blk * kOpenCap * 12 + t;
+        float v = s_box[t][s_cnt[0]];
+        out[0] = v;
+#pragma unroll 4
+        for (uint32_t k = 1; k < m; ++k) {
+            const float x = s_box[t][s_cnt[k]];
+            v = t < 3 ? omin(v, x) : omax(v, x);
+            out[12 * k] = v;
+        }
+        reinterpret_cast<float*>(lists.level[0].box + blk)[t] = v;  // BoxRec is lo.xyz, hi.xyz in order
+    } else if (t >= 64 && t < 70 && m > 1) {
+        const uint32_t c = t - 64u;
+        float* out = lists.unions + (size_t)blk * kOpenCap * 12 + 6u + c;
+        float v = s_box[c][s_cnt[m - 1]];
+        out[12 * (m - 2)] = v;
+#pragma unroll 4
+        for (uint32_t k = m - 2; k > 0; --k) {
+            const float x = s_box[c][s_cnt[k]];
+            v = c < 3 ? omin(x, v) : omax(x, v);
+            out[12 * (k - 1)] = v;
+        }
+    } else if (wave == 2) {
+        int d = 127;
+        for (uint32_t k = (uint32_t)lane; k < m; k += 64u) d = min(d, (int)s_delta[s_q[0][k] + 1]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) d = min(d, __shfl_xor(d, off));
+        if (lane == 0) {
+            lists.level[0].minDelta[blk] = (uint8_t)(d + 1);
+            lists.count[blk] = m;
         }
     }
     // Records of the nodes completed here, as consecutive 16-B parts. A node
@@ -958,81 +948,236 @@ __global__ __launch_bounds__(kHierThreads) void k_hier_local(
     }
 }
 
-template <typename KeyT, bool SEG = false>
-__global__ __launch_bounds__(kBlock) void k_hier_global(
-    const KeyT* __restrict__ skeys, uint32_t n, int keyBits, uint32_t* __restrict__ otherEnd,
-    uint64_t* __restrict__ xchg, const uint32_t* __restrict__ epochWord, uint32_t* __restrict__ devStatus,
-    clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves,
-    const Pending* __restrict__ pend, uint32_t numPending, SegView sv = SegView{nullptr, nullptr, nullptr}) {
-    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= numPending) return;
-    if constexpr (SEG)
-        if (*sv.valid == 0u) return;
-    const uint32_t epoch = *epochWord;
-    const Pending P = pend[p];
-    if (!P.valid) return;
-    uint32_t l = P.l, r = P.r, split = P.split;
-    bool internal = P.internal != 0u;
-    int dl = P.dl, dr = P.dr;
-    Box box;
+__device__ __forceinline__ Box boxOfRec(const BoxRec& r) {
+    Box o;
+    o.lo[0] = r.a.x; o.lo[1] = r.a.y; o.lo[2] = r.a.z;
+    o.hi[0] = r.a.w; o.hi[1] = r.b.x; o.hi[2] = r.b.y;
+    return o;
+}
+__device__ __forceinline__ void storeRec(BoxRec* p, const Box& b) {
+    p->a = make_float4(b.lo[0], b.lo[1], b.lo[2], b.hi[0]);
+    p->b = make_float4(b.hi[1], b.hi[2], 0.0f, 0.0f);
+}
+// l united with r, l's leaves before r's.
+__device__ __forceinline__ Box unite(const Box& l, const Box& r) {
+    Box o;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        box.lo[k] = P.box[k];
-        box.hi[k] = P.box[3 + k];
+        o.lo[k] = omin(l.lo[k], r.lo[k]);
+        o.hi[k] = omax(l.hi[k], r.hi[k]);
     }
-    uint32_t seg = 0, segS = 0, segE = n;
-    if constexpr (SEG) {
-        seg = sv.segOf[l];
-        segS = sv.segOff[seg];
-        segE = sv.segOff[seg + 1];
-    }
-    bool written = true;  // phase 1 already wrote this node's record
-    while (true) {
-        if (l == segS && r == segE - 1) {
-            if (internal) writeNode(inodes, segS - seg, box, split, l, r, segS);
-            return;
-        }
-        const bool isLeft = dr > dl;
-        const uint32_t parentSplit = isLeft ? r : l - 1;
-        if (internal) {
-            const uint32_t self = isLeft ? r : l;
-            if (!written) writeNode(inodes, self - seg, box, split, l, r, segS);
-            publishBox(xchg + 6 * (size_t)self, box, epoch);
-        }
-        written = false;
-        // Keep the publish ahead of the arrival in program order: a sibling in
-        // the same wave may be the one that waits for it.
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        const uint32_t other = __hip_atomic_exchange(otherEnd + parentSplit, isLeft ? l : r,
-                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (other == kEmpty) return;  // first arrival: the sibling finishes the parent
-        const uint32_t s = isLeft ? parentSplit + 1u : parentSplit;
-        int dNew;
-        if (isLeft)
-            dNew = deltaAt<KeyT, SEG>(skeys, (int64_t)other, n, keyBits, sv);
-        else
-            dNew = deltaAt<KeyT, SEG>(skeys, (int64_t)other - 1, n, keyBits, sv);
-        const Box sb = (s == other) ? leafBox(leaves, s)
-                                    : awaitBox(xchg + 6 * (size_t)s, epoch, devStatus);
-        if (isLeft) {
+    return o;
+}
+__device__ __forceinline__ Box shuffled(const Box& b, int from) {
+    Box o;
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                box.lo[k] = omin(box.lo[k], sb.lo[k]);
-                box.hi[k] = omax(box.hi[k], sb.hi[k]);
+    for (int k = 0; k < 3; ++k) {
+        o.lo[k] = __shfl(b.lo[k], from);
+        o.hi[k] = __shfl(b.hi[k], from);
+    }
+    return o;
+}
+
+// One level of groups: a wave per group of 64 items of `in`, their running
+// unions from both ends, and the group's item of the next level.
+__global__ __launch_bounds__(kBlock) void k_hier_levels(Level in, Level out, const uint32_t* __restrict__ valid) {
+    if (valid && *valid == 0u) return;
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x, first = i & ~63u;
+    if (first >= in.count) return;  // the whole wave
+    const int lane = (int)(threadIdx.x & 63u), last = (int)min(in.count - first, 64u) - 1;
+    const uint32_t at = min(i, in.count - 1u);
+    const Box b = boxOfRec(in.box[at]);
+    int d = in.minDelta[at];
+    Box up = b, down = b, span = b;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const Box l = shuffled(up, lane - off), r = shuffled(down, lane + off);
+        if (lane >= off) up = unite(l, up);
+        if (lane + off <= last) down = unite(down, r);
+        d = min(d, __shfl_xor(d, off));
+        if (off < kSpan) {
+            const Box next = shuffled(span, lane + off);
+            if (lane + off <= last) span = unite(span, next);
+        }
+    }
+    if (lane <= last) {
+        storeRec(in.span + i, span);
+        storeRec(in.before + i, up);
+        storeRec(in.after + i, down);
+    }
+    if (lane == last) {
+        storeRec(out.box + (i >> 6), up);
+        out.minDelta[i >> 6] = (uint8_t)d;
+    }
+}
+
+// Position of the first (FIRST) or last item in [lo, hi] with a value (below 128)
+// under d, or -1; 64 values are loaded at once. `v` holds whole 64-byte groups.
+template <bool FIRST>
+__device__ __forceinline__ int64_t findBelow(const uint8_t* v, int64_t lo, int64_t hi, uint32_t d) {
+    const int64_t stop = FIRST ? hi >> 6 : lo >> 6;
+    for (int64_t c = FIRST ? lo >> 6 : hi >> 6; FIRST ? c <= stop : c >= stop; c += FIRST ? 1 : -1) {
+        uint4 w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = reinterpret_cast<const uint4*>(v)[4 * c + q];
+        uint64_t below = 0;  // a bit per value
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t ws[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                // Bit 7 of each byte: value < d. The product gathers the four bits.
+                const uint32_t m = ~((ws[k] | 0x80808080u) - d * 0x01010101u) & 0x80808080u;
+                below |= (uint64_t)(((m >> 7) * 0x10204080u) >> 28) << (16 * q + 4 * k);
             }
-            r = other;
-            dr = dNew;
+        }
+        if (lo > 64 * c) below &= ~0ull << (lo - 64 * c);
+        if (hi < 64 * c + 63) below &= ~0ull >> (63 - (hi - 64 * c));
+        if (below) return 64 * c + (FIRST ? __builtin_ctzll(below) : 63 - __builtin_clzll(below));
+    }
+    return -1;
+}
+// The nearest block from `b` on (FIRST: rightwards, else leftwards) whose smallest
+// delta + 1 is below d, or -1.
+template <bool FIRST>
+__device__ __forceinline__ int64_t findBlock(const HierLists& H, int64_t b, uint32_t d) {
+    int k = 0;
+    int64_t i = b;
+    while (true) {  // up: the rest of the group, then the group's neighbours
+        const int64_t count = H.level[k].count;
+        if (i < 0 || i >= count) return -1;
+        const int64_t g = i >> 6;
+        const int64_t f = FIRST ? findBelow<true>(H.level[k].minDelta, i, min(count, 64 * (g + 1)) - 1, d)
+                                : findBelow<false>(H.level[k].minDelta, 64 * g, i, d);
+        if (f >= 0) {
+            i = f;
+            break;
+        }
+        if (k + 1 >= H.levels) return -1;
+        ++k;
+        i = FIRST ? g + 1 : g - 1;
+    }
+    while (k > 0) {  // down: the end of the group that was found
+        --k;
+        const int64_t hi = min((int64_t)H.level[k].count, 64 * (i + 1)) - 1;
+        i = FIRST ? findBelow<true>(H.level[k].minDelta, 64 * i, hi, d)
+                  : findBelow<false>(H.level[k].minDelta, 64 * i, hi, d);
+    }
+    return i;
+}
+// acc united with blocks [i, j]. Four boxes are loaded at once; those of a span
+// or a group may overlap or repeat, which changes no union.
+__device__ __forceinline__ Box uniteBlocks(const HierLists& H, Box acc, int64_t i, int64_t j) {
+    Box right{};
+    bool hasRight = false;
+    for (int k = 0; i <= j; ++k) {
+        const Level& L = H.level[k];
+        if ((i >> 6) == (j >> 6)) {
+            const bool spans = k + 1 < H.levels && j - i >= kSpan - 1;
+            const BoxRec* from = spans ? L.span : L.box;
+            const int64_t step = spans ? kSpan : 1, end = spans ? j - (kSpan - 1) : j;
+            for (int64_t c = i; c < end + step; c += 4 * step) {
+                BoxRec r[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) r[q] = from[min(c + q * step, end)];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc = unite(acc, boxOfRec(r[q]));
+            }
+            break;
+        }
+        acc = unite(acc, boxOfRec(L.after[i]));
+        const Box r = boxOfRec(L.before[j]);
+        right = hasRight ? unite(r, right) : r;
+        hasRight = true;
+        i = (i >> 6) + 1;
+        j = (j >> 6) - 1;
+    }
+    return hasRight ? unite(acc, right) : acc;
+}
+
+// The nodes that cross blocks: 32 lanes per block, one per entry of its list
+// (about 25 entries at 1024 leaves).
+constexpr uint32_t kGlobalLanes = 32;
+template <int B, bool SEG = false>
+__global__ __launch_bounds__(kBlock) void k_hier_global(HierLists H, uint32_t n, clr_lbvh_inode* __restrict__ inodes,
+                                                        SegView sv = SegView{nullptr, nullptr, nullptr}) {
+    if constexpr (SEG)
+        if (*sv.valid == 0u) return;
+    const uint32_t blk =
+        xcdContiguous(blockIdx.x, gridDim.x) * (kBlock / kGlobalLanes) + threadIdx.x / kGlobalLanes;
+    if (blk >= H.level[0].count) return;
+    const uint32_t m = H.count[blk];
+    const uint32_t* list = H.entries + (size_t)blk * kOpenCap;
+    for (uint32_t k = threadIdx.x % kGlobalLanes; k < m; k += kGlobalLanes) {
+        const uint32_t own = list[k], prev = list[k ? k - 1u : 0u], next = list[min(k + 1u, m - 1u)];
+        const uint32_t d = own >> 16;  // delta + 1
+        if (d == 0u) continue;         // a scene boundary, or the end
+        const uint32_t x = blk * (uint32_t)B + (own & 0xFFFFu);
+        // Along the list deltas fall to the smallest and rise after it, so the
+        // nearest smaller one inside the block is a neighbour, if any.
+        const int left = k && (prev >> 16) < d ? (int)k - 1 : -1;
+        const int right = k + 1u < m && (next >> 16) < d ? (int)k + 1 : -1;
+        auto part = [&](uint32_t b, uint32_t entry, bool after) {
+            const float* u = H.unions + ((size_t)b * kOpenCap + entry) * 12 + (after ? 6 : 0);
+            return Box{{u[0], u[1], u[2]}, {u[3], u[4], u[5]}};
+        };
+        // Left end: the first leaf l, delta(l - 1) + 1, the first block whose
+        // leaves are united whole and, before it, the part of another.
+        uint32_t l = 0, dl = 0;
+        int64_t whole = 0;
+        bool hasPart = false;
+        Box acc{};
+        auto leftEntry = [&](uint32_t b, uint32_t entry) {
+            const uint32_t e = H.entries[(size_t)b * kOpenCap + entry];
+            l = b * (uint32_t)B + (e & 0xFFFFu) + 1u;
+            dl = e >> 16;
+            whole = (int64_t)b + 1;
+            if ((e & 0xFFFFu) + 1u < (uint32_t)B && l < n) {
+                acc = part(b, entry, true);
+                hasPart = true;
+            }
+        };
+        if (left >= 0) {
+            leftEntry(blk, (uint32_t)left);
         } else {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                box.lo[k] = omin(sb.lo[k], box.lo[k]);
-                box.hi[k] = omax(sb.hi[k], box.hi[k]);
+            const int64_t c = findBlock<false>(H, (int64_t)blk - 1, d);
+            if (c >= 0) {
+                const int64_t j = findBelow<false>(H.deltas + (size_t)c * kOpenCap, 0, (int64_t)H.count[c] - 1, d);
+                if (j < 0) continue;  // not with consistent lists, here and below
+                leftEntry((uint32_t)c, (uint32_t)j);
             }
-            l = other;
-            dl = dNew;
         }
-        split = parentSplit;
-        internal = true;
+        // Right end: the last leaf r, delta(r) + 1, its block and entry.
+        int64_t rb = blk;
+        uint32_t re = 0;
+        if (right >= 0) {
+            re = (uint32_t)right;
+        } else {
+            rb = findBlock<true>(H, (int64_t)blk + 1, d);
+            if (rb < 0) continue;
+            const int64_t j = findBelow<true>(H.deltas + (size_t)rb * kOpenCap, 0, (int64_t)H.count[rb] - 1, d);
+            if (j < 0) continue;
+            re = (uint32_t)j;
+        }
+        const uint32_t er = H.entries[(size_t)rb * kOpenCap + re];
+        const uint32_t r = (uint32_t)rb * (uint32_t)B + (er & 0xFFFFu), dr = er >> 16;
+        // [whole, rb - 1] and the part of rb up to r.
+        if (!hasPart && whole < rb) {
+            acc = boxOfRec(H.level[0].box[whole]);
+            hasPart = true;
+            ++whole;
+        }
+        if (whole <= rb) {
+            const Box last = part((uint32_t)rb, re, false);
+            acc = hasPart ? unite(uniteBlocks(H, acc, whole, rb - 1), last) : last;
+        }
+        uint32_t seg = 0, segS = 0;
+        if constexpr (SEG) {
+            seg = sv.segOf[x];
+            segS = sv.segOff[seg];
+        }
+        const uint32_t idx = dl == 0u && dr == 0u ? segS : (dr > dl ? r : l);
+        writeNode(inodes, idx - seg, acc, x, l, r, segS);
     }
 }
 
@@ -1047,8 +1192,7 @@ struct Layout {
     void* keysB;
     uint32_t* valsA;
     uint32_t* valsB;
-    uint32_t* otherEnd;
-    Pending* pend;
+    HierLists lists;
     size_t bytes;
 };
 
@@ -1072,8 +1216,24 @@ Layout layoutFor(Carve& c, uint32_t n, size_t keyBytes, int P, uint32_t tile) {
     L.keysB = c.take<char>(keyBytes * n);
     L.valsA = c.take<uint32_t>(n);
     L.valsB = c.take<uint32_t>(n);
-    L.otherEnd = c.take<uint32_t>(n);
-    L.pend = c.take<Pending>(2 * (size_t)((n + kLocalLeaves - 1) / kLocalLeaves));
+    const uint32_t leavesPerBlock = localLeavesFor(n);
+    uint32_t count = (n + leavesPerBlock - 1) / leavesPerBlock;
+    HierLists& H = L.lists;
+    H.count = c.take<uint32_t>(count);
+    H.entries = c.take<uint32_t>((size_t)count * kOpenCap);
+    H.deltas = c.take<uint8_t>((size_t)count * kOpenCap);
+    H.unions = c.take<float>((size_t)count * kOpenCap * 12);
+    for (H.levels = 0; H.levels < kMaxLevels;) {
+        Level& v = H.level[H.levels++];
+        v.count = count;
+        v.minDelta = c.take<uint8_t>((count + 63) & ~63u);
+        v.box = c.take<BoxRec>(count);
+        if (count <= 64) break;
+        v.before = c.take<BoxRec>(count);
+        v.after = c.take<BoxRec>(count);
+        v.span = c.take<BoxRec>(count);
+        count = (count + 63) / 64;
+    }
     L.bytes = c.off + 256;
     return L;
 }
@@ -1087,22 +1247,35 @@ inline unsigned gridFor(uint32_t n, unsigned cap) {
     return g < 1 ? 1 : (g > cap ? cap : g);
 }
 
-// Working memory of one build: the layout region, the hierarchy's exchange
-// words (six per internal node) and the epoch word that tags them. The
-// context's pool and exchange buffer, or the no-allocation entry point's
-// static array.
-struct BuildScratch {
-    void* base;
-    uint64_t* xchg;
-    size_t xchgNodes;
-    uint32_t* epochWord;
-};
+// The hierarchy's launches on sorted keys and payloads.
+template <bool SOUP, typename KeyT, bool SEG>
+void launchHierarchy(clr_ctx* ctx, const Layout& L, const PrimSrc& src, const KeyT* keys, const uint32_t* vals,
+                     uint32_t n, int keyBits, clr_lbvh_inode* inodes, clr_lbvh_leaf* leaves, const SegView& sv,
+                     hipStream_t stream, hipEvent_t afterLocal) {
+    const HierLists& H = L.lists;
+    const uint32_t blocks = H.level[0].count;
+    const bool small = localLeavesFor(n) == (uint32_t)kSmallLeaves;
+    if (small)
+        k_hier_local<SOUP, KeyT, kSmallLeaves, SEG><<<blocks, kHierThreads, 0, stream>>>(
+            src, keys, vals, n, keyBits, inodes, leaves, H, ctx->devStatus, sv);
+    else
+        k_hier_local<SOUP, KeyT, kLocalLeaves, SEG><<<blocks, kHierThreads, 0, stream>>>(
+            src, keys, vals, n, keyBits, inodes, leaves, H, ctx->devStatus, sv);
+    if (afterLocal) (void)hipEventRecord(afterLocal, stream);
+    if (blocks < 2) return;  // one block completes every node
+    for (int k = 0; k + 1 < H.levels; ++k)
+        k_hier_levels<<<(H.level[k].count + kBlock - 1) / kBlock, kBlock, 0, stream>>>(H.level[k], H.level[k + 1],
+                                                                                       sv.valid);
+    constexpr uint32_t perGroup = kBlock / kGlobalLanes;
+    const uint32_t grid = (blocks + perGroup - 1) / perGroup;
+    if (small) k_hier_global<kSmallLeaves, SEG><<<grid, kBlock, 0, stream>>>(H, n, inodes, sv);
+    else k_hier_global<kLocalLeaves, SEG><<<grid, kBlock, 0, stream>>>(H, n, inodes, sv);
+}
 
 template <typename KeyT, bool SOUP>
 int runBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
-             clr_lbvh_inode* inodes, clr_lbvh_leaf* leaves, hipStream_t stream, const BuildScratch& W) {
-    uint32_t* epochWord = W.epochWord;
-    Layout L = layoutFor(W.base, n, bits);
+             clr_lbvh_inode* inodes, clr_lbvh_leaf* leaves, hipStream_t stream, void* base) {
+    Layout L = layoutFor(base, n, bits);
     const int P = numPassesFor(bits);
     const uint32_t tile = tileFor(bits);
     const uint32_t parts = (n + tile - 1) / tile;
@@ -1113,7 +1286,7 @@ int runBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
     };
     ev(0);
     k_init<<<gridFor((uint32_t)std::min<size_t>(L.clearWords, 0xFFFFFFFFu), 2048), kBlock, 0, stream>>>(
-        L.hist, L.clearWords, L.sceneOrd, epochWord, reinterpret_cast<uint32_t*>(W.xchg), W.xchgNodes * 12);
+        L.hist, L.clearWords, L.sceneOrd);
     // One set of same-address atomics per block: a few blocks per CU.
     const unsigned reduceGrid = (unsigned)std::max(1, ctx->numCUs) * 4u;
     // Box centres live in buffers the first radix pass has not written yet:
@@ -1123,7 +1296,7 @@ int runBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
     float* cy = reinterpret_cast<float*>(L.valsA);
     float* cz = reinterpret_cast<float*>(L.valsB);
     k_bounds<SOUP><<<gridFor(n, reduceGrid), kBlock, 0, stream>>>(in.tris, in.vertices, in.faces, n, L.boxes, cx,
-                                                                  cy, cz, L.sceneOrd, epochWord);
+                                                                  cy, cz, L.sceneOrd);
     ev(1);
     PrimSrc src{in.tris, L.boxes};
     k_morton<KeyT><<<gridFor(n, reduceGrid), kBlock, 0, stream>>>(
@@ -1147,13 +1320,9 @@ int runBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
         std::swap(vin, vout);
     }
     ev(3);
-    const uint32_t localBlocks = (n + kLocalLeaves - 1) / kLocalLeaves;
-    k_hier_local<SOUP, KeyT><<<localBlocks, kHierThreads, 0, stream>>>(
-        src, kin, vin, n, keyBits, L.otherEnd, W.xchg, epochWord, inodes, leaves, L.pend, ctx->devStatus);
-    ev(4);
-    k_hier_global<KeyT><<<(2 * localBlocks + kBlock - 1) / kBlock, kBlock, 0, stream>>>(
-        kin, n, keyBits, L.otherEnd, W.xchg, epochWord, ctx->devStatus, inodes, leaves, L.pend,
-        2 * localBlocks);
+    launchHierarchy<SOUP, KeyT, false>(ctx, L, src, kin, vin, n, keyBits, inodes, leaves,
+                                       SegView{nullptr, nullptr, nullptr}, stream,
+                                       prof ? ctx->events[ctx->profiledBuilds][4] : nullptr);
     ev(5);
     if (prof) ++ctx->profiledBuilds;
     return hipCheck(ctx, hipGetLastError(), "LBVH build launch");
@@ -1235,10 +1404,8 @@ __global__ __launch_bounds__(kSegScanThreads) void k_seg_chunks(const uint32_t* 
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_seg_init(uint32_t* segBox, uint32_t numSegments,
-                                                     uint32_t* epochWord) {
+__global__ __launch_bounds__(kBlock) void k_seg_init(uint32_t* segBox, uint32_t numSegments) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i == 0) advanceEpoch(epochWord);
     if (i < 6 * numSegments) segBox[i] = (i % 6) < 3 ? ordOf(INFINITY) : ordOf(-INFINITY);
 }
 
@@ -1359,8 +1526,10 @@ SegLayout segLayoutFor(void* base, uint32_t n, uint32_t numSegments, int P) {
 }  // namespace
 
 size_t lbvhSegScratchBytes(uint32_t totalTris, uint32_t numSegments, uint32_t bitsPerDim) {
+    // As lbvhScratchBytes: enough for every smaller build too.
     const int P = (segKeyBits(bitsPerDim, numSegments) + 7) / 8;
-    return segLayoutFor(nullptr, totalTris, numSegments, P).bytes;
+    return std::max(segLayoutFor(nullptr, totalTris, numSegments, P).bytes,
+                    segLayoutFor(nullptr, std::min(totalTris, kSmallBuild), numSegments, P).bytes);
 }
 
 int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffsets, uint32_t numSegments,
@@ -1373,17 +1542,14 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
     if (rc) return rc;
     rc = ensureStatus(ctx);
     if (rc) return rc;
-    rc = ensureExchange(ctx, n);
-    if (rc) return rc;
-    uint32_t* epochWord = ctx->devStatus + kWordEpoch;
     SegLayout S = segLayoutFor(ctx->pool, n, numSegments, P);
     Layout& L = S.L;
     const uint32_t maxChunks = segChunkBound(n, numSegments);
     const uint32_t tile = (uint32_t)(kSortBlock * SortCfg<uint64_t>::kItems);
     const uint32_t parts = (n + tile - 1) / tile;
     k_init<<<gridFor((uint32_t)std::min<size_t>(L.clearWords, 0xFFFFFFFFu), 2048), kBlock, 0, stream>>>(
-        L.hist, L.clearWords, nullptr, epochWord, reinterpret_cast<uint32_t*>(ctx->xchg), ctx->xchgNodes * 12);
-    k_seg_init<<<(6 * numSegments + kBlock - 1) / kBlock, kBlock, 0, stream>>>(S.segBox, numSegments, epochWord);
+        L.hist, L.clearWords, nullptr);
+    k_seg_init<<<(6 * numSegments + kBlock - 1) / kBlock, kBlock, 0, stream>>>(S.segBox, numSegments);
     k_seg_chunks<<<1, kSegScanThreads, 0, stream>>>(segOffsets, numSegments, n, S.chunks, S.words, ctx->devStatus);
     k_seg_bounds<<<maxChunks, kBlock, 0, stream>>>(tris, S.chunks, S.words, S.segBox);
     k_seg_morton<<<maxChunks, kBlock, 0, stream>>>(tris, L.boxes, n, bits, S.chunks, S.words, S.segBox,
@@ -1407,12 +1573,7 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
     }
     const SegView sv{S.segOf, segOffsets, S.words + kSegWordValid};
     PrimSrc src{tris, L.boxes};
-    const uint32_t localBlocks = (n + kLocalLeaves - 1) / kLocalLeaves;
-    k_hier_local<true, uint64_t, true><<<localBlocks, kHierThreads, 0, stream>>>(
-        src, kin, vin, n, keyBits, L.otherEnd, ctx->xchg, epochWord, inodes, leaves, L.pend, ctx->devStatus, sv);
-    k_hier_global<uint64_t, true><<<(2 * localBlocks + kBlock - 1) / kBlock, kBlock, 0, stream>>>(
-        kin, n, keyBits, L.otherEnd, ctx->xchg, epochWord, ctx->devStatus, inodes, leaves, L.pend, 2 * localBlocks,
-        sv);
+    launchHierarchy<true, uint64_t, true>(ctx, L, src, kin, vin, n, keyBits, inodes, leaves, sv, stream, nullptr);
     return hipCheck(ctx, hipGetLastError(), "segmented LBVH build launch");
 }
 
@@ -1422,38 +1583,34 @@ void fillZero(uint32_t* words, size_t count, hipStream_t stream) {
 }
 
 size_t lbvhScratchBytes(uint32_t n, uint32_t bitsPerDim) {
-    return layoutFor(nullptr, n, bitsPerDim).bytes;
+    // Enough for every smaller build too, so that memory reserved for n serves
+    // them: a build of kSmallBuild triangles has more blocks than one just above.
+    return std::max(layoutFor(nullptr, n, bitsPerDim).bytes,
+                    layoutFor(nullptr, std::min(n, kSmallBuild), bitsPerDim).bytes);
 }
 
 int lbvhBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
               clr_lbvh_inode* inodes, clr_lbvh_leaf* leaves, hipStream_t stream) {
     int rc = ensurePool(ctx, lbvhScratchBytes(n, bits));
     if (!rc) rc = ensureStatus(ctx);
-    if (!rc) rc = ensureExchange(ctx, n);
     if (rc) return rc;
-    const BuildScratch W{ctx->pool, ctx->xchg, ctx->xchgNodes, ctx->devStatus + kWordEpoch};
     const bool soup = in.tris != nullptr;
     if (bits <= 10)
-        return soup ? runBuild<uint32_t, true>(ctx, in, n, bits, inodes, leaves, stream, W)
-                    : runBuild<uint32_t, false>(ctx, in, n, bits, inodes, leaves, stream, W);
-    return soup ? runBuild<uint64_t, true>(ctx, in, n, bits, inodes, leaves, stream, W)
-                : runBuild<uint64_t, false>(ctx, in, n, bits, inodes, leaves, stream, W);
+        return soup ? runBuild<uint32_t, true>(ctx, in, n, bits, inodes, leaves, stream, ctx->pool)
+                    : runBuild<uint32_t, false>(ctx, in, n, bits, inodes, leaves, stream, ctx->pool);
+    return soup ? runBuild<uint64_t, true>(ctx, in, n, bits, inodes, leaves, stream, ctx->pool)
+                : runBuild<uint64_t, false>(ctx, in, n, bits, inodes, leaves, stream, ctx->pool);
 }
 
 // ---- the build that allocates nothing ----------------------------------------
 // clr_lbvh_build_soup_noalloc's working memory: one static array per device
 // (each device that loads this code object holds its own copy until the
-// process ends), laid out as 256 B of control words (word 0: the build epoch
-// of this array's exchange words), the exchange words for kNoAllocMaxTris
-// triangles, then the build layout for kNoAllocMaxTris triangles with 30-bit
+// process ends) with the build layout for kNoAllocMaxTris triangles and 30-bit
 // keys. Host code never passes `scratch` itself to a kernel (its host-side
 // name is not a device address): lbvhNoAllocInit looks up its device address
 // once per device and every later use goes through that pointer.
 constexpr uint32_t kNoAllocMaxTris = 1u << 20;
-constexpr size_t kNoAllocCtrlBytes = 256;
-constexpr size_t kNoAllocXchgBytes = (size_t)kNoAllocMaxTris * 6 * sizeof(uint64_t);
-constexpr size_t kNoAllocLayoutBytes = (size_t)56 << 20;  // >= layoutFor(kNoAllocMaxTris, 10 bits), checked
-constexpr size_t kNoAllocScratchBytes = kNoAllocCtrlBytes + kNoAllocXchgBytes + kNoAllocLayoutBytes;
+constexpr size_t kNoAllocScratchBytes = (size_t)72 << 20;  // >= every layoutFor up to kNoAllocMaxTris, checked
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1463,18 +1620,13 @@ void* g_noAllocPtr[kMaxDevices] = {};
 int lbvhNoAllocInit(clr_ctx* ctx) {
     if (ctx->device < 0 || ctx->device >= kMaxDevices)
         return fail(ctx, CLR_ERR_UNSUPPORTED, "device ordinal beyond the no-allocation table");
-    if (layoutFor(nullptr, kNoAllocMaxTris, 10).bytes > kNoAllocLayoutBytes)
+    if (lbvhScratchBytes(kNoAllocMaxTris, 10) > kNoAllocScratchBytes)
         return fail(ctx, CLR_ERR_UNSUPPORTED, "no-allocation scratch smaller than its layout");
     std::lock_guard<std::mutex> lock(g_noAllocMutex);
     void*& slot = g_noAllocPtr[ctx->device];
     if (!slot) {
         void* ptr = nullptr;
         int rc = hipCheck(ctx, hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)), "no-allocation scratch address");
-        if (rc) return rc;
-        // Once per device: the epoch starts at 0 and no exchange word carries
-        // a later epoch.
-        fillZero(static_cast<uint32_t*>(ptr), (kNoAllocCtrlBytes + kNoAllocXchgBytes) / 4, nullptr);
-        rc = hipCheck(ctx, hipDeviceSynchronize(), "no-allocation scratch clear");
         if (rc) return rc;
         slot = ptr;
     }
@@ -1491,12 +1643,9 @@ int lbvhBuildSoupNoAlloc(clr_ctx* ctx, const float* tris, uint32_t n, uint32_t b
         return fail(ctx, CLR_ERR_UNSUPPORTED, "numTris " + std::to_string(n) + " exceeds the no-allocation limit of " +
                                                   std::to_string(kNoAllocMaxTris));
     if (bits > 10) return fail(ctx, CLR_ERR_UNSUPPORTED, "the no-allocation build supports numBitsPerDim 1..10");
-    char* base = static_cast<char*>(ctx->noAllocScratch);
-    const BuildScratch W{base + kNoAllocCtrlBytes + kNoAllocXchgBytes, reinterpret_cast<uint64_t*>(base + kNoAllocCtrlBytes),
-                         kNoAllocMaxTris, reinterpret_cast<uint32_t*>(base)};
     LbvhInput in;
     in.tris = tris;
-    return runBuild<uint32_t, true>(ctx, in, n, bits, inodes, leaves, stream, W);
+    return runBuild<uint32_t, true>(ctx, in, n, bits, inodes, leaves, stream, ctx->noAllocScratch);
 }
 
 }  // namespace clr

@@ -7,7 +7,7 @@
  * (a hipStream_t passed as void*; NULL = the default stream) and is
  * stream-ordered: no entry point synchronises the host unless its comment says
  * so. A clr_ctx is externally synchronised: one host thread at a time, and
- * its scratch (LBVH pool, exchange words, render and wavefront state) is shared
+ * its scratch (LBVH pool, render and wavefront state) is shared
  * by all its calls, so work enqueued through one context must stay on one
  * stream, or calls on different streams must be ordered by the caller (use
  * one context per concurrent stream).
@@ -146,7 +146,7 @@ int clr_lbvh_build_soup(clr_ctx* ctx, const float* tris, uint32_t numTris,
  * reference: it is for callers that cannot allocate device memory (code
  * under hipGraph stream capture, tight serving loops, harnesses that forbid
  * hipMalloc). Instead of the context's scratch pool it works in a static
- * device array of 104 MiB + 256 B that every device loading the library
+ * device array of 72 MiB that every device loading the library
  * holds until the process ends, sized for numTris <=
  * clr_lbvh_noalloc_max_tris() (1,048,576) and numBitsPerDim 1..10; larger
  * requests return CLR_ERR_UNSUPPORTED. The call enqueues kernels only: no
@@ -160,10 +160,10 @@ int clr_lbvh_build_soup_noalloc(clr_ctx* ctx, const float* tris, uint32_t numTri
 /* Largest numTris clr_lbvh_build_soup_noalloc accepts. */
 uint32_t clr_lbvh_noalloc_max_tris(void);
 
-/* Pre-grows the scratch pool and the hierarchy's exchange buffer for builds
- * of up to maxFaces triangles (mirrors the capacity argument of the
- * LBVHBuilder ctor). Synchronous. After it, builds of up to maxFaces
- * triangles allocate nothing and may be captured into a hipGraph. */
+/* Pre-grows the scratch pool for builds of up to maxFaces triangles (mirrors
+ * the capacity argument of the LBVHBuilder ctor). Synchronous. After it,
+ * builds of up to maxFaces triangles allocate nothing and may be captured into
+ * a hipGraph. */
 int clr_lbvh_reserve(clr_ctx* ctx, uint32_t maxFaces, uint32_t numBitsPerDim);
 
 /* Segmented build: numSegments independent scenes in one set of launches.
