@@ -51,6 +51,14 @@ constexpr uint32_t kFlagMask = 3u << 30;
 constexpr uint32_t kCountMask = (1u << 30) - 1;
 constexpr int kMaxPasses = 8;
 
+// Keys per thread of a radix pass. Large sorts want few tiles to look back over,
+// until keys and payloads in LDS leave too few waves: passes on 64-bit keys with
+// 6 / 8 / 10 / 12 / 16 keys per thread make a build of 3.1 M triangles in 678 / 658 /
+// 643 / 641 / 656 us, one of 64 scenes in 787 / 776 / 755 / 802 / 779. Small sorts are a
+// few tiles on an empty chip, where a tile's own latency counts: builds with 4
+// keys per thread / the large shape take (us) 80 / 101 (30-bit keys) and 116 / 136
+// (60-bit) at 35,000 triangles, 140 / 153 and 197 / 207 at 2^18, 166 / 172 and 242 /
+// 239 at 2^19, 221 / 207 and 324 / 299 at 2^20: the line lies at 2 MB of keys.
 template <typename KeyT>
 struct SortCfg;
 template <>
@@ -59,8 +67,10 @@ struct SortCfg<uint32_t> {
 };
 template <>
 struct SortCfg<uint64_t> {
-    static constexpr int kItems = 6;
+    static constexpr int kItems = 10;
 };
+constexpr int kSmallItems = 4;
+constexpr uint32_t smallSort(size_t keyBytes) { return (uint32_t)((1u << 21) / keyBytes); }  // up to this many keys
 
 // OpenCL fmin/fmax with a fixed answer for +-0 ties (left operand) and NaN
 // (the other operand); the oracle uses the same rule.
@@ -325,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void k_morton(const float* __restrict__ cx,
 // ------------------------------------------------------------ onesweep ----
 // One stable LSD pass on the 8-bit digit at `shift`. FIRST generates the
 // payload (original index) instead of reading it.
-template <typename KeyT, bool FIRST>
+template <typename KeyT, bool FIRST, int kItems>
 __global__ __launch_bounds__(kSortBlock) void k_onesweep(const KeyT* __restrict__ keysIn,
                                                          const uint32_t* __restrict__ valsIn,
                                                          KeyT* __restrict__ keysOut,
@@ -335,7 +345,6 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const KeyT* __restrict_
                                                          uint32_t* __restrict__ status,
                                                          uint32_t* __restrict__ partCounter,
                                                          uint32_t* __restrict__ devStatus) {
-    constexpr int kItems = SortCfg<KeyT>::kItems;
     constexpr int kTile = kSortBlock * kItems;
     __shared__ uint32_t s_part;
     __shared__ uint32_t s_waveHist[kWaves][256];
@@ -413,7 +422,7 @@ __global__ __launch_bounds__(kSortBlock) void k_onesweep(const KeyT* __restrict_
     // overlaps that work. Earlier partitions took their ids before this one,
     // so they are resident and will publish; the bound only guards against a
     // bug.
-    constexpr int kWin = 4;
+    constexpr int kWin = 4;  // 8 and 16 are slower at every size
     uint32_t exclusive = 0;
     uint32_t win[kWin];
     int64_t look = (int64_t)part - 1;
@@ -1197,13 +1206,16 @@ struct Layout {
 };
 
 inline int numPassesFor(uint32_t bits) { return (int)((3 * bits + 7) / 8); }
-inline uint32_t tileFor(uint32_t bits) {
-    return bits <= 10 ? (uint32_t)(kSortBlock * SortCfg<uint32_t>::kItems)
-                      : (uint32_t)(kSortBlock * SortCfg<uint64_t>::kItems);
+inline uint32_t tileFor(uint32_t n, size_t keyBytes) {
+    const int items = n <= smallSort(keyBytes) ? kSmallItems
+                      : keyBytes == 4          ? SortCfg<uint32_t>::kItems
+                                               : SortCfg<uint64_t>::kItems;
+    return (uint32_t)(kSortBlock * items);
 }
 
-Layout layoutFor(Carve& c, uint32_t n, size_t keyBytes, int P, uint32_t tile) {
+Layout layoutFor(Carve& c, uint32_t n, size_t keyBytes, int P) {
     Layout L{};
+    const uint32_t tile = tileFor(n, keyBytes);
     const uint32_t parts = (n + tile - 1) / tile;
     L.sceneOrd = c.take<uint32_t>(8);
     // hist, counters and status carved back to back so one fill clears them
@@ -1239,12 +1251,47 @@ Layout layoutFor(Carve& c, uint32_t n, size_t keyBytes, int P, uint32_t tile) {
 }
 Layout layoutFor(void* base, uint32_t n, uint32_t bits) {
     Carve c(base);
-    return layoutFor(c, n, bits <= 10 ? 4 : 8, numPassesFor(bits), tileFor(bits));
+    return layoutFor(c, n, bits <= 10 ? 4 : 8, numPassesFor(bits));
+}
+
+// Scratch for every build of up to n triangles, so that memory reserved for n
+// serves the smaller ones: a build at the end of a small shape's range has more
+// blocks or tiles than one just above.
+template <typename F>
+size_t bytesUpTo(uint32_t n, size_t keyBytes, F layoutBytes) {
+    return std::max({layoutBytes(n), layoutBytes(std::min(n, kSmallBuild)),
+                     layoutBytes(std::min(n, smallSort(keyBytes)))});
 }
 
 inline unsigned gridFor(uint32_t n, unsigned cap) {
     unsigned g = (unsigned)((n + kBlock - 1) / kBlock);
     return g < 1 ? 1 : (g > cap ? cap : g);
+}
+
+// The radix passes. On return keys and payloads are in kin and vin.
+template <typename KeyT, int ITEMS>
+void launchPasses(clr_ctx* ctx, const Layout& L, KeyT*& kin, uint32_t*& vin, uint32_t n, int P, hipStream_t stream) {
+    KeyT* kout = static_cast<KeyT*>(L.keysB);
+    uint32_t* vout = L.valsB;
+    const uint32_t tile = (uint32_t)(kSortBlock * ITEMS), parts = (n + tile - 1) / tile;
+    for (int p = 0; p < P; ++p) {
+        uint32_t* st = L.status + (size_t)p * parts * 256;
+        if (p == 0)
+            k_onesweep<KeyT, true, ITEMS><<<parts, kSortBlock, 0, stream>>>(
+                kin, vin, kout, vout, n, 8 * p, L.hist + 256 * p, st, L.partCounters + p, ctx->devStatus);
+        else
+            k_onesweep<KeyT, false, ITEMS><<<parts, kSortBlock, 0, stream>>>(
+                kin, vin, kout, vout, n, 8 * p, L.hist + 256 * p, st, L.partCounters + p, ctx->devStatus);
+        std::swap(kin, kout);
+        std::swap(vin, vout);
+    }
+}
+template <typename KeyT>
+void launchSort(clr_ctx* ctx, const Layout& L, KeyT*& kin, uint32_t*& vin, uint32_t n, int P, hipStream_t stream) {
+    kin = static_cast<KeyT*>(L.keysA);
+    vin = L.valsA;
+    if (n <= smallSort(sizeof(KeyT))) launchPasses<KeyT, kSmallItems>(ctx, L, kin, vin, n, P, stream);
+    else launchPasses<KeyT, SortCfg<KeyT>::kItems>(ctx, L, kin, vin, n, P, stream);
 }
 
 // The hierarchy's launches on sorted keys and payloads.
@@ -1277,8 +1324,6 @@ int runBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
              clr_lbvh_inode* inodes, clr_lbvh_leaf* leaves, hipStream_t stream, void* base) {
     Layout L = layoutFor(base, n, bits);
     const int P = numPassesFor(bits);
-    const uint32_t tile = tileFor(bits);
-    const uint32_t parts = (n + tile - 1) / tile;
     const int keyBits = (int)(3 * bits);
     const bool prof = ctx->profiling && ctx->profiledBuilds < clr_ctx::kMaxProfiledBuilds;
     auto ev = [&](int k) {
@@ -1302,23 +1347,9 @@ int runBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,
     k_morton<KeyT><<<gridFor(n, reduceGrid), kBlock, 0, stream>>>(
         cx, cy, cz, n, bits, L.sceneOrd, static_cast<KeyT*>(L.keysA), L.hist, P);
     ev(2);
-    KeyT* kin = static_cast<KeyT*>(L.keysA);
-    KeyT* kout = static_cast<KeyT*>(L.keysB);
-    uint32_t* vin = L.valsA;
-    uint32_t* vout = L.valsB;
-    for (int p = 0; p < P; ++p) {
-        uint32_t* st = L.status + (size_t)p * parts * 256;
-        if (p == 0)
-            k_onesweep<KeyT, true><<<parts, kSortBlock, 0, stream>>>(
-                kin, vin, kout, vout, n, 8 * p, L.hist + 256 * p, st, L.partCounters + p,
-                ctx->devStatus);
-        else
-            k_onesweep<KeyT, false><<<parts, kSortBlock, 0, stream>>>(
-                kin, vin, kout, vout, n, 8 * p, L.hist + 256 * p, st, L.partCounters + p,
-                ctx->devStatus);
-        std::swap(kin, kout);
-        std::swap(vin, vout);
-    }
+    KeyT* kin;
+    uint32_t* vin;
+    launchSort<KeyT>(ctx, L, kin, vin, n, P, stream);
     ev(3);
     launchHierarchy<SOUP, KeyT, false>(ctx, L, src, kin, vin, n, keyBits, inodes, leaves,
                                        SegView{nullptr, nullptr, nullptr}, stream,
@@ -1514,7 +1545,7 @@ int segKeyBits(uint32_t bits, uint32_t numSegments) {
 SegLayout segLayoutFor(void* base, uint32_t n, uint32_t numSegments, int P) {
     Carve c(base);
     SegLayout S;
-    S.L = layoutFor(c, n, 8, P, (uint32_t)(kSortBlock * SortCfg<uint64_t>::kItems));
+    S.L = layoutFor(c, n, 8, P);
     S.segOf = c.take<uint32_t>(n);
     S.words = c.take<uint32_t>(64);
     S.segBox = c.take<uint32_t>(6 * (size_t)numSegments);
@@ -1526,10 +1557,8 @@ SegLayout segLayoutFor(void* base, uint32_t n, uint32_t numSegments, int P) {
 }  // namespace
 
 size_t lbvhSegScratchBytes(uint32_t totalTris, uint32_t numSegments, uint32_t bitsPerDim) {
-    // As lbvhScratchBytes: enough for every smaller build too.
     const int P = (segKeyBits(bitsPerDim, numSegments) + 7) / 8;
-    return std::max(segLayoutFor(nullptr, totalTris, numSegments, P).bytes,
-                    segLayoutFor(nullptr, std::min(totalTris, kSmallBuild), numSegments, P).bytes);
+    return bytesUpTo(totalTris, 8, [&](uint32_t n) { return segLayoutFor(nullptr, n, numSegments, P).bytes; });
 }
 
 int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffsets, uint32_t numSegments,
@@ -1545,8 +1574,6 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
     SegLayout S = segLayoutFor(ctx->pool, n, numSegments, P);
     Layout& L = S.L;
     const uint32_t maxChunks = segChunkBound(n, numSegments);
-    const uint32_t tile = (uint32_t)(kSortBlock * SortCfg<uint64_t>::kItems);
-    const uint32_t parts = (n + tile - 1) / tile;
     k_init<<<gridFor((uint32_t)std::min<size_t>(L.clearWords, 0xFFFFFFFFu), 2048), kBlock, 0, stream>>>(
         L.hist, L.clearWords, nullptr);
     k_seg_init<<<(6 * numSegments + kBlock - 1) / kBlock, kBlock, 0, stream>>>(S.segBox, numSegments);
@@ -1554,23 +1581,9 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
     k_seg_bounds<<<maxChunks, kBlock, 0, stream>>>(tris, S.chunks, S.words, S.segBox);
     k_seg_morton<<<maxChunks, kBlock, 0, stream>>>(tris, L.boxes, n, bits, S.chunks, S.words, S.segBox,
                                                    static_cast<uint64_t*>(L.keysA), S.segOf, L.hist, P);
-    uint64_t* kin = static_cast<uint64_t*>(L.keysA);
-    uint64_t* kout = static_cast<uint64_t*>(L.keysB);
-    uint32_t* vin = L.valsA;
-    uint32_t* vout = L.valsB;
-    for (int p = 0; p < P; ++p) {
-        uint32_t* st = L.status + (size_t)p * parts * 256;
-        if (p == 0)
-            k_onesweep<uint64_t, true><<<parts, kSortBlock, 0, stream>>>(kin, vin, kout, vout, n, 8 * p,
-                                                                         L.hist + 256 * p, st, L.partCounters + p,
-                                                                         ctx->devStatus);
-        else
-            k_onesweep<uint64_t, false><<<parts, kSortBlock, 0, stream>>>(kin, vin, kout, vout, n, 8 * p,
-                                                                          L.hist + 256 * p, st, L.partCounters + p,
-                                                                          ctx->devStatus);
-        std::swap(kin, kout);
-        std::swap(vin, vout);
-    }
+    uint64_t* kin;
+    uint32_t* vin;
+    launchSort<uint64_t>(ctx, L, kin, vin, n, P, stream);
     const SegView sv{S.segOf, segOffsets, S.words + kSegWordValid};
     PrimSrc src{tris, L.boxes};
     launchHierarchy<true, uint64_t, true>(ctx, L, src, kin, vin, n, keyBits, inodes, leaves, sv, stream, nullptr);
@@ -1583,10 +1596,7 @@ void fillZero(uint32_t* words, size_t count, hipStream_t stream) {
 }
 
 size_t lbvhScratchBytes(uint32_t n, uint32_t bitsPerDim) {
-    // Enough for every smaller build too, so that memory reserved for n serves
-    // them: a build of kSmallBuild triangles has more blocks than one just above.
-    return std::max(layoutFor(nullptr, n, bitsPerDim).bytes,
-                    layoutFor(nullptr, std::min(n, kSmallBuild), bitsPerDim).bytes);
+    return bytesUpTo(n, bitsPerDim <= 10 ? 4 : 8, [&](uint32_t m) { return layoutFor(nullptr, m, bitsPerDim).bytes; });
 }
 
 int lbvhBuild(clr_ctx* ctx, const LbvhInput& in, uint32_t n, uint32_t bits,

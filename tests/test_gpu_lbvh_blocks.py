@@ -41,8 +41,9 @@ def test_block_edges_byte_exact(gpu_ctx, n, bits, soup):
     assert_same_as_oracle(gpu_ctx, SOUPS[soup](n), bits)
 
 
-@pytest.mark.parametrize("n,bits", [(1 << 19, 10), ((1 << 19) + 1, 10), ((1 << 19) + 1, 20)])
-def test_block_size_rule_byte_exact(gpu_ctx, n, bits):
+@pytest.mark.parametrize("n,bits", [(1 << 19, 10), ((1 << 19) + 1, 10), ((1 << 19) + 1, 20),
+                                    (1 << 18, 20), ((1 << 18) + 1, 20)])
+def test_block_and_tile_rules_byte_exact(gpu_ctx, n, bits):
     assert_same_as_oracle(gpu_ctx, random_soup(n, 3, dup=True), bits)
 
 
@@ -61,17 +62,18 @@ def test_segmented_scenes_across_blocks(gpu_ctx, sizes):
     assert gpu_ctx.device_status() == 0
 
 
-def test_memory_reserved_for_more_serves_fewer(gpu_ctx):
-    """Below 2^19 triangles there are more blocks than just above."""
+@pytest.mark.parametrize("n,bits", [(1 << 19, 10), (1 << 19, 20), (1 << 18, 20)])
+def test_memory_reserved_for_more_serves_fewer(gpu_ctx, n, bits):
+    """At the end of a small shape's range there are more blocks of leaves or
+    sort tiles than just above."""
     import torch
 
     ctx = ca.Context()
-    ca.LBVHBuilder(ctx, (1 << 19) + 1, 10)
-    soup = random_soup(1 << 19, 9, dup=False)
-    tris = torch.from_numpy(soup).cuda()
-    inodes, leaves = ca.node_buffers(1 << 19)
+    ca.LBVHBuilder(ctx, n + 1, bits)
+    tris = torch.from_numpy(random_soup(n, 9, dup=False)).cuda()
+    inodes, leaves = ca.node_buffers(n)
     torch.cuda.synchronize()
     before = torch.cuda.mem_get_info()[0]
-    ca.LBVHBuilder(ctx, 0).perform_soup(tris, 1 << 19, 10, inodes, leaves)
+    ca.LBVHBuilder(ctx, 0).perform_soup(tris, n, bits, inodes, leaves)
     torch.cuda.synchronize()
     assert torch.cuda.mem_get_info()[0] == before
