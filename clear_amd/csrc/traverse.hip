@@ -1,7 +1,8 @@
 // Closest-hit traversal of the LBVH for gfx950.
 //
 // Replaces rayIntersection (OpenCL_PathTracer/OpenCL/bvh_traversal.cl:182-215)
-// with the same visiting order and tests, so hits agree bit for bit:
+// with the same visiting order and tests, so hits agree bit for bit
+// (k_trace_closest; many rays: k_trace_reference):
 //   * pop a node, test its own box (rayAABBIntersection, :160-179) against the
 //     current t; for child 0 then child 1: push an internal child, or test the
 //     leaf box and then the triangle (Moller-Trumbore, :54-108);
@@ -80,6 +81,12 @@ __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const c
         for (int k = 0; k < 2; ++k) {
             const bool leaf = ((c.x >> (8 * k)) & 0xFFu) != 0;
             const uint32_t ci = k ? c.z : c.y;
+            if (leaf ? ci >= n : ci + 1 >= n) {  // malformed nodes: an empty box and no child
+                box[k][0] = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
+                box[k][1] = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+                ref[k] = dev::kNone;
+                continue;
+            }
             const float4* p = leaf ? reinterpret_cast<const float4*>(leaves + ci)
                                    : reinterpret_cast<const float4*>(inodes + ci);
             box[k][0] = p[0];
@@ -349,6 +356,54 @@ __device__ __forceinline__ void traceTwo(W& w0, W& w1, const float* __restrict__
     if (over) atomicOr(status, kStatusStackOverflow);
 }
 
+// The reference's walk over the traversal layout. A wave takes as long as its
+// longest rays (thousands of visits where k_trace_closest's rays cross a whole
+// scene before they meet anything), so a visit's own latency counts: one ray
+// per lane, both children's records requested before their boxes are tested.
+// 1,000,003 triangles, 524,309 rays: 8.07 ms with k_trace_closest, 5.61 with two
+// rays per lane and no early requests, 4.25 now; with 2,000,000
+// triangles and 1,000,000 rays 21.0 and 7.1 (first and last). A third
+// request for the stack's top was slower (3.7 -> 4.2 ms): a visit is bound by
+// its instructions.
+template <bool STATS>
+__global__ __launch_bounds__(kOrdBlock) void k_trace_reference(
+    dev::GeomScene g, const float* __restrict__ rays, uint32_t numRays, uint32_t* __restrict__ hitFace,
+    float* __restrict__ hitT, uint32_t* __restrict__ stats, uint32_t* __restrict__ status,
+    uint32_t* __restrict__ spill) {
+    constexpr int kPairs = kOrdHalf;
+    using S = dev::PairStack<kPairs, dev::kStackDepth>;
+    __shared__ uint2 s_stack[kPairs * kOrdBlock];
+    const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
+    const uint32_t lanes = gridDim.x * kOrdBlock;
+    const S stk{s_stack + threadIdx.x, kOrdBlock, reinterpret_cast<uint2*>(spill) + gid, lanes};
+    dev::ReferenceWalk<STATS, S> w(g, stk);
+    const size_t R = numRays;
+    bool over = false;
+    auto start = [&](uint32_t r) {
+        const dev::V3 o = {rays[r], rays[R + r], rays[2 * R + r]};
+        const dev::V3 d = {rays[3 * R + r], rays[4 * R + r], rays[5 * R + r]};
+        w.begin(o, d, rays[6 * R + r]);
+    };
+    uint32_t r = gid;
+    if (r < numRays) start(r);
+    while (r < numRays) {
+        if (!w.done()) w.step();
+        if (w.done()) {
+            over |= w.over();
+            const bool hit = w.best != kEmpty && !isinf(w.t);
+            hitFace[r] = hit ? w.best : kEmpty;
+            hitT[r] = w.t;
+            if constexpr (STATS) {
+                stats[2 * (size_t)r] = w.st.visits;
+                stats[2 * (size_t)r + 1] = w.st.tests;
+            }
+            r = numRays - r > lanes ? r + lanes : numRays;
+            if (r < numRays) start(r);
+        }
+    }
+    if (over) atomicOr(status, kStatusStackOverflow);
+}
+
 // With counts per ray: the walks whose visits and tests are defined.
 template <bool WIDE>
 __global__ __launch_bounds__(kOrdBlock) void k_trace_counts(
@@ -474,19 +529,27 @@ void launchAccelBuild(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves,
         k_accel_build<<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, vertices, faces, anodes, atris);
 }
 
+namespace {
+// Grid of a kernel that runs traceTwo (16 waves per CU; LDS: 16 KiB per
+// 128-thread block) and its stacks' spill memory.
+int traceGrid(clr_ctx* ctx, uint32_t numRays, uint32_t& grid) {
+    int cus = 0;
+    int rc = hipCheck(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
+    if (rc) return rc;
+    grid = std::max(1u, std::min((uint32_t)cus * 8u, (numRays + kOrdBlock - 1) / kOrdBlock));
+    const size_t lanes = (size_t)grid * kOrdBlock;
+    return ensureTraceSpill(ctx, lanes * 2 * (dev::kStackPairs - kOrdHalf) * sizeof(uint32_t));
+}
+}  // namespace
+
 int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
                  uint32_t n, const clr_float3* vertices, const clr_face* faces, const float* rays, uint32_t numRays,
                  uint32_t* hitFace, float* hitT, uint32_t* stats, hipStream_t stream, bool wide) {
     if (numRays == 0) return CLR_OK;
     int rc = ensureStatus(ctx);
     if (rc) return rc;
-    int cus = 0;
-    rc = hipCheck(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
-    if (rc) return rc;
-    // 16 waves per CU (LDS: 16 KiB per 128-thread block).
-    const uint32_t grid = std::max(1u, std::min((uint32_t)cus * 8u, (numRays + kOrdBlock - 1) / kOrdBlock));
-    const size_t lanes = (size_t)grid * kOrdBlock;
-    rc = ensureTraceSpill(ctx, lanes * 2 * (dev::kStackPairs - kOrdHalf) * sizeof(uint32_t));
+    uint32_t grid = 0;
+    rc = traceGrid(ctx, numRays, grid);
     if (rc) return rc;
     clr_scene_dev sd{};
     sd.vertices = vertices;
@@ -509,6 +572,13 @@ int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     return hipCheck(ctx, hipGetLastError(), "trace launch");
 }
 
+// The layout pays for itself from 2^14 rays, 4096 triangles and a ray for every
+// 128 triangles on (us over the drop-in nodes / over the layout): 1000 triangles,
+// 16384 rays 75 / 74 and 2 triangles 12 / 21; 20,000 triangles, 4096 rays 198 / 217,
+// 16384 rays 238 / 234, 100,000 rays 283 / 272; 300,000 triangles, 4096 rays 729 / 740,
+// 16384 rays 1224 / 940; 2,000,000 triangles, 16384 rays 3819 / 3342.
+constexpr uint32_t kLayoutMinRays = 1u << 14, kLayoutMinFaces = 4096, kLayoutFacesPerRay = 128;
+
 int traceClosest(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh,
                  uint32_t n, const clr_float3* vertices, const clr_face* faces, const float* rays,
                  uint32_t numRays, uint32_t* hitFace, float* hitT, uint32_t* stats,
@@ -516,6 +586,38 @@ int traceClosest(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     if (numRays == 0) return CLR_OK;
     int rc = ensureStatus(ctx);
     if (rc) return rc;
+    // Enough rays of an LBVH walk over the traversal layout, which needs memory:
+    // not while the stream is being captured (a graph would keep its address),
+    // and not when there is none.
+    if (!bvh && numRays >= kLayoutMinRays && n >= kLayoutMinFaces && numRays >= n / kLayoutFacesPerRay) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+            (void)hipGetLastError();
+            capture = hipStreamCaptureStatusActive;
+        }
+        if (capture == hipStreamCaptureStatusNone) {
+            uint32_t grid = 0;
+            clr_scene_dev sd{};
+            sd.vertices = vertices;
+            sd.faces = faces;
+            sd.internalNodes = inodes;
+            sd.leafNodes = leaves;
+            sd.numFaces = n;
+            dev::GeomScene g;
+            rc = traceGrid(ctx, numRays, grid);
+            if (!rc) rc = buildAccel(ctx, sd, AccelKind::kBinary, g, stream);
+            if (!rc) {
+                if (stats)
+                    k_trace_reference<true><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats,
+                                                                            ctx->devStatus, ctx->traceSpill);
+                else
+                    k_trace_reference<false><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats,
+                                                                             ctx->devStatus, ctx->traceSpill);
+                return hipCheck(ctx, hipGetLastError(), "trace launch");
+            }
+            (void)hipGetLastError();  // no memory for it
+        }
+    }
     const unsigned grid = (numRays + kTraceBlock - 1) / kTraceBlock;
     const float4* b4 = reinterpret_cast<const float4*>(bvh);
     if (stats)

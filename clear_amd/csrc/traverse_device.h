@@ -95,11 +95,14 @@ struct TraceStats {
 // rayAABBIntersection (bvh_traversal.cl:160-179): per axis the candidate plane
 // on the origin's side, t = (plane - org) / dir (-1 when inside or dir == 0),
 // maxt = max t; reject if maxt < 0 or > tBound; the entry point must lie in the
-// box on every axis (or that axis produced maxt).
-__device__ __forceinline__ bool boxTest(float4 mn, float4 mx, V3 o, V3 d, float tBound) {
+// box on every axis (or that axis produced maxt). `enter` gets maxt, or -inf
+// for an origin inside: a box that passes for one bound passes for every bound
+// that is not below `enter`, and one that fails fails for every smaller bound.
+__device__ __forceinline__ bool boxEnter(float4 mn, float4 mx, V3 o, V3 d, float tBound, float& enter) {
     const int lx = o.x < mn.x ? -1 : (o.x > mx.x ? 1 : 0);
     const int ly = o.y < mn.y ? -1 : (o.y > mx.y ? 1 : 0);
     const int lz = o.z < mn.z ? -1 : (o.z > mx.z ? 1 : 0);
+    enter = -INFINITY;
     if ((lx | ly | lz) == 0) return true;
     const float px = o.x < mn.x ? mn.x : (o.x > mx.x ? mx.x : 0.0f);
     const float py = o.y < mn.y ? mn.y : (o.y > mx.y ? mx.y : 0.0f);
@@ -108,6 +111,7 @@ __device__ __forceinline__ bool boxTest(float4 mn, float4 mx, V3 o, V3 d, float 
     const float ty = (ly != 0 && d.y != 0.0f) ? ((py - o.y) / d.y) : -1.0f;
     const float tz = (lz != 0 && d.z != 0.0f) ? ((pz - o.z) / d.z) : -1.0f;
     const float maxt = omax(tx, omax(ty, tz));
+    enter = maxt;
     if (maxt < 0.0f || maxt > tBound) return false;
     const float cx = o.x + maxt * d.x;
     const float cy = o.y + maxt * d.y;
@@ -116,6 +120,10 @@ __device__ __forceinline__ bool boxTest(float4 mn, float4 mx, V3 o, V3 d, float 
     const bool hy = (cy >= mn.y && cy <= mx.y) || ty == maxt;
     const bool hz = (cz >= mn.z && cz <= mx.z) || tz == maxt;
     return hx && hy && hz;
+}
+__device__ __forceinline__ bool boxTest(float4 mn, float4 mx, V3 o, V3 d, float tBound) {
+    float enter;
+    return boxEnter(mn, mx, o, d, tBound, enter);
 }
 
 // Geometric part of rayTriangleIntersection (bvh_traversal.cl:54-92) with a
@@ -744,6 +752,161 @@ struct PairStack {
     }
     __device__ __forceinline__ uint64_t* global(int k) const {
         return reinterpret_cast<uint64_t*>(spill + (size_t)(k - L) * spillStride);
+    }
+};
+
+// The reference's walk (lbvhClosest: its order, box tests, hits, counts and
+// overflow) over the binary traversal layout, for many rays. lbvhClosest is
+// bound by the latency of a pop: a node's record, then its leaves, their faces
+// and their vertices, each a dependent load, for boxes that mostly fail. Here a
+// visit tests both children's boxes, which came with the node's own record: a
+// box that fails now fails at its pop, when t is smaller still, so it is never
+// fetched; one that passes is kept with its entry distance, which decides at
+// its pop (boxEnter). A kept child lies in the slot that it has on the
+// reference's stack, where failing ones take slots too (`live` marks the kept
+// ones), so a push beyond 64 entries is dropped at the same place. The one way
+// for t to let a box in again is a triangle with vertices that are not finite,
+// which is accepted with t = NaN, and every box within NaN: the ray then
+// starts again and keeps every box it meets (`keepAll`).
+template <bool STATS, class Stack>
+struct ReferenceWalk {
+    GeomScene g;
+    const Stack& stack;
+    V3 o, d;
+    float t;
+    uint32_t best, node, pops;
+    uint64_t live;
+    bool ended, overflowed, keepAll;
+    TraceStats st;
+    __device__ __forceinline__ bool done() const { return ended; }
+    __device__ __forceinline__ bool over() const { return overflowed; }
+
+    __device__ __forceinline__ ReferenceWalk(const GeomScene& g_, const Stack& s_) : g(g_), stack(s_) {}
+
+    __device__ __forceinline__ void leaf(uint32_t face) {
+        if constexpr (STATS) ++st.tests;
+        if (face >= g.n) {  // malformed nodes
+            overflowed = true;
+            return;
+        }
+        float b1, b2;
+        uint32_t flag;
+        if (triTestPacked(g.atris, o, d, face, t, b1, b2, flag)) best = face;
+    }
+
+    __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax) {
+        o = o_;
+        d = d_;
+        start = tmax;
+        keepAll = false;
+        restart();
+    }
+    __device__ __forceinline__ void restart() {
+        t = start;
+        best = kNone;
+        node = kNone;
+        live = 0;
+        ended = overflowed = false;
+        pops = 1;
+        depth = 0;
+        st = {0u, 0u};
+        const float4* p = g.n == 1 ? reinterpret_cast<const float4*>(g.leaves) : reinterpret_cast<const float4*>(g.inodes);
+        const bool pass = boxTest(p[0], p[1], o, d, t);
+        if (g.n == 1 && pass) leaf(reinterpret_cast<const uint32_t*>(p + 2)[0]);
+        if (g.n > 1 && pass) {
+            node = 0;
+            cur = load(0);
+        } else {
+            ended = true;
+        }
+    }
+
+    __device__ __forceinline__ void step() {
+        if constexpr (STATS) ++st.visits;
+        const float4 lo0 = cur.v[0], hi0 = cur.v[1], lo1 = cur.v[2], hi1 = cur.v[3];
+        const Record c0 = load(__float_as_uint(lo0.w)), c1 = load(__float_as_uint(hi0.w));
+        const uint32_t r0 = __float_as_uint(lo0.w), r1 = __float_as_uint(hi0.w);
+        float e0, e1;
+        const float bound = keepAll ? INFINITY : t;
+        const bool p0 = boxEnter(lo0, hi0, o, d, bound, e0), p1 = boxEnter(lo1, hi1, o, d, bound, e1);
+        const bool l0 = (r0 & kLeafRef) != 0, l1 = (r1 & kLeafRef) != 0;
+        if (l0 && p0 && !(e0 > t)) leaf(r0 & ~kLeafRef);
+        if (l1 && p1 && !(e1 > t)) leaf(r1 & ~kLeafRef);
+        if (best != kNone && t != t && !keepAll) {
+            keepAll = true;
+            restart();
+            return;
+        }
+        bool k0 = false, k1 = false;
+        int s0 = 0, s1 = 0;
+        if (!l0) {
+            s0 = depth++;
+            k0 = keep(p0, r0, s0);
+        }
+        if (!l1) {
+            s1 = depth++;
+            k1 = keep(p1, r1, s1);
+        }
+        if (k1 && !(e1 > t)) {
+            if (k0) {
+                stack.put(s0, r0, e0);
+                live |= 1ull << s0;
+            }
+            node = r1;
+            cur = c1;
+            depth = s1;
+            ++pops;
+        } else {
+            pops += k1;
+            if (k0 && !(e0 > t)) {
+                node = r0;
+                cur = c0;
+                depth = s0;
+                ++pops;
+            } else {
+                pops += k0;
+                node = kNone;
+                while (live) {
+                    depth = 63 - __builtin_clzll(live);
+                    live &= ~(1ull << depth);
+                    ++pops;
+                    const uint2 v = stack.get(depth);
+                    if (!(__uint_as_float(v.y) > t)) {
+                        node = v.x;
+                        break;
+                    }
+                }
+                ended = node == kNone;
+                cur = load(node);
+            }
+        }
+        if (pops > 2u * g.n + 2u) {  // malformed nodes: stop and flag
+            ended = true;
+            overflowed = true;
+        }
+    }
+
+private:
+    struct Record {
+        float4 v[4];
+    };
+    Record cur;  // of `node`
+    __device__ __forceinline__ Record load(uint32_t ref) const {
+        const float4* p = g.anodes + 4 * (size_t)(ref < g.n - 1u ? ref : 0u);  // a leaf, or kNone: any record
+        return {p[0], p[1], p[2], p[3]};
+    }
+    int depth;    // slots in use on the reference's stack
+    float start;  // the ray's bound
+    // Whether an internal child in `slot` is kept. One that fails is popped
+    // later for nothing.
+    __device__ __forceinline__ bool keep(bool pass, uint32_t ref, int slot) {
+        if (slot >= kStackDepth || ref >= g.n - 1u) {
+            overflowed = true;
+            if (slot >= kStackDepth) --depth;
+            return false;
+        }
+        pops += !pass;
+        return pass;
     }
 };
 

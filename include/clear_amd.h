@@ -212,7 +212,10 @@ int clr_lbvh_last_profile(clr_ctx* ctx, float* msPerStage, int maxStages, int* n
  *   stats   optional device uint32_t[2*numRays]: internal-node visits and
  *           triangle tests per ray (NULL to skip)
  * Face indices are 32-bit (the reference truncates to 16 bits,
- * bvh_traversal.cl:43,55). */
+ * bvh_traversal.cl:43,55). Many rays against a scene that is not small walk a
+ * copy of the nodes in the context's scratch (the same order, tests, hits and
+ * counts); without memory for it, and in a call that is being captured, the
+ * nodes themselves. */
 int clr_trace_closest(clr_ctx* ctx, const clr_lbvh_inode* internalNodes,
                       const clr_lbvh_leaf* leafNodes, uint32_t numFaces,
                       const clr_float3* vertices, const clr_face* faces,
