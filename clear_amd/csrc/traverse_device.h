@@ -62,7 +62,7 @@ struct GeomScene {
     uint32_t n;
     const clr_float3* verts;
     const clr_face* faces;
-    const float4* anodes = nullptr;  // [n - 1][4] (LBVH) or [2n - 1][4] by node (midpoint BVH); walks that count only
+    const float4* anodes = nullptr;  // [n - 1][4] (LBVH) or [2n - 1][4] by node (midpoint BVH); counting and reference walks
     const float4* atris = nullptr;   // [n][3]
     // CPU midpoint BVH (clr_bvh_node[2n - 1], 3 float4 each). When set, the
     // reference-order walks use it instead of inodes / leaves, and the
