@@ -143,11 +143,11 @@ int lbvhBuildSegmented(clr_ctx* ctx, const float* tris, const uint32_t* segOffse
 
 // ---- rendering (render.hip, wavefront.hip) ----
 // The traversal layout a call needs: none (the reference walks read the
-// drop-in nodes), the binary or the 4-wide float records (the counting
-// walks), or the 4-wide byte records (every other walk).
-enum class AccelKind { kNone, kBinary, kWide, kBytes };
+// drop-in nodes), the binary records (the binary counting walk and the
+// reference's walk of many rays), or the 4-wide records (every other walk).
+enum class AccelKind { kNone, kBinary, kWide };
 inline AccelKind accelFor(const clr_render_params& rp) {
-    return (rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL) ? AccelKind::kNone : AccelKind::kBytes;
+    return (rp.flags & CLR_RENDER_REFERENCE_TRAVERSAL) ? AccelKind::kNone : AccelKind::kWide;
 }
 int prepareRenderScene(clr_ctx* ctx, const clr_scene_dev& sd, dev::RScene& S, AccelKind kind, hipStream_t stream);
 int ensureRenderScratch(clr_ctx* ctx, uint32_t numFaces);
@@ -190,10 +190,10 @@ void launchAccelBuild(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves,
                       hipStream_t stream);
 // Bytes of the traversal layout's node array (256-B aligned).
 size_t accelNodeBytes(uint32_t n, bool midpoint);
-// The 4-wide byte records (64 B per node slot) and their build.
-size_t accelByteBytes(uint32_t n, bool midpoint);
-void launchAccelBytes(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
-                      float4* qnodes, hipStream_t stream);
+// The 4-wide records (128 B per node slot) and their build.
+size_t accelWideBytes(uint32_t n, bool midpoint);
+void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
+                     float4* wnodes, hipStream_t stream);
 // Face -> first light map and first environment light of one scene.
 void launchFaceLights(const clr_light_info* lights, uint32_t numLights, uint32_t numFaces, uint32_t* faceLight,
                       int* envLight, hipStream_t stream);

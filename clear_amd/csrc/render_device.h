@@ -55,7 +55,7 @@ __device__ __forceinline__ RScene tableScene(const RScene* table, uint32_t i) {
     S.g.faces = asGlobal(S.g.faces);
     S.g.atris = asGlobal(S.g.atris);
     S.g.bvh = asGlobal(S.g.bvh);
-    S.g.qnodes = asGlobal(S.g.qnodes);
+    S.g.wnodes = asGlobal(S.g.wnodes);
     S.normals = asGlobal(S.normals);
     S.tangents = asGlobal(S.tangents);
     S.uvs = asGlobal(S.uvs);

@@ -168,65 +168,8 @@ struct WideSlots {
                            __uint_as_float(ref[3]));
         o[7] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
-    // The 64-byte form (GeomScene::qnodes). Per axis the grid starts at the
-    // lowest plane and its step is the smallest power of two that reaches the
-    // highest plane in 255 steps; planes round outwards, and a box whose
-    // plane is not ordered against the grid's ends (NaN) takes the end.
-    __device__ __forceinline__ void storeBytes(float4* o) const {
-        float org[3], scale[3];
-        uint32_t qlo[3], qhi[3];
-        for (int a = 0; a < 3; ++a) {
-            float l = INFINITY, h = -INFINITY;
-            bool finite = true;
-            for (int c = 0; c < 4; ++c)
-                if (ref[c] != dev::kNone) {
-                    l = fminf(l, lo[a][c]);
-                    h = fmaxf(h, hi[a][c]);
-                    finite &= fabsf(lo[a][c]) < INFINITY && fabsf(hi[a][c]) < INFINITY;
-                }
-            const float ext = h - l;
-            finite &= ext < 1e38f;
-            qlo[a] = qhi[a] = 0;
-            if (!finite) {
-                org[a] = 0.0f;
-                scale[a] = INFINITY;
-                qhi[a] = 0xFFFFFFFFu;
-                continue;
-            }
-            // 2^e with 255 * 2^e >= ext: the exponent of ext / 255 rounded up.
-            const uint32_t bits = __float_as_uint(ext * (1.0f / 254.5f));
-            const uint32_t e = max((bits + 0x007FFFFFu) >> 23, 1u);
-            const float s = __uint_as_float(e << 23), inv = __uint_as_float(min(254u - e, 254u) << 23);
-            org[a] = l;
-            scale[a] = s;
-            for (int c = 0; c < 4; ++c) {
-                if (ref[c] == dev::kNone) {
-                    qlo[a] |= 255u << (8 * c);
-                    continue;
-                }
-                float fl = floorf((lo[a][c] - l) * inv), fh = ceilf((hi[a][c] - l) * inv);
-                if (l + fl * s > lo[a][c]) fl -= 1.0f;
-                if (l + fh * s < hi[a][c]) fh += 1.0f;
-                const uint32_t ql = fl >= 0.0f && fl <= 255.0f ? (uint32_t)fl : 0u;
-                const uint32_t qh = fh >= 0.0f && fh <= 255.0f ? (uint32_t)fh : 255u;
-                qlo[a] |= ql << (8 * c);
-                qhi[a] |= qh << (8 * c);
-            }
-        }
-        uint4* u = reinterpret_cast<uint4*>(o);
-        o[0] = make_float4(org[0], org[1], org[2], scale[0]);
-        u[1] = make_uint4(qlo[0], qhi[0], qlo[1], qhi[1]);
-        u[2] = make_uint4(qlo[2], qhi[2], __float_as_uint(scale[1]), __float_as_uint(scale[2]));
-        u[3] = make_uint4(ref[0], ref[1], ref[2], ref[3]);
-    }
-    template <bool BYTES>
-    __device__ __forceinline__ void put(float4* records, size_t i) const {
-        if constexpr (BYTES) storeBytes(records + 4 * i);
-        else store(records + 8 * i);
-    }
 };
 
-template <bool BYTES>
 __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves,
                              uint32_t n, float4* __restrict__ records) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -235,7 +178,7 @@ __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const cl
     if (n == 1 && i == 0) {  // a tree of one leaf: a record that holds it
         const float4* p = reinterpret_cast<const float4*>(leaves);
         w.put(0, p[0], p[1], leaves[0].objIdx | dev::kLeafRef);
-        w.put<BYTES>(records, 0);
+        w.store(records);
         return;
     }
     if (i + 1 >= n) return;
@@ -262,12 +205,11 @@ __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const cl
             w.put(2 * k + m, p[0], p[1], gl ? (leaves[gi].objIdx | dev::kLeafRef) : gi);
         }
     }
-    w.put<BYTES>(records, i);
+    w.store(records + 8 * (size_t)i);
 }
 
 // The same records for a CPU midpoint BVH, by node number (leaf node slots
 // stay unused).
-template <bool BYTES>
 __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, float4* __restrict__ records) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t numNodes = 2 * n - 1;
@@ -277,7 +219,7 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
     w.clear();
     if (n == 1 && c.y == kEmpty) {  // a tree of one leaf: a record that holds it
         w.put(0, bvh[0], bvh[1], c.x | dev::kLeafRef);
-        w.put<BYTES>(records, 0);
+        w.store(records);
         return;
     }
     if (c.y == kEmpty || c.x >= numNodes || c.y >= numNodes) return;
@@ -299,7 +241,7 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
             w.put(2 * k + m, q[0], q[1], gc.y == kEmpty ? (gc.x | dev::kLeafRef) : gi);
         }
     }
-    w.put<BYTES>(records, i);
+    w.store(records + 8 * (size_t)i);
 }
 
 // Trace with the ordered traversal, grid-stride over the rays with a fixed
@@ -460,23 +402,13 @@ size_t accelNodeBytes(uint32_t n, bool midpoint) {
 }
 
 size_t accelWideBytes(uint32_t n, bool midpoint) { return 2 * accelNodeBytes(n, midpoint); }
-size_t accelByteBytes(uint32_t n, bool midpoint) { return accelNodeBytes(n, midpoint); }
 
-namespace {
-template <bool BYTES>
-void launchWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
-                float4* records, hipStream_t stream) {
+void launchAccelWide(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
+                     float4* wnodes, hipStream_t stream) {
     if (bvh)
-        k_accel_wide_bvh<BYTES><<<(2 * n - 1 + 255) / 256, 256, 0, stream>>>(reinterpret_cast<const float4*>(bvh), n,
-                                                                             records);
+        k_accel_wide_bvh<<<(2 * n - 1 + 255) / 256, 256, 0, stream>>>(reinterpret_cast<const float4*>(bvh), n, wnodes);
     else
-        k_accel_wide<BYTES><<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, records);
-}
-}  // namespace
-
-void launchAccelBytes(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves, const clr_bvh_node* bvh, uint32_t n,
-                      float4* qnodes, hipStream_t stream) {
-    launchWide<true>(inodes, leaves, bvh, n, qnodes, stream);
+        k_accel_wide<<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, wnodes);
 }
 
 int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomScene& g, hipStream_t stream) {
@@ -485,22 +417,27 @@ int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomS
     g = dev::GeomScene{sd.internalNodes, sd.leafNodes, n, sd.vertices, sd.faces};
     g.bvh = reinterpret_cast<const float4*>(sd.bvhNodes);
     if (kind == AccelKind::kNone) return CLR_OK;
-    const size_t nodeBytes = kind == AccelKind::kBinary ? accelNodeBytes(n, midpoint)
-                             : kind == AccelKind::kWide ? accelWideBytes(n, midpoint)
-                                                        : accelByteBytes(n, midpoint);
-    const size_t need = nodeBytes + (((size_t)n * 48 + 255) & ~size_t(255));
+    const size_t nodeBytes = kind == AccelKind::kBinary ? accelNodeBytes(n, midpoint) : accelWideBytes(n, midpoint);
+    const size_t triBytes = ((size_t)n * 48 + 255) & ~size_t(255);
+    // Room for either kind where it can be had, so that after a call of one
+    // kind a captured call of the other allocates nothing.
+    const size_t need = nodeBytes + triBytes, either = accelWideBytes(n, midpoint) + triBytes;
     if (ctx->accelBytes < need) {
         int rc = hipCheck(ctx, hipDeviceSynchronize(), "accel regrow sync");
         if (rc) return rc;
         if (ctx->accel) (void)hipFree(ctx->accel);
         ctx->accel = nullptr;
         ctx->accelBytes = 0;
-        hipError_t e = hipMalloc(&ctx->accel, need);
-        if (e != hipSuccess) {
+        for (size_t bytes : {either, need}) {
+            if (hipMalloc(&ctx->accel, bytes) == hipSuccess) {
+                ctx->accelBytes = bytes;
+                break;
+            }
             (void)hipGetLastError();
-            return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "traversal layout of " + std::to_string(need) + " bytes");
+            ctx->accel = nullptr;
         }
-        ctx->accelBytes = need;
+        if (!ctx->accel)
+            return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "traversal layout of " + std::to_string(need) + " bytes");
     }
     float4* nodes = static_cast<float4*>(ctx->accel);
     float4* tris = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes);
@@ -509,12 +446,9 @@ int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomS
     g.atris = tris;
     if (kind == AccelKind::kBinary) {
         g.anodes = nodes;
-    } else if (kind == AccelKind::kWide) {
-        g.wnodes = nodes;
-        launchWide<false>(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, nodes, stream);
     } else {
-        g.qnodes = nodes;
-        launchWide<true>(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, nodes, stream);
+        g.wnodes = nodes;
+        launchAccelWide(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, nodes, stream);
     }
     return hipCheck(ctx, hipGetLastError(), "traversal layout launch");
 }
@@ -559,7 +493,7 @@ int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     sd.numFaces = n;
     sd.bvhNodes = bvh;
     dev::GeomScene g;
-    rc = buildAccel(ctx, sd, !stats ? AccelKind::kBytes : wide ? AccelKind::kWide : AccelKind::kBinary, g, stream);
+    rc = buildAccel(ctx, sd, !stats || wide ? AccelKind::kWide : AccelKind::kBinary, g, stream);
     if (rc) return rc;
     if (!stats)
         k_trace_wide<<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, ctx->devStatus, ctx->traceSpill);

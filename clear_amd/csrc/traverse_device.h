@@ -68,21 +68,13 @@ struct GeomScene {
     // reference-order walks use it instead of inodes / leaves, and the
     // traversal layout is indexed by its node numbers.
     const float4* bvh = nullptr;
-    // 4-wide records of the counting 4-wide walk ([slots][8], slots as anodes):
+    // 4-wide records of the 4-wide walks ([slots][8], slots as anodes):
     // record i holds the up to four grandchildren of internal node i (the
     // children of each internal child, a leaf child itself), as SoA
     // float4s: lo.x, lo.y, lo.z, hi.x, hi.y, hi.z of slots 0..3, then the
     // four references (face | kLeafRef, node, or kNone for an empty slot
     // with an empty box). Unused when null.
     const float4* wnodes = nullptr;
-    // The same records in 64 bytes for WideWalk ([slots][4]): child boxes as
-    // bytes on the record's own grid. float4s: origin.xyz, scale.x | bytes of
-    // lo.x, hi.x, lo.y, hi.y of slots 0..3 | bytes of lo.z, hi.z, then
-    // scale.y, scale.z | the four references. A plane is origin + byte *
-    // scale, rounded outwards (scale a power of two); an axis on which some
-    // box is not finite has scale infinity and bytes 0 and 255, which every
-    // ray passes.
-    const float4* qnodes = nullptr;
 };
 constexpr uint32_t kLeafRef = 0x80000000u;
 static_assert(sizeof(clr_lbvh_inode) == 48 && sizeof(clr_lbvh_leaf) == 48 && sizeof(clr_bvh_node) == 48,
@@ -916,18 +908,11 @@ private:
 // way, as long as none that holds an accepted triangle is passed over. That
 // leaves the box arithmetic free, and a visit is bound by its instructions
 // (few lanes are active, so every instruction counts in full):
-//   * a record is 64 bytes (GeomScene::qnodes): four 16-byte loads from half a
-//     cache line where the float planes took seven from a whole one; the
-//     walks wait on L2, and the records of a scene take half of it;
-//   * near and far planes are chosen by the ray's direction signs (two planes
-//     an axis instead of four and a min and max each), and a plane's distance
-//     is one fma: t = byte * (scale * inv) + (origin * inv - o * inv). The
-//     cancellation error of that form, a few 2^-24 |o * inv| (or of t), is
-//     covered by moving the near planes' constant down and the far planes'
-//     up by 2^-21 |o * inv|; the relative pad of slabEnter (1 -+ 2^-16 on entry
-//     and exit) is one factor 1 - 2^-15 on the entry. Every box that
-//     slabEnter admits is admitted; NaNs (from infinite products) are ignored
-//     by min / max and so admit.
+//   * near and far planes are chosen by the ray's direction signs: two planes
+//     an axis instead of four and a min and max each. The plane distances, pads
+//     and comparisons are slabEnter's, in its order, so a box is admitted exactly
+//     when slabEnter admits it (min and max pick the same planes, since rounding
+//     keeps (lo - o) * inv and (hi - o) * inv in order);
 //   * leaf entries are tested in a loop over each lane's own leaves, so the
 //     triangle test runs as often as the lane with the most leaves has, not
 //     once for each of the four slots in which some lane has one;
@@ -942,19 +927,18 @@ private:
 // Against the counting walk in the same kernels: 2^22 random rays on 2^24
 // triangles 8.72 -> 8.10 ms, 512x512 at 8 spp of the differentiation scene
 // 31.9 -> 26.3 ms (forward and adjoint), 640x360 at 16 spp of the showcase
-// scene on the wavefront renderer 24.3 -> 21.4 ms (with float records). Byte
-// records, the branch-free leaf test, the stack without flat accesses and the
-// alpha lookup out of line: the random rays 9.99 -> 8.33 ms (2.79 -> 1.85 ->
-// 1.2 ms of it building records), 1080p at 32 spp on the megakernel 124 ->
-// 107 ms.
+// scene on the wavefront renderer 24.3 -> 21.4 ms. Records of 64 bytes (child
+// boxes as bytes on the record's own grid, 9.27 -> 8.22 ms on the random rays,
+// 110 -> 107 ms on 1080p at 32 spp) hold planes in fewer bits than the boxes
+// have, and a plane far from the record's corner lost hits: not used.
 template <class Alpha, class Stack>
 struct WideWalk {
-    const float4* qn;
+    const float4* wn;
     const float4* tris;
     uint32_t limit;  // more visits than this mean malformed records
     const Stack& stack;
     Alpha alpha;
-    V3 o, d, inv, cn, cf;  // near plane distance: plane * inv + cn; far: plane * inv + cf
+    V3 o, d, inv;
     float t, b1, b2;
     uint32_t best, bound, node, left;  // node: kNone when the walk has ended
     int depth;
@@ -962,9 +946,9 @@ struct WideWalk {
     static constexpr uint32_t kAny = 1u, kOver = 2u;
 
     __device__ __forceinline__ WideWalk(const GeomScene& g, const Stack& s_, const Alpha& a_)
-        : qn(asGlobal(g.qnodes)), tris(asGlobal(g.atris)), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
+        : wn(asGlobal(g.wnodes)), tris(asGlobal(g.atris)), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
     __device__ __forceinline__ void rebind(const GeomScene& g, const Alpha& a_) {
-        qn = asGlobal(g.qnodes);
+        wn = asGlobal(g.wnodes);
         tris = asGlobal(g.atris);
         limit = 2u * g.n + 2u;
         alpha = a_;
@@ -975,12 +959,7 @@ struct WideWalk {
     __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax, bool anyHit = false, uint32_t bestFace = kNone) {
         o = o_;
         d = d_;
-        auto recip = [](float v) { return __builtin_amdgcn_rcpf(fabsf(v) > 1e-20f ? v : copysignf(1e-20f, v)); };
-        inv = {recip(d.x), recip(d.y), recip(d.z)};
-        constexpr float kSlack = 1.0f / 2097152.0f;
-        const V3 oi = {o.x * inv.x, o.y * inv.y, o.z * inv.z};
-        cn = {-oi.x - fabsf(oi.x) * kSlack, -oi.y - fabsf(oi.y) * kSlack, -oi.z - fabsf(oi.z) * kSlack};
-        cf = {-oi.x + fabsf(oi.x) * kSlack, -oi.y + fabsf(oi.y) * kSlack, -oi.z + fabsf(oi.z) * kSlack};
+        inv = {safeInv(d.x), safeInv(d.y), safeInv(d.z)};
         t = tmax;
         b1 = b2 = 0.0f;
         best = bound = bestFace;
@@ -1022,32 +1001,24 @@ struct WideWalk {
 
     // Visits `node`.
     __device__ __forceinline__ void step() {
-        const float4* qp = qn + 4 * (size_t)node;
-        const float4 q0 = qp[0];
-        const uint4 q1 = reinterpret_cast<const uint4*>(qp)[1], q2 = reinterpret_cast<const uint4*>(qp)[2];
-        const uint4 r = reinterpret_cast<const uint4*>(qp)[3];
-        const bool sx = inv.x < 0.0f, sy = inv.y < 0.0f, sz = inv.z < 0.0f;
-        const uint32_t nx = sx ? q1.y : q1.x, fx = sx ? q1.x : q1.y;
-        const uint32_t ny = sy ? q1.w : q1.z, fy = sy ? q1.z : q1.w;
-        const uint32_t nz = sz ? q2.y : q2.x, fz = sz ? q2.x : q2.y;
-        const float kx = q0.w * inv.x, ky = __uint_as_float(q2.z) * inv.y, kz = __uint_as_float(q2.w) * inv.z;
-        const float nbx = __builtin_fmaf(q0.x, inv.x, cn.x), fbx = __builtin_fmaf(q0.x, inv.x, cf.x);
-        const float nby = __builtin_fmaf(q0.y, inv.y, cn.y), fby = __builtin_fmaf(q0.y, inv.y, cf.y);
-        const float nbz = __builtin_fmaf(q0.z, inv.z, cn.z), fbz = __builtin_fmaf(q0.z, inv.z, cf.z);
+        const float4* wp = wn + 8 * (size_t)node;
+        const int nx = inv.x < 0.0f ? 3 : 0, ny = inv.y < 0.0f ? 4 : 1, nz = inv.z < 0.0f ? 5 : 2;
+        const float4 ax = wp[nx], ay = wp[ny], az = wp[nz], bx = wp[3 - nx], by = wp[5 - ny], bz = wp[7 - nz];
+        const uint4 r = reinterpret_cast<const uint4*>(wp)[6];
         uint32_t leaves = 0;
-        auto entry = [&](uint32_t slot, uint32_t ref) {
-            auto byte = [&](uint32_t v) { return (float)((v >> (8u * slot)) & 0xFFu); };
-            const float tn = fmaxf(fmaxf(__builtin_fmaf(byte(nx), kx, nbx), __builtin_fmaf(byte(ny), ky, nby)),
-                                   fmaxf(__builtin_fmaf(byte(nz), kz, nbz), 0.0f)) *
-                             (1.0f - 1.0f / 32768.0f);
-            const float tf = fminf(fminf(__builtin_fmaf(byte(fx), kx, fbx), __builtin_fmaf(byte(fy), ky, fby)),
-                                   fminf(__builtin_fmaf(byte(fz), kz, fbz), t));
-            const bool pass = tn <= tf;
+        auto entry = [&](uint32_t slot, V3 lo, V3 hi, uint32_t ref) {
+            const float tn = fmaxf(fmaxf((lo.x - o.x) * inv.x, (lo.y - o.y) * inv.y), fmaxf((lo.z - o.z) * inv.z, 0.0f));
+            const float tf = fminf(fminf((hi.x - o.x) * inv.x, (hi.y - o.y) * inv.y), (hi.z - o.z) * inv.z) * kPadUp;
+            const float e = tn * kPadDown;
+            const bool pass = e <= fminf(tf, t);
             const uint32_t isLeaf = (uint32_t)((int32_t)ref >> 31);  // all ones; empty slots too, skipped below
             leaves |= (pass ? 1u << slot : 0u) & isLeaf;
-            return (pass ? ((__float_as_uint(tn) & ~3u) | slot) : 0xFFFFFFFFu) | isLeaf;
+            return (pass ? ((__float_as_uint(e) & ~3u) | slot) : 0xFFFFFFFFu) | isLeaf;
         };
-        uint32_t k0 = entry(0u, r.x), k1 = entry(1u, r.y), k2 = entry(2u, r.z), k3 = entry(3u, r.w);
+        uint32_t k0 = entry(0u, {ax.x, ay.x, az.x}, {bx.x, by.x, bz.x}, r.x);
+        uint32_t k1 = entry(1u, {ax.y, ay.y, az.y}, {bx.y, by.y, bz.y}, r.y);
+        uint32_t k2 = entry(2u, {ax.z, ay.z, az.z}, {bx.z, by.z, bz.z}, r.z);
+        uint32_t k3 = entry(3u, {ax.w, ay.w, az.w}, {bx.w, by.w, bz.w}, r.w);
         while (leaves) {
             const uint32_t slot = (uint32_t)__builtin_ctz(leaves);
             leaves &= leaves - 1u;

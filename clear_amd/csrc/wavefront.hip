@@ -1113,7 +1113,7 @@ int prepareBatchScenes(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t numSc
     size_t bytes = align(sizeof(RScene) * numScenes) + align(sizeof(int) * numScenes);
     for (uint32_t s = 0; s < numScenes; ++s) {
         const uint32_t n = scenes[s].numFaces;
-        bytes += accelByteBytes(n, scenes[s].bvhNodes != nullptr) + align(48ull * n) + align(4ull * n);
+        bytes += accelWideBytes(n, scenes[s].bvhNodes != nullptr) + align(48ull * n) + align(4ull * n);
     }
     if (ctx->batchBytes < bytes) {
         bool capturing = false;
@@ -1148,7 +1148,7 @@ int prepareBatchScenes(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t numSc
     std::vector<float4*> wns(numScenes), ats(numScenes);
     std::vector<uint32_t*> fls(numScenes);
     for (uint32_t s = 0; s < numScenes; ++s)
-        wns[s] = c.take<float4>(accelByteBytes(scenes[s].numFaces, scenes[s].bvhNodes != nullptr) / sizeof(float4));
+        wns[s] = c.take<float4>(accelWideBytes(scenes[s].numFaces, scenes[s].bvhNodes != nullptr) / sizeof(float4));
     for (uint32_t s = 0; s < numScenes; ++s) ats[s] = c.take<float4>(3ull * scenes[s].numFaces);
     for (uint32_t s = 0; s < numScenes; ++s) fls[s] = c.take<uint32_t>(scenes[s].numFaces);
     for (uint32_t s = 0; s < numScenes; ++s) {
@@ -1157,14 +1157,14 @@ int prepareBatchScenes(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t numSc
         float4 *wn = wns[s], *at = ats[s];
         uint32_t* fl = fls[s];
         launchAccelBuild(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, sd.vertices, sd.faces, nullptr, at, stream);
-        launchAccelBytes(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, wn, stream);
+        launchAccelWide(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, wn, stream);
         launchFaceLights(sd.lights, sd.numLights, n, fl, envWords + s, stream);
         RScene& S = table[s];
         std::memset(&S, 0, sizeof(S));
         S.g = GeomScene{sd.internalNodes, sd.leafNodes, n, sd.vertices, sd.faces};
         S.g.bvh = reinterpret_cast<const float4*>(sd.bvhNodes);
         S.g.atris = at;
-        S.g.qnodes = wn;
+        S.g.wnodes = wn;
         S.normals = sd.normals;
         S.tangents = sd.tangents;
         S.uvs = sd.uvs;

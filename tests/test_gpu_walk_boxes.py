@@ -1,0 +1,90 @@
+"""Walks without per-ray counts against the walks whose box decisions are
+defined (the oracle's ordered traversal and the same calls with counts), where
+those decisions are close: boxes and rays that meet near the coordinate
+planes, far from their record's corner."""
+import numpy as np
+import pytest
+
+import clear_amd as ca
+import oracle as orc
+from test_gpu_trace_nocounts import cuda, results, same
+
+pytestmark = pytest.mark.gpu
+
+
+def aimed(p, d, dist):
+    """Rays of directions d that reach the points p after `dist`."""
+    d = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.empty((7, len(p)), np.float32)
+    rays[0:3], rays[3:6], rays[6] = (p - d * dist[:, None]).T, d.T, np.inf
+    return rays
+
+
+def traced(ctx, v, f, rays, walk):
+    """Hits of one of the walks without counts, on the device."""
+    import torch
+
+    n, R = len(f), rays.shape[1]
+    hit, t = results(R)
+    tv, tf, tr = cuda(v), cuda(f), cuda(rays)
+    if walk == "midpoint":
+        ca.trace_closest_bvh(ctx, cuda(ca.build_midpoint_bvh(v, f)), n, tv, tf, tr, R, hit, t, ordered=True)
+    else:
+        inodes, leaves = ca.node_buffers(n)
+        ca.LBVHBuilder(ctx, n).perform(tv, tf, n, 10, inodes, leaves)
+        ca.trace_closest(ctx, inodes, leaves, n, tv, tf, tr, R, hit, t, ordered=walk == "ordered", wide=walk == "wide")
+    torch.cuda.synchronize()
+    assert ctx.device_status() == 0
+    return hit, t
+
+
+@pytest.mark.parametrize("walk", ["ordered", "wide", "midpoint"])
+@pytest.mark.parametrize("extent", [1, 10, 100, 1000])
+def test_flat_boxes_far_from_their_records_corner(gpu_ctx, extent, walk):
+    """A triangle in the plane x = 0 with corners on the axes, beside one whose
+    box starts at -extent: rays from 1e-7 to 1 before the plane, and rays aimed
+    at an edge."""
+    e, R = float(extent), 20000
+    soup = np.array([[-e, -e, -e, 1 - e, 1 - e, -e, -e, 1 - e, 1 - e], [0, 0, 0, 0, 1, 0, 0, 0, 1]], np.float32)
+    rng = np.random.default_rng(extent)
+    b = rng.random((R, 2))
+    b = np.where(b.sum(1, keepdims=True) > 1, 1 - b, b)
+    b[R // 2:, 0] *= 1e-3
+    dist = np.where(np.arange(R) < R // 2, 10.0 ** rng.uniform(-7, 0, R), rng.uniform(0.05, 0.5, R))
+    rays = aimed(np.c_[np.zeros(R), b], rng.normal(size=(R, 3)), dist)
+    if extent == 100:
+        rays[:6, 0] = [0.152555928, 0.0348040573, 0.32536763, -0.888217509, -0.202636451, -0.412320524]
+    v, f = ca.soup_to_mesh(soup)
+    o = orc.lbvh_build(v, f, 10)
+    h, bt, _ = orc.trace_wide(o["inodes"], o["leaves"], 2, v, f, rays)
+    assert (h == 1).mean() > 0.99
+    print(f"[walk boxes] flat box, extent {extent}, {walk}", flush=True)
+    same(*traced(gpu_ctx, v, f, rays, walk), h, bt)
+
+
+@pytest.mark.parametrize("walk", ["ordered", "wide", "midpoint"])
+def test_grid_geometry_around_the_origin(gpu_ctx, walk):
+    """Unit squares in the planes x, y, z = 0 of a scene of extent 64 with
+    coinciding copies (ties in t), and rays that start near those planes."""
+    rng = np.random.default_rng(3)
+    k = rng.integers(-64, 64, size=(1500, 2)).astype(np.float32)
+    quads = []
+    for axis in range(3):
+        c = np.zeros((500, 4, 3), np.float32)
+        c[:, :, (axis + 1) % 3] = k[500 * axis:500 * axis + 500, :1] + np.array([0, 1, 1, 0], np.float32)
+        c[:, :, (axis + 2) % 3] = k[500 * axis:500 * axis + 500, 1:] + np.array([0, 0, 1, 1], np.float32)
+        quads.append(c)
+    q = np.concatenate(quads)
+    soup = np.concatenate([q[:, [0, 1, 2]].reshape(-1, 9), q[:, [0, 2, 3]].reshape(-1, 9)])
+    soup = np.concatenate([soup, soup[::3]])
+    R = 20000
+    pick = rng.integers(0, len(q), R)
+    w = rng.random((R, 2, 1)) * np.where(rng.random((R, 1, 1)) < 0.3, 1e-3, 1.0)
+    p = q[pick, 0] + w[:, 0] * (q[pick, 1] - q[pick, 0]) + w[:, 1] * (q[pick, 3] - q[pick, 0])
+    rays = aimed(p, rng.normal(size=(R, 3)), 10.0 ** rng.uniform(-7, 1, R))
+    v, f = ca.soup_to_mesh(soup)
+    o = orc.lbvh_build(v, f, 10)
+    h, bt, _ = orc.trace_wide(o["inodes"], o["leaves"], len(f), v, f, rays)
+    assert (h != 0xFFFFFFFF).mean() > 0.8
+    print(f"[walk boxes] grid, {walk}", flush=True)
+    same(*traced(gpu_ctx, v, f, rays, walk), h, bt)
