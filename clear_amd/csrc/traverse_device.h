@@ -916,9 +916,10 @@ private:
 //   * leaf entries are tested in a loop over each lane's own leaves, so the
 //     triangle test runs as often as the lane with the most leaves has, not
 //     once for each of the four slots in which some lane has one;
-//   * internal entries are sorted as one word each (entry distance with its
-//     two lowest bits replaced by the slot: rounded down, so a pop never
-//     drops a candidate it should not).
+//   * internal entries are sorted by entry distance, references along with
+//     them. (One word an entry, its two lowest bits replaced by the slot, saves
+//     instructions but is no distance: above zero for a ray that starts inside a
+//     box, so that a hit at t = 0 dropped boxes with an equal one.)
 // begin() with `any` stops at the first accepted triangle of finite distance;
 // with a bound (tmax, bestFace) it accepts only triangles before it in (t,
 // face) order, so an any walk bounded by a light's own hit answers whether
@@ -1009,11 +1010,11 @@ struct WideWalk {
         auto entry = [&](uint32_t slot, V3 lo, V3 hi, uint32_t ref) {
             const float tn = fmaxf(fmaxf((lo.x - o.x) * inv.x, (lo.y - o.y) * inv.y), fmaxf((lo.z - o.z) * inv.z, 0.0f));
             const float tf = fminf(fminf((hi.x - o.x) * inv.x, (hi.y - o.y) * inv.y), (hi.z - o.z) * inv.z) * kPadUp;
-            const float e = tn * kPadDown;
+            const float e = fabsf(tn) * kPadDown;  // no -0: entries are sorted by their bits
             const bool pass = e <= fminf(tf, t);
             const uint32_t isLeaf = (uint32_t)((int32_t)ref >> 31);  // all ones; empty slots too, skipped below
             leaves |= (pass ? 1u << slot : 0u) & isLeaf;
-            return (pass ? ((__float_as_uint(e) & ~3u) | slot) : 0xFFFFFFFFu) | isLeaf;
+            return (pass ? __float_as_uint(e) : 0xFFFFFFFFu) | isLeaf;
         };
         uint32_t k0 = entry(0u, {ax.x, ay.x, az.x}, {bx.x, by.x, bz.x}, r.x);
         uint32_t k1 = entry(1u, {ax.y, ay.y, az.y}, {bx.y, by.y, bz.y}, r.y);
@@ -1025,16 +1026,20 @@ struct WideWalk {
             const uint32_t ref = pick(r, slot);
             if (ref != kNone) leaf(ref & ~kLeafRef);
         }
-        auto cx = [](uint32_t& a, uint32_t& b) {
-            const uint32_t lo = min(a, b);
-            b = max(a, b);
-            a = lo;
+        uint32_t r0 = r.x, r1 = r.y, r2 = r.z, r3 = r.w;
+        auto cx = [](uint32_t& ka, uint32_t& ra, uint32_t& kb, uint32_t& rb) {
+            const bool swap = kb < ka;
+            const uint32_t k = swap ? kb : ka, q = swap ? rb : ra;
+            kb = swap ? ka : kb;
+            rb = swap ? ra : rb;
+            ka = k;
+            ra = q;
         };
-        cx(k0, k1);
-        cx(k2, k3);
-        cx(k0, k2);
-        cx(k1, k3);
-        cx(k1, k2);
+        cx(k0, r0, k1, r1);
+        cx(k2, r2, k3, r3);
+        cx(k0, r0, k2, r2);
+        cx(k1, r1, k3, r3);
+        cx(k1, r1, k2, r2);
         // Push all but the nearest, farthest first. Entries beyond a hit of
         // this visit's own leaves stay (their pop drops them); 0xFFFFFFFF is a
         // NaN and fails every compare.
@@ -1043,21 +1048,21 @@ struct WideWalk {
         // branches: what is not pushed goes to the free slot above the top.
         const bool deep = __ballot(depth + 3 > Stack::kInLds) != 0;
         if (!deep) {
-            auto put = [&](uint32_t k, int j) {
+            auto put = [&](uint32_t k, uint32_t ref, int j) {
                 const int at = depth + more - (k != 0xFFFFFFFFu ? j + 1 : 0);
-                stack.lds[at * stack.stride] = make_uint2(pick(r, k & 3u), k);
+                stack.lds[at * stack.stride] = make_uint2(ref, k);
             };
-            if (__ballot(k3 != 0xFFFFFFFFu)) put(k3, 2);
-            if (__ballot(k2 != 0xFFFFFFFFu)) put(k2, 1);
-            put(k1, 0);
+            if (__ballot(k3 != 0xFFFFFFFFu)) put(k3, r3, 2);
+            if (__ballot(k2 != 0xFFFFFFFFu)) put(k2, r2, 1);
+            put(k1, r1, 0);
             depth += more;
         } else {
-            if (k3 != 0xFFFFFFFFu) push(pick(r, k3 & 3u), __uint_as_float(k3));
-            if (k2 != 0xFFFFFFFFu) push(pick(r, k2 & 3u), __uint_as_float(k2));
-            if (k1 != 0xFFFFFFFFu) push(pick(r, k1 & 3u), __uint_as_float(k1));
+            if (k3 != 0xFFFFFFFFu) push(r3, __uint_as_float(k3));
+            if (k2 != 0xFFFFFFFFu) push(r2, __uint_as_float(k2));
+            if (k1 != 0xFFFFFFFFu) push(r1, __uint_as_float(k1));
         }
         const bool go = __uint_as_float(k0) <= t;
-        node = go ? pick(r, k0 & 3u) : kNone;
+        node = go ? r0 : kNone;
         if (!go) {
             while (depth > 0) {
                 const uint2 e = stack.get(--depth);

@@ -88,3 +88,29 @@ def test_grid_geometry_around_the_origin(gpu_ctx, walk):
     assert (h != 0xFFFFFFFF).mean() > 0.8
     print(f"[walk boxes] grid, {walk}", flush=True)
     same(*traced(gpu_ctx, v, f, rays, walk), h, bt)
+
+
+@pytest.mark.parametrize("walk", ["ordered", "wide", "midpoint"])
+@pytest.mark.parametrize("bound", [np.inf, 0.0])
+def test_hits_at_distance_zero(gpu_ctx, bound, walk):
+    """Rays that start on the vertices, edges and faces of a bent sheet: all the
+    triangles there are hit at t = 0 and the smallest face index wins, so no
+    box with entry 0 may be dropped, also for a ray that ends at 0."""
+    m = 24
+    x, y = np.meshgrid(np.arange(m + 1), np.arange(m + 1), indexing="ij")
+    p = np.stack([x, y, (x * y) % 3], -1).astype(np.float32)
+    a, b, c, d = p[:-1, :-1], p[1:, :-1], p[1:, 1:], p[:-1, 1:]
+    tri = np.concatenate([np.stack([a, b, c], 2).reshape(-1, 3, 3), np.stack([a, c, d], 2).reshape(-1, 3, 3)])
+    rng = np.random.default_rng(8)
+    tri = tri[rng.permutation(len(tri))]
+    R = 9000
+    at, u = rng.integers(0, len(tri), R), np.zeros((R, 3))
+    k = np.arange(R) % 3  # a vertex, the middle of an edge, a quarter point of a face
+    u[k == 0], u[k == 1], u[k == 2] = [1, 0, 0], [0.5, 0.5, 0], [0.25, 0.5, 0.25]
+    rays = aimed((tri[at] * u[:, :, None]).sum(1), rng.normal(size=(R, 3)), np.zeros(R))
+    rays[6] = bound
+    v, f = ca.soup_to_mesh(tri.reshape(-1, 9))
+    h, bt = orc.trace_bruteforce_minid(v, f, rays)
+    assert (bt[h != 0xFFFFFFFF] == 0).mean() > 0.5
+    print(f"[walk boxes] distance zero, bound {bound}, {walk}", flush=True)
+    same(*traced(gpu_ctx, v, f, rays, walk), h, bt)
