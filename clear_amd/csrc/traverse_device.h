@@ -913,9 +913,12 @@ private:
 //     and comparisons are slabEnter's, in its order, so a box is admitted exactly
 //     when slabEnter admits it (min and max pick the same planes, since rounding
 //     keeps (lo - o) * inv and (hi - o) * inv in order);
-//   * leaf entries are tested in a loop over each lane's own leaves, so the
-//     triangle test runs as often as the lane with the most leaves has, not
-//     once for each of the four slots in which some lane has one;
+//   * leaf entries are tested nearest first, while they are within t, in a loop
+//     over each lane's own leaves, so the triangle test runs as often as the lane
+//     with the most such leaves has, not once for each of the four slots in which
+//     some lane has one. (A triangle with vertices that are not finite can be
+//     accepted at t = NaN: nothing is within that, so the walk ends there, as the
+//     counting walks do.)
 //   * internal entries are sorted by entry distance, references along with
 //     them. (One word an entry, its two lowest bits replaced by the slot, saves
 //     instructions but is no distance: above zero for a ray that starts inside a
@@ -936,7 +939,8 @@ template <class Alpha, class Stack>
 struct WideWalk {
     const float4* wn;
     const float4* tris;
-    uint32_t limit;  // more visits than this mean malformed records
+    const float4* root;  // the root's box
+    uint32_t limit;      // more visits than this mean malformed records
     const Stack& stack;
     Alpha alpha;
     V3 o, d, inv;
@@ -947,12 +951,19 @@ struct WideWalk {
     static constexpr uint32_t kAny = 1u, kOver = 2u;
 
     __device__ __forceinline__ WideWalk(const GeomScene& g, const Stack& s_, const Alpha& a_)
-        : wn(asGlobal(g.wnodes)), tris(asGlobal(g.atris)), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
+        : wn(asGlobal(g.wnodes)), tris(asGlobal(g.atris)), root(rootBox(g)), limit(2u * g.n + 2u), stack(s_), alpha(a_), node(kNone), mode(0u) {}
     __device__ __forceinline__ void rebind(const GeomScene& g, const Alpha& a_) {
         wn = asGlobal(g.wnodes);
         tris = asGlobal(g.atris);
+        root = rootBox(g);
         limit = 2u * g.n + 2u;
         alpha = a_;
+    }
+    // Every node record starts with its box.
+    static __device__ __forceinline__ const float4* rootBox(const GeomScene& g) {
+        return asGlobal(g.bvh ? g.bvh
+                              : g.n == 1 ? reinterpret_cast<const float4*>(g.leaves)
+                                         : reinterpret_cast<const float4*>(g.inodes));
     }
     __device__ __forceinline__ bool done() const { return node == kNone; }
     __device__ __forceinline__ bool over() const { return (mode & kOver) != 0; }
@@ -964,7 +975,7 @@ struct WideWalk {
         t = tmax;
         b1 = b2 = 0.0f;
         best = bound = bestFace;
-        node = tmax >= 0.0f ? 0u : kNone;  // no t >= 0 lies before a negative or NaN bound
+        node = slabEnter(root[0], root[1], o, inv, t) <= t ? 0u : kNone;
         left = limit;
         depth = 0;
         mode = anyHit ? kAny : 0u;
@@ -995,37 +1006,43 @@ struct WideWalk {
         b2 = v;
     }
 
-    static __device__ __forceinline__ uint32_t pick(const uint4& r, uint32_t slot) {
-        const uint32_t lo = (slot & 1u) ? r.y : r.x, hi = (slot & 1u) ? r.w : r.z;
-        return (slot & 2u) ? hi : lo;
-    }
-
     // Visits `node`.
     __device__ __forceinline__ void step() {
         const float4* wp = wn + 8 * (size_t)node;
         const int nx = inv.x < 0.0f ? 3 : 0, ny = inv.y < 0.0f ? 4 : 1, nz = inv.z < 0.0f ? 5 : 2;
         const float4 ax = wp[nx], ay = wp[ny], az = wp[nz], bx = wp[3 - nx], by = wp[5 - ny], bz = wp[7 - nz];
         const uint4 r = reinterpret_cast<const uint4*>(wp)[6];
-        uint32_t leaves = 0;
-        auto entry = [&](uint32_t slot, V3 lo, V3 hi, uint32_t ref) {
+        auto entry = [&](V3 lo, V3 hi) {
             const float tn = fmaxf(fmaxf((lo.x - o.x) * inv.x, (lo.y - o.y) * inv.y), fmaxf((lo.z - o.z) * inv.z, 0.0f));
             const float tf = fminf(fminf((hi.x - o.x) * inv.x, (hi.y - o.y) * inv.y), (hi.z - o.z) * inv.z) * kPadUp;
             const float e = fabsf(tn) * kPadDown;  // no -0: entries are sorted by their bits
-            const bool pass = e <= fminf(tf, t);
-            const uint32_t isLeaf = (uint32_t)((int32_t)ref >> 31);  // all ones; empty slots too, skipped below
-            leaves |= (pass ? 1u << slot : 0u) & isLeaf;
-            return (pass ? __float_as_uint(e) : 0xFFFFFFFFu) | isLeaf;
+            return e <= fminf(tf, t) ? __float_as_uint(e) : 0xFFFFFFFFu;
         };
-        uint32_t k0 = entry(0u, {ax.x, ay.x, az.x}, {bx.x, by.x, bz.x}, r.x);
-        uint32_t k1 = entry(1u, {ax.y, ay.y, az.y}, {bx.y, by.y, bz.y}, r.y);
-        uint32_t k2 = entry(2u, {ax.z, ay.z, az.z}, {bx.z, by.z, bz.z}, r.z);
-        uint32_t k3 = entry(3u, {ax.w, ay.w, az.w}, {bx.w, by.w, bz.w}, r.w);
-        while (leaves) {
-            const uint32_t slot = (uint32_t)__builtin_ctz(leaves);
-            leaves &= leaves - 1u;
-            const uint32_t ref = pick(r, slot);
+        const uint32_t e0 = entry({ax.x, ay.x, az.x}, {bx.x, by.x, bz.x});
+        const uint32_t e1 = entry({ax.y, ay.y, az.y}, {bx.y, by.y, bz.y});
+        const uint32_t e2 = entry({ax.z, ay.z, az.z}, {bx.z, by.z, bz.z});
+        const uint32_t e3 = entry({ax.w, ay.w, az.w}, {bx.w, by.w, bz.w});
+        auto mask = [](uint32_t ref) { return (uint32_t)((int32_t)ref >> 31); };  // all ones: a leaf or an empty slot
+        uint32_t l0 = e0 | ~mask(r.x), l1 = e1 | ~mask(r.y), l2 = e2 | ~mask(r.z), l3 = e3 | ~mask(r.w);
+        while (true) {
+            const uint32_t m = min(min(l0, l1), min(l2, l3));
+            if (!(__uint_as_float(m) <= t)) break;
+            uint32_t ref = r.w;
+            if (l0 == m) {
+                ref = r.x;
+                l0 = 0xFFFFFFFFu;
+            } else if (l1 == m) {
+                ref = r.y;
+                l1 = 0xFFFFFFFFu;
+            } else if (l2 == m) {
+                ref = r.z;
+                l2 = 0xFFFFFFFFu;
+            } else {
+                l3 = 0xFFFFFFFFu;
+            }
             if (ref != kNone) leaf(ref & ~kLeafRef);
         }
+        uint32_t k0 = e0 | mask(r.x), k1 = e1 | mask(r.y), k2 = e2 | mask(r.z), k3 = e3 | mask(r.w);
         uint32_t r0 = r.x, r1 = r.y, r2 = r.z, r3 = r.w;
         auto cx = [](uint32_t& ka, uint32_t& ra, uint32_t& kb, uint32_t& rb) {
             const bool swap = kb < ka;
@@ -1072,9 +1089,9 @@ struct WideWalk {
                 }
             }
         }
-        // An any walk ends at its first hit of finite distance, every walk at
-        // a NaN distance (nothing compares with it) or with its visits used up.
-        const bool stop = ((mode & kAny) && best != bound && !isinf(t)) || t != t;
+        // An any walk ends at its first hit of finite distance, every walk with
+        // its visits used up.
+        const bool stop = (mode & kAny) && best != bound && !isinf(t);
         if (--left == 0u) {
             mode |= kOver;
             node = kNone;

@@ -114,3 +114,34 @@ def test_hits_at_distance_zero(gpu_ctx, bound, walk):
     assert (bt[h != 0xFFFFFFFF] == 0).mean() > 0.5
     print(f"[walk boxes] distance zero, bound {bound}, {walk}", flush=True)
     same(*traced(gpu_ctx, v, f, rays, walk), h, bt)
+
+
+@pytest.mark.parametrize("walk", ["ordered", "wide"])
+@pytest.mark.parametrize("n", [1, 2, 5, 600, 5000])
+def test_vertices_that_are_not_finite(gpu_ctx, n, walk):
+    """Triangles with vertices that are not finite can be accepted at t = NaN,
+    after which nothing else is: hits and distances are those of the 4-wide walk
+    with counts, which tests the leaves of a visit nearest first."""
+    import torch
+
+    soup = ca.gen_cluster_soup(n, seed=n + 3, num_clusters=4, sigma=0.1, e_min=0.05, e_max=0.2)
+    rng = np.random.default_rng(n)
+    bad = rng.random((n, 9)) < 0.02
+    bad[0, 4] = n < 600
+    soup[bad] = rng.choice(np.array([np.nan, np.inf, -np.inf], np.float32), bad.sum())
+    v, f = ca.soup_to_mesh(soup)
+    rays = ca.gen_random_rays(4099, seed=n)
+    R = rays.shape[1]
+    tv, tf, tr = cuda(v), cuda(f), cuda(rays)
+    inodes, leaves = ca.node_buffers(n)
+    ca.LBVHBuilder(gpu_ctx, n).perform(tv, tf, n, 10, inodes, leaves)
+    print(f"[walk boxes] vertices not finite, n={n}, {walk}", flush=True)
+    a, b = results(R), results(R)
+    counts = torch.empty(2 * R, dtype=torch.int32, device="cuda")
+    ca.trace_closest(gpu_ctx, inodes, leaves, n, tv, tf, tr, R, *a, counts, wide=True)
+    ca.trace_closest(gpu_ctx, inodes, leaves, n, tv, tf, tr, R, *b, ordered=walk == "ordered", wide=walk == "wide")
+    torch.cuda.synchronize()
+    at, bt = a[1].cpu().numpy(), b[1].cpu().numpy()
+    assert n <= 2 or np.isnan(at).any()
+    np.testing.assert_array_equal(b[0].cpu().numpy(), a[0].cpu().numpy())
+    np.testing.assert_array_equal(bt, at)
