@@ -372,12 +372,15 @@ __global__ __launch_bounds__(kOrdBlock) void k_trace_counts(
 }
 
 // Without counts: WideWalk, whatever ordered walk the caller asked for (the
-// hit is the same).
+// hit is the same). A level of the binary walk's tree leaves it one entry, a
+// record (two levels) leaves up to three here: kTracePairs entries suffice for
+// every tree of 64 levels, the depth at which the binary walk's 64 always do.
+constexpr int kTracePairs = 96;
 __global__ __launch_bounds__(kOrdBlock) void k_trace_wide(
     dev::GeomScene g, const float* __restrict__ rays, uint32_t numRays, uint32_t* __restrict__ hitFace,
     float* __restrict__ hitT, uint32_t* __restrict__ status, uint32_t* __restrict__ spill) {
     constexpr int kPairs = kOrdHalf / 2;
-    using S = dev::PairStack<kPairs, dev::kStackPairs / 2>;
+    using S = dev::PairStack<kPairs, kTracePairs>;
     __shared__ uint2 s_stack[2 * kPairs * kOrdBlock];
     const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
     const uint32_t lanes = gridDim.x * kOrdBlock;
@@ -472,7 +475,10 @@ int traceGrid(clr_ctx* ctx, uint32_t numRays, uint32_t& grid) {
     if (rc) return rc;
     grid = std::max(1u, std::min((uint32_t)cus * 8u, (numRays + kOrdBlock - 1) / kOrdBlock));
     const size_t lanes = (size_t)grid * kOrdBlock;
-    return ensureTraceSpill(ctx, lanes * 2 * (dev::kStackPairs - kOrdHalf) * sizeof(uint32_t));
+    // Of the kernels without and with counts the former takes more; both find
+    // room after either.
+    static_assert(2 * kTracePairs >= dev::kStackPairs, "spill covers the counting walks");
+    return ensureTraceSpill(ctx, lanes * 2 * (2 * kTracePairs - kOrdHalf) * sizeof(uint32_t));
 }
 }  // namespace
 

@@ -1057,28 +1057,29 @@ struct WideWalk {
         cx(k0, r0, k2, r2);
         cx(k1, r1, k3, r3);
         cx(k1, r1, k2, r2);
-        // Push all but the nearest, farthest first. Entries beyond a hit of
-        // this visit's own leaves stay (their pop drops them); 0xFFFFFFFF is a
+        // Push all but the nearest that are still within t (this visit's own
+        // leaves may have brought it closer), farthest first. 0xFFFFFFFF is a
         // NaN and fails every compare.
-        const int more = (int)(k1 != 0xFFFFFFFFu) + (int)(k2 != 0xFFFFFFFFu) + (int)(k3 != 0xFFFFFFFFu);
+        const bool go = __uint_as_float(k0) <= t;
+        const bool p1 = __uint_as_float(k1) <= t, p2 = __uint_as_float(k2) <= t, p3 = __uint_as_float(k3) <= t;
         // Unless some lane's stack nears its global part, three stores without
         // branches: what is not pushed goes to the free slot above the top.
         const bool deep = __ballot(depth + 3 > Stack::kInLds) != 0;
         if (!deep) {
-            auto put = [&](uint32_t k, uint32_t ref, int j) {
-                const int at = depth + more - (k != 0xFFFFFFFFu ? j + 1 : 0);
+            const int more = (int)p1 + (int)p2 + (int)p3;
+            auto put = [&](bool push, uint32_t k, uint32_t ref, int j) {
+                const int at = depth + more - (push ? j + 1 : 0);
                 stack.lds[at * stack.stride] = make_uint2(ref, k);
             };
-            if (__ballot(k3 != 0xFFFFFFFFu)) put(k3, r3, 2);
-            if (__ballot(k2 != 0xFFFFFFFFu)) put(k2, r2, 1);
-            put(k1, r1, 0);
+            if (__ballot(p3)) put(p3, k3, r3, 2);
+            if (__ballot(p2)) put(p2, k2, r2, 1);
+            put(p1, k1, r1, 0);
             depth += more;
         } else {
-            if (k3 != 0xFFFFFFFFu) push(r3, __uint_as_float(k3));
-            if (k2 != 0xFFFFFFFFu) push(r2, __uint_as_float(k2));
-            if (k1 != 0xFFFFFFFFu) push(r1, __uint_as_float(k1));
+            if (p3) push(r3, __uint_as_float(k3));
+            if (p2) push(r2, __uint_as_float(k2));
+            if (p1) push(r1, __uint_as_float(k1));
         }
-        const bool go = __uint_as_float(k0) <= t;
         node = go ? r0 : kNone;
         if (!go) {
             while (depth > 0) {

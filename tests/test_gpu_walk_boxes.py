@@ -145,3 +145,50 @@ def test_vertices_that_are_not_finite(gpu_ctx, n, walk):
     assert n <= 2 or np.isnan(at).any()
     np.testing.assert_array_equal(b[0].cpu().numpy(), a[0].cpu().numpy())
     np.testing.assert_array_equal(bt, at)
+
+
+def chain(levels):
+    """A chain of nodes, each with the next link as one child and a node over
+    two pairs of leaves as the other: one entry a level for the binary walk,
+    three every other level for the 4-wide one. All boxes overlap."""
+    n = 4 * levels + 1
+    soup = np.random.default_rng(levels).random((n, 9)).astype(np.float32)
+    tri = soup.reshape(n, 3, 3)
+    lo, hi = tri.min(1), tri.max(1)
+    leaves, inodes = np.zeros((n, 12), np.uint32), np.zeros((n - 1, 12), np.uint32)
+
+    def record(rec, a, b, words):
+        rec[0:3], rec[4:7] = lo[a:b].min(0).view(np.uint32), hi[a:b].max(0).view(np.uint32)
+        rec[8:8 + len(words)] = words
+
+    for k in range(n):
+        record(leaves[k], k, k + 1, [k])
+    for k in range(levels):  # link k is node k; its tooth is node levels + 3 k over the next two
+        tooth, last = levels + 3 * k, k + 1 == levels
+        record(inodes[k], 4 * k, n, [0x100 if last else 0, tooth, n - 1 if last else k + 1])
+        record(inodes[tooth], 4 * k, 4 * k + 4, [0, tooth + 1, tooth + 2])
+        for m in range(2):
+            record(inodes[tooth + 1 + m], 4 * k + 2 * m, 4 * k + 2 * m + 2, [0x101, 4 * k + 2 * m, 4 * k + 2 * m + 1])
+    return soup, inodes, leaves
+
+
+@pytest.mark.parametrize("levels", [20, 45, 62])
+def test_deep_trees_within_the_binary_walks_stack(gpu_ctx, levels):
+    import torch
+
+    soup, inodes, leaves = chain(levels)
+    v, f = ca.soup_to_mesh(soup)
+    n, R = len(f), 4096
+    rng = np.random.default_rng(6)
+    rays = np.empty((7, R), np.float32)
+    rays[0:3], rays[3:6], rays[6] = rng.random((3, R)), rng.normal(size=(3, R)), np.inf
+    h, bt = orc.trace_bruteforce_minid(v, f, rays)
+    tv, tf, tr, ti, tl = (cuda(a) for a in (v, f, rays, inodes, leaves))
+    counts = torch.empty(2 * R, dtype=torch.int32, device="cuda")
+    print(f"[walk boxes] chain of {levels} levels", flush=True)
+    for walk in ({"ordered": True, "stats": counts}, {"ordered": True}):
+        hit, t = results(R)
+        ca.trace_closest(gpu_ctx, ti, tl, n, tv, tf, tr, R, hit, t, **walk)
+        torch.cuda.synchronize()
+        assert gpu_ctx.device_status() == 0
+        same(hit, t, h, bt)
