@@ -222,7 +222,7 @@ __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint3
     while (true) {
         bool ray = false, newSample = false, anyRay = false;
         V3 org = v3z(), dir = v3z();
-        float bound = INFINITY;
+        float bound = INFINITY;  // of the next ray: a shadow ray's light, set only where one is cast
         uint32_t boundFace = kNone;
         if (live) {
             over |= w.over();
@@ -314,11 +314,14 @@ __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint3
                                 target = atInf ? kNone : lp.face;
                                 shadow = !job.unseen(contrib);
                                 if (shadow && !atInf) {
-                                    float x1, x2;
+                                    float tl = INFINITY, x1, x2;
                                     uint32_t flag;
-                                    shadow = triTestPacked(S.g.atris, org, dir, lp.face, bound, x1, x2, flag) &&
-                                             !isinf(bound) && !(flag && RareAlpha{&S}.reject(lp.face, x1, x2));
-                                    boundFace = lp.face;
+                                    shadow = triTestPacked(S.g.atris, org, dir, lp.face, tl, x1, x2, flag) &&
+                                             !isinf(tl) && !(flag && RareAlpha{&S}.reject(lp.face, x1, x2));
+                                    if (shadow) {
+                                        bound = tl;
+                                        boundFace = lp.face;
+                                    }
                                 }
                                 if (shadow)
                                     job.lightSample(atInf ? 0xFFFFFFFFu : (uint32_t)S.g.faces[lp.face].lightPtr, F.matPtr,
@@ -344,8 +347,6 @@ __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint3
                     } else {
                         org = nextOrg;
                         dir = nextDir;
-                        bound = INFINITY;
-                        boundFace = kNone;
                         ray = true;
                     }
                 }

@@ -54,3 +54,21 @@ def test_direct_lighting_closed_form(gpu_ctx, detail):
     assert ratio == pytest.approx(1.0, abs=3e-3)
     assert close[mask].mean() >= 0.99
     assert (img[mask & dark] == 0.0).all()
+
+
+@pytest.mark.parametrize("mode", [ca.RENDER_MEGAKERNEL, ca.RENDER_WAVEFRONT])
+def test_emitter_with_an_alpha_texture(gpu_ctx, mode):
+    """The showcase scene with its alpha grid on the ceiling light too: light
+    samples in the cut-out parts are not cast, and end many paths whose BSDF
+    sample is zero; the next sample's camera ray must not inherit their bound."""
+    host = ca.HostScene(ca.SCENE_SHOWCASE, 64, 64)
+    light = host.faces["lightPtr"] != 0xFFFF
+    cut = np.flatnonzero(host.faces["alphaTexPtr"] != 0xFFFFFFFF)
+    assert light.sum() == 2 and len(cut) == 2
+    host.faces["uv"][light] = host.faces["uv"][cut]
+    host.faces["alphaTexPtr"][light] = host.faces["alphaTexPtr"][cut[0]]
+    print(f"[alpha emitter] mode={mode}", flush=True)
+    g = gpu_render(gpu_ctx, host, 16, 5, mode=mode)
+    compare(f"alpha emitter mode={mode}", host, 16, 5, g, oracle_render(host, 16, 5))
+    other = ca.RENDER_WAVEFRONT if mode == ca.RENDER_MEGAKERNEL else ca.RENDER_MEGAKERNEL
+    np.testing.assert_array_equal(g[0], gpu_render(gpu_ctx, host, 16, 5, mode=other)[0])
