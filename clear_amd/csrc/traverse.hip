@@ -81,7 +81,10 @@ __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const c
         for (int k = 0; k < 2; ++k) {
             const bool leaf = ((c.x >> (8 * k)) & 0xFFu) != 0;
             const uint32_t ci = k ? c.z : c.y;
-            if (leaf ? ci >= n : ci + 1 >= n) {  // malformed nodes: an empty box and no child
+            // Malformed nodes: an empty box, which the walks may still enter
+            // (slabEnter admits it), and as its reference a leaf of a face that
+            // is not there, which they flag.
+            if (leaf ? ci >= n : ci >= n - 1) {
                 box[k][0] = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
                 box[k][1] = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
                 ref[k] = dev::kNone;
@@ -150,7 +153,8 @@ struct WideSlots {
             ref[c] = dev::kNone;
         }
     }
-    __device__ __forceinline__ void put(int c, float4 l, float4 h, uint32_t r) {
+    __device__ __forceinline__ void put(int c, float4 l, float4 h, uint32_t r, uint32_t n) {
+        if ((r & dev::kLeafRef) && (r & ~dev::kLeafRef) >= n) return;  // a face that is not there
         lo[0][c] = l.x;
         lo[1][c] = l.y;
         lo[2][c] = l.z;
@@ -177,7 +181,7 @@ __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const cl
     w.clear();
     if (n == 1 && i == 0) {  // a tree of one leaf: a record that holds it
         const float4* p = reinterpret_cast<const float4*>(leaves);
-        w.put(0, p[0], p[1], leaves[0].objIdx | dev::kLeafRef);
+        w.put(0, p[0], p[1], leaves[0].objIdx | dev::kLeafRef, n);
         w.store(records);
         return;
     }
@@ -190,19 +194,19 @@ __global__ void k_accel_wide(const clr_lbvh_inode* __restrict__ inodes, const cl
         if (leaf) {
             if (ci >= n) continue;  // malformed nodes leave the slot empty
             const float4* p = reinterpret_cast<const float4*>(leaves + ci);
-            w.put(2 * k, p[0], p[1], leaves[ci].objIdx | dev::kLeafRef);
+            w.put(2 * k, p[0], p[1], leaves[ci].objIdx | dev::kLeafRef, n);
             continue;
         }
-        if (ci + 1 >= n) continue;
+        if (ci >= n - 1) continue;
         const uint4 cc = reinterpret_cast<const uint4*>(inodes + ci)[2];
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
             const bool gl = ((cc.x >> (8 * m)) & 0xFFu) != 0;
             const uint32_t gi = m ? cc.z : cc.y;
-            if (gl ? gi >= n : gi + 1 >= n) continue;
+            if (gl ? gi >= n : gi >= n - 1) continue;
             const float4* p = gl ? reinterpret_cast<const float4*>(leaves + gi)
                                  : reinterpret_cast<const float4*>(inodes + gi);
-            w.put(2 * k + m, p[0], p[1], gl ? (leaves[gi].objIdx | dev::kLeafRef) : gi);
+            w.put(2 * k + m, p[0], p[1], gl ? (leaves[gi].objIdx | dev::kLeafRef) : gi, n);
         }
     }
     w.store(records + 8 * (size_t)i);
@@ -218,7 +222,7 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
     WideSlots w;
     w.clear();
     if (n == 1 && c.y == kEmpty) {  // a tree of one leaf: a record that holds it
-        w.put(0, bvh[0], bvh[1], c.x | dev::kLeafRef);
+        w.put(0, bvh[0], bvh[1], c.x | dev::kLeafRef, n);
         w.store(records);
         return;
     }
@@ -229,16 +233,16 @@ __global__ void k_accel_wide_bvh(const float4* __restrict__ bvh, uint32_t n, flo
         const float4* p = bvh + 3 * (size_t)ci;
         const uint2 cc = *reinterpret_cast<const uint2*>(p + 2);
         if (cc.y == kEmpty) {  // a leaf: its face
-            w.put(2 * k, p[0], p[1], cc.x | dev::kLeafRef);
+            w.put(2 * k, p[0], p[1], cc.x | dev::kLeafRef, n);
             continue;
         }
-        if (cc.x >= numNodes || cc.y >= numNodes) continue;  // malformed: the binary walk flags it
+        if (cc.x >= numNodes || cc.y >= numNodes) continue;  // malformed nodes leave the slots empty
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
             const uint32_t gi = m ? cc.y : cc.x;
             const float4* q = bvh + 3 * (size_t)gi;
             const uint2 gc = *reinterpret_cast<const uint2*>(q + 2);
-            w.put(2 * k + m, q[0], q[1], gc.y == kEmpty ? (gc.x | dev::kLeafRef) : gi);
+            w.put(2 * k + m, q[0], q[1], gc.y == kEmpty ? (gc.x | dev::kLeafRef) : gi, n);
         }
     }
     w.store(records + 8 * (size_t)i);

@@ -458,6 +458,10 @@ struct Ordered {
         : g(g_), stack(s_), alpha(a_) {}
 
     __device__ __forceinline__ void leaf(uint32_t face) {
+        if (face >= g.n) {  // malformed nodes
+            overflowed = true;
+            return;
+        }
         ++st.tests;
         float tt = t, x1, x2;
         uint32_t flag;
@@ -598,6 +602,10 @@ struct Wide {
         : g(g_), stack(s_), alpha(a_) {}
 
     __device__ __forceinline__ void leaf(uint32_t face) {
+        if (face >= g.n) {  // malformed nodes
+            overflowed = true;
+            return;
+        }
         ++st.tests;
         float tt = t, x1, x2;
         uint32_t flag;

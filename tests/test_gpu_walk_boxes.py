@@ -192,3 +192,40 @@ def test_deep_trees_within_the_binary_walks_stack(gpu_ctx, levels):
         torch.cuda.synchronize()
         assert gpu_ctx.device_status() == 0
         same(hit, t, h, bt)
+
+
+@pytest.mark.parametrize("child", [0xFFFFFFFF, 0xFFFFFFF0, 299, 100000])
+def test_malformed_children_are_flagged_by_the_walks_with_counts(gpu_ctx, child):
+    """A node whose left child does not exist: the subtree is missing, the
+    binary walk flags it, and both walks return the hits of what is left."""
+    import torch
+
+    n, R = 300, 4096
+    soup = ca.gen_cluster_soup(n, seed=4, num_clusters=4, sigma=0.1, e_min=0.05, e_max=0.2)
+    v, f = ca.soup_to_mesh(soup)
+    o = orc.lbvh_build(v, f, 10)
+    nodes = np.ascontiguousarray(o["inodes"]).view(np.uint32).reshape(-1, 12).copy()
+    at = int(np.flatnonzero((nodes[:, 8] & 0xFF) == 0)[1])
+    lost, stack = set(), [int(nodes[at, 9])]
+    while stack:
+        k = stack.pop()
+        for c in range(2):
+            if (nodes[k, 8] >> (8 * c)) & 0xFF:
+                lost.add(int(np.ascontiguousarray(o["leaves"]).view(np.uint32).reshape(-1, 12)[nodes[k, 9 + c], 8]))
+            else:
+                stack.append(int(nodes[k, 9 + c]))
+    nodes[at, 9] = child
+    kept = np.array([k for k in range(n) if k not in lost])
+    assert 0 < len(kept) < n
+    rays = ca.gen_random_rays(R, seed=9)
+    h, bt = orc.trace_bruteforce_minid(v, f[kept], rays)
+    h = np.where(h == 0xFFFFFFFF, h, kept[np.minimum(h, len(kept) - 1)].astype(np.uint32))
+    tn, tl, tv, tf, tr = (cuda(a) for a in (nodes, o["leaves"], v, f, rays))
+    counts = torch.empty(2 * R, dtype=torch.int32, device="cuda")
+    for wide, status in ((False, 4), (True, 0)):
+        print(f"[walk boxes] malformed child {child:#x}, wide={wide}", flush=True)
+        hit, t = results(R)
+        ca.trace_closest(gpu_ctx, tn, tl, n, tv, tf, tr, R, hit, t, counts, ordered=not wide, wide=wide)
+        torch.cuda.synchronize()
+        assert gpu_ctx.device_status() == status
+        same(hit, t, h, bt)
