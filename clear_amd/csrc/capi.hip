@@ -91,6 +91,41 @@ int ensureTraceSpill(clr_ctx* ctx, size_t bytes) {
     return CLR_OK;
 }
 
+bool roomForOutgrown(clr_ctx* ctx) {
+    try {
+        ctx->outgrown.reserve(ctx->outgrown.size() + 1);
+    } catch (...) {
+        return false;
+    }
+    return true;
+}
+
+bool ensureClosest(clr_ctx* ctx, size_t bytes) {
+    if (ctx->closestBytes >= bytes) return true;
+    if (!roomForOutgrown(ctx)) return false;
+    // Blocks at least double, so the outgrown ones take less than the last. A
+    // caller may be capturing another stream, which forbids allocations unless
+    // the thread says that it knows.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* block = nullptr;
+    size_t got = 0;
+    for (size_t want : {std::max(bytes, 2 * ctx->closestBytes), bytes}) {
+        if (hipMalloc(&block, want) == hipSuccess) {
+            got = want;
+            break;
+        }
+        block = nullptr;
+    }
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    (void)hipGetLastError();
+    if (!block) return false;
+    if (ctx->closest) ctx->outgrown.push_back(ctx->closest);
+    ctx->closest = block;
+    ctx->closestBytes = got;
+    return true;
+}
+
 int ensureStatus(clr_ctx* ctx) {
     if (ctx->devStatus) return CLR_OK;
     hipError_t e = hipMalloc(&ctx->devStatus, 256);
@@ -143,6 +178,10 @@ int clr_create(clr_ctx** out, int device) {
                 delete ctx;
                 return CLR_ERR_HIP;
             }
+    if (hipEventCreateWithFlags(&ctx->closestDone, hipEventDisableTiming) != hipSuccess) {
+        clr_destroy(ctx);
+        return CLR_ERR_HIP;
+    }
     if (hipDeviceGetAttribute(&ctx->numCUs, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         (void)hipGetLastError();
         ctx->numCUs = 0;
@@ -172,6 +211,9 @@ int clr_destroy(clr_ctx* ctx) {
         if (ctx->wfPool) (void)hipFree(ctx->wfPool);
         if (ctx->traceSpill) (void)hipFree(ctx->traceSpill);
         if (ctx->accel) (void)hipFree(ctx->accel);
+        if (ctx->closest) (void)hipFree(ctx->closest);
+        for (void* p : ctx->outgrown) (void)hipFree(p);
+        if (ctx->closestDone) (void)hipEventDestroy(ctx->closestDone);
         if (ctx->adjTable) (void)hipFree(ctx->adjTable);
         if (ctx->batch) (void)hipFree(ctx->batch);
         destroyWfState(ctx);

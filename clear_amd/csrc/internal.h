@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <string>
+#include <vector>
 
 #include "../../include/clear_amd.h"
 
@@ -55,6 +56,13 @@ struct clr_ctx {
     // Traversal-stack overflow region of the ordered trace kernel.
     uint32_t* traceSpill = nullptr;
     size_t traceSpillBytes = 0;
+    // Layout and stacks of clr_trace_closest's walk of many rays (traverse.hip):
+    // a block of its own, which no captured call uses, and the end of the last
+    // call's work in it. Outgrown blocks are kept until the context goes.
+    void* closest = nullptr;
+    size_t closestBytes = 0;
+    hipEvent_t closestDone = nullptr;
+    std::vector<void*> outgrown;
     // Device address of this device's static working array of
     // clr_lbvh_build_soup_noalloc (looked up by clr_create; not owned).
     void* noAllocScratch = nullptr;
@@ -182,6 +190,11 @@ int checkRenderArgs(clr_ctx* ctx, const clr_scene_dev* scene, const clr_render_p
 
 // ---- traversal (traverse.hip) ----
 int ensureTraceSpill(clr_ctx* ctx, size_t bytes);
+// Makes room for one more block in ctx->outgrown; false without memory for it.
+bool roomForOutgrown(clr_ctx* ctx);
+// Makes sure ctx->closest holds `bytes`, without synchronising; false if there
+// is no memory for it (the block stays as it is).
+bool ensureClosest(clr_ctx* ctx, size_t bytes);
 // Launches the traversal-layout build into caller-given arrays (from the
 // LBVH pair, or from a CPU midpoint BVH when bvh is not null; without node
 // records when anodes is null).

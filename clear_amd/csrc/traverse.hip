@@ -311,14 +311,14 @@ __device__ __forceinline__ void traceTwo(W& w0, W& w1, const float* __restrict__
 // triangles and 1,000,000 rays 21.0 and 7.1 (first and last). A third
 // request for the stack's top was slower (3.7 -> 4.2 ms): a visit is bound by
 // its instructions.
+constexpr int kReferencePairs = kOrdHalf;  // stack entries in LDS
 template <bool STATS>
 __global__ __launch_bounds__(kOrdBlock) void k_trace_reference(
     dev::GeomScene g, const float* __restrict__ rays, uint32_t numRays, uint32_t* __restrict__ hitFace,
     float* __restrict__ hitT, uint32_t* __restrict__ stats, uint32_t* __restrict__ status,
     uint32_t* __restrict__ spill) {
-    constexpr int kPairs = kOrdHalf;
-    using S = dev::PairStack<kPairs, dev::kStackDepth>;
-    __shared__ uint2 s_stack[kPairs * kOrdBlock];
+    using S = dev::PairStack<kReferencePairs, dev::kStackDepth>;
+    __shared__ uint2 s_stack[kReferencePairs * kOrdBlock];
     const uint32_t gid = blockIdx.x * kOrdBlock + threadIdx.x;
     const uint32_t lanes = gridDim.x * kOrdBlock;
     const S stk{s_stack + threadIdx.x, kOrdBlock, reinterpret_cast<uint2*>(spill) + gid, lanes};
@@ -471,18 +471,14 @@ void launchAccelBuild(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves,
 }
 
 namespace {
-// Grid of a kernel that runs traceTwo (16 waves per CU; LDS: 16 KiB per
-// 128-thread block) and its stacks' spill memory.
+// Grid of the kernels with 128-thread blocks: 16 waves per CU (LDS: 16 KiB per
+// block).
 int traceGrid(clr_ctx* ctx, uint32_t numRays, uint32_t& grid) {
     int cus = 0;
     int rc = hipCheck(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
     if (rc) return rc;
     grid = std::max(1u, std::min((uint32_t)cus * 8u, (numRays + kOrdBlock - 1) / kOrdBlock));
-    const size_t lanes = (size_t)grid * kOrdBlock;
-    // Of the kernels without and with counts the former takes more; both find
-    // room after either.
-    static_assert(2 * kTracePairs >= dev::kStackPairs, "spill covers the counting walks");
-    return ensureTraceSpill(ctx, lanes * 2 * (2 * kTracePairs - kOrdHalf) * sizeof(uint32_t));
+    return CLR_OK;
 }
 }  // namespace
 
@@ -494,6 +490,11 @@ int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     if (rc) return rc;
     uint32_t grid = 0;
     rc = traceGrid(ctx, numRays, grid);
+    if (rc) return rc;
+    // Of the kernels without and with counts the former takes more spill
+    // memory; both find room after either.
+    static_assert(2 * kTracePairs >= dev::kStackPairs, "spill covers the counting walks");
+    rc = ensureTraceSpill(ctx, (size_t)grid * kOrdBlock * 2 * (2 * kTracePairs - kOrdHalf) * sizeof(uint32_t));
     if (rc) return rc;
     clr_scene_dev sd{};
     sd.vertices = vertices;
@@ -539,27 +540,32 @@ int traceClosest(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
             (void)hipGetLastError();
             capture = hipStreamCaptureStatusActive;
         }
-        if (capture == hipStreamCaptureStatusNone) {
-            uint32_t grid = 0;
-            clr_scene_dev sd{};
-            sd.vertices = vertices;
-            sd.faces = faces;
-            sd.internalNodes = inodes;
-            sd.leafNodes = leaves;
-            sd.numFaces = n;
-            dev::GeomScene g;
-            rc = traceGrid(ctx, numRays, grid);
-            if (!rc) rc = buildAccel(ctx, sd, AccelKind::kBinary, g, stream);
-            if (!rc) {
-                if (stats)
-                    k_trace_reference<true><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats,
-                                                                            ctx->devStatus, ctx->traceSpill);
-                else
-                    k_trace_reference<false><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats,
-                                                                             ctx->devStatus, ctx->traceSpill);
-                return hipCheck(ctx, hipGetLastError(), "trace launch");
-            }
-            (void)hipGetLastError();  // no memory for it
+        uint32_t grid = 0;
+        rc = traceGrid(ctx, numRays, grid);
+        if (rc) return rc;
+        const size_t nodeBytes = accelNodeBytes(n, false), triBytes = ((size_t)n * 48 + 255) & ~size_t(255);
+        const size_t stackBytes = (size_t)grid * kOrdBlock * (dev::kStackDepth - kReferencePairs) * sizeof(uint2);
+        if (capture == hipStreamCaptureStatusNone && ensureClosest(ctx, nodeBytes + triBytes + stackBytes)) {
+            // Calls on several streams of the context take turns in the block
+            // (the first wait finds nothing recorded and passes).
+            rc = hipCheck(ctx, hipStreamWaitEvent(stream, ctx->closestDone, 0), "trace order");
+            if (rc) return rc;
+            dev::GeomScene g{inodes, leaves, n, vertices, faces};
+            char* block = static_cast<char*>(ctx->closest);
+            float4* nodes = reinterpret_cast<float4*>(block);
+            float4* tris = reinterpret_cast<float4*>(block + nodeBytes);
+            uint32_t* spill = reinterpret_cast<uint32_t*>(block + nodeBytes + triBytes);
+            launchAccelBuild(inodes, leaves, nullptr, n, vertices, faces, nodes, tris, stream);
+            g.anodes = nodes;
+            g.atris = tris;
+            if (stats)
+                k_trace_reference<true><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats,
+                                                                        ctx->devStatus, spill);
+            else
+                k_trace_reference<false><<<grid, kOrdBlock, 0, stream>>>(g, rays, numRays, hitFace, hitT, stats,
+                                                                         ctx->devStatus, spill);
+            rc = hipCheck(ctx, hipGetLastError(), "trace launch");
+            return rc ? rc : hipCheck(ctx, hipEventRecord(ctx->closestDone, stream), "trace order");
         }
     }
     const unsigned grid = (numRays + kTraceBlock - 1) / kTraceBlock;

@@ -7,8 +7,8 @@
  * (a hipStream_t passed as void*; NULL = the default stream) and is
  * stream-ordered: no entry point synchronises the host unless its comment says
  * so. A clr_ctx is externally synchronised: one host thread at a time, and
- * its scratch (LBVH pool, render and wavefront state) is shared
- * by all its calls, so work enqueued through one context must stay on one
+ * its scratch (LBVH pool, traversal layout and stacks, render and wavefront
+ * state) is shared by all its calls, so work enqueued through one context must stay on one
  * stream, or calls on different streams must be ordered by the caller (use
  * one context per concurrent stream).
  *
@@ -213,9 +213,11 @@ int clr_lbvh_last_profile(clr_ctx* ctx, float* msPerStage, int maxStages, int* n
  *           triangle tests per ray (NULL to skip)
  * Face indices are 32-bit (the reference truncates to 16 bits,
  * bvh_traversal.cl:43,55). Many rays against a scene that is not small walk a
- * copy of the nodes in the context's scratch (the same order, tests, hits and
- * counts); without memory for it, and in a call that is being captured, the
- * nodes themselves. */
+ * copy of the nodes (the same order, tests, hits and counts) in a block that
+ * the context keeps for these calls alone: it grows without synchronising, no
+ * captured call uses it, and calls on several streams are ordered through it.
+ * Without memory for it, and in a call that is being captured, the nodes
+ * themselves are walked. */
 int clr_trace_closest(clr_ctx* ctx, const clr_lbvh_inode* internalNodes,
                       const clr_lbvh_leaf* leafNodes, uint32_t numFaces,
                       const clr_float3* vertices, const clr_face* faces,
