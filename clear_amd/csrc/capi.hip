@@ -74,20 +74,39 @@ int ensureRenderScratch(clr_ctx* ctx, uint32_t numFaces) {
     return CLR_OK;
 }
 
-int ensureTraceSpill(clr_ctx* ctx, size_t bytes) {
-    if (ctx->traceSpillBytes >= bytes) return CLR_OK;
-    int rc = hipCheck(ctx, hipDeviceSynchronize(), "trace spill regrow sync");
-    if (rc) return rc;
-    if (ctx->traceSpill) (void)hipFree(ctx->traceSpill);
-    ctx->traceSpill = nullptr;
-    ctx->traceSpillBytes = 0;
-    hipError_t e = hipMalloc(&ctx->traceSpill, bytes);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->traceSpill = nullptr;
-        return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "trace spill");
+void holdIfCapturing(hipStream_t stream, bool& held) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) (void)hipGetLastError();
+    else if (capture != hipStreamCaptureStatusNone) held = true;
+}
+
+int giveUp(clr_ctx* ctx, void* block, bool& held) {
+    if (block && held) {
+        if (!roomForOutgrown(ctx)) return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "list of captured blocks");
+        ctx->outgrown.push_back(block);
+    } else if (block) {
+        (void)hipFree(block);
     }
-    ctx->traceSpillBytes = bytes;
+    held = false;
+    return CLR_OK;
+}
+
+int ensureTraceSpill(clr_ctx* ctx, size_t bytes, hipStream_t stream) {
+    if (ctx->traceSpillBytes < bytes) {
+        int rc = hipCheck(ctx, hipDeviceSynchronize(), "trace spill regrow sync");
+        if (!rc) rc = giveUp(ctx, ctx->traceSpill, ctx->traceSpillHeld);
+        if (rc) return rc;
+        ctx->traceSpill = nullptr;
+        ctx->traceSpillBytes = 0;
+        hipError_t e = hipMalloc(&ctx->traceSpill, bytes);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->traceSpill = nullptr;
+            return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "trace spill");
+        }
+        ctx->traceSpillBytes = bytes;
+    }
+    holdIfCapturing(stream, ctx->traceSpillHeld);
     return CLR_OK;
 }
 

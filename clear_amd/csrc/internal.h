@@ -53,15 +53,19 @@ struct clr_ctx {
     // Traversal layout of the ordered walk (rebuilt by every call that uses it).
     void* accel = nullptr;
     size_t accelBytes = 0;
+    bool accelHeld = false;  // a captured call may refer to it
     // Traversal-stack overflow region of the ordered trace kernel.
     uint32_t* traceSpill = nullptr;
     size_t traceSpillBytes = 0;
+    bool traceSpillHeld = false;  // a captured call may refer to it
     // Layout and stacks of clr_trace_closest's walk of many rays (traverse.hip):
     // a block of its own, which no captured call uses, and the end of the last
-    // call's work in it. Outgrown blocks are kept until the context goes.
+    // call's work in it.
     void* closest = nullptr;
     size_t closestBytes = 0;
     hipEvent_t closestDone = nullptr;
+    // Outgrown blocks that are kept until the context goes: those of `closest`,
+    // which may be in use, and those that a captured call may refer to.
     std::vector<void*> outgrown;
     // Device address of this device's static working array of
     // clr_lbvh_build_soup_noalloc (looked up by clr_create; not owned).
@@ -189,7 +193,14 @@ int renderBvhVisualizer(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_
 int checkRenderArgs(clr_ctx* ctx, const clr_scene_dev* scene, const clr_render_params* params);
 
 // ---- traversal (traverse.hip) ----
-int ensureTraceSpill(clr_ctx* ctx, size_t bytes);
+// Makes sure ctx->traceSpill holds `bytes` for a call on `stream`; synchronises
+// the device when it has to regrow.
+int ensureTraceSpill(clr_ctx* ctx, size_t bytes, hipStream_t stream);
+// Marks a block as held if `stream` is being captured.
+void holdIfCapturing(hipStream_t stream, bool& held);
+// Gives up a block that is to be replaced, after a synchronise: freed, or kept
+// until the context goes if it is held.
+int giveUp(clr_ctx* ctx, void* block, bool& held);
 // Makes room for one more block in ctx->outgrown; false without memory for it.
 bool roomForOutgrown(clr_ctx* ctx);
 // Makes sure ctx->closest holds `bytes`, without synchronising; false if there

@@ -974,7 +974,7 @@ int renderMegakernel(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_par
         std::max(1u, std::min(tiles, (uint32_t)cus * (reference ? kReferenceWavesPerCU : kMegaWavesPerCU)));
     uint32_t* counter = ctx->devStatus + kWordMegaTiles;
     if (!reference) {
-        rc = ensureTraceSpill(ctx, (size_t)grid * 64 * (dev::kStackDepth - kMegaLds) * sizeof(uint32_t));
+        rc = ensureTraceSpill(ctx, (size_t)grid * 64 * (dev::kStackDepth - kMegaLds) * sizeof(uint32_t), stream);
         if (rc) return rc;
     }
     k_mega_reset<<<1, 64, 0, stream>>>(counter);
@@ -1010,7 +1010,7 @@ int renderMegakernelBatch(clr_ctx* ctx, const clr_scene_dev* scenes, uint32_t nu
             return fail(ctx, CLR_ERR_INVALID_ARG,
                         "the trace spill must be sized by an eager render of this batch before capture");
     }
-    rc = ensureTraceSpill(ctx, spillBytes);
+    rc = ensureTraceSpill(ctx, spillBytes, stream);
     if (rc) return rc;
     dev::RScene* table = nullptr;
     dev::RScene first;
@@ -1072,7 +1072,7 @@ int renderAdjoint(clr_ctx* ctx, const clr_scene_dev& sd, const clr_render_params
     rc = hipCheck(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
     if (rc) return rc;
     const uint32_t grid = std::max(1u, std::min(tiles, (uint32_t)cus * kAdjWavesPerCU));
-    rc = ensureTraceSpill(ctx, (size_t)grid * 64 * (dev::kStackDepth - kAdjLds) * sizeof(uint32_t));
+    rc = ensureTraceSpill(ctx, (size_t)grid * 64 * (dev::kStackDepth - kAdjLds) * sizeof(uint32_t), stream);
     if (rc) return rc;
     uint32_t* counter = ctx->devStatus + kWordMegaTiles;
     k_mega_reset<<<1, 64, 0, stream>>>(counter);

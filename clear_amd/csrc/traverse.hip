@@ -431,8 +431,8 @@ int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomS
     const size_t need = nodeBytes + triBytes, either = accelWideBytes(n, midpoint) + triBytes;
     if (ctx->accelBytes < need) {
         int rc = hipCheck(ctx, hipDeviceSynchronize(), "accel regrow sync");
+        if (!rc) rc = giveUp(ctx, ctx->accel, ctx->accelHeld);
         if (rc) return rc;
-        if (ctx->accel) (void)hipFree(ctx->accel);
         ctx->accel = nullptr;
         ctx->accelBytes = 0;
         for (size_t bytes : {either, need}) {
@@ -446,6 +446,7 @@ int buildAccel(clr_ctx* ctx, const clr_scene_dev& sd, AccelKind kind, dev::GeomS
         if (!ctx->accel)
             return fail(ctx, CLR_ERR_OUT_OF_MEMORY, "traversal layout of " + std::to_string(need) + " bytes");
     }
+    holdIfCapturing(stream, ctx->accelHeld);
     float4* nodes = static_cast<float4*>(ctx->accel);
     float4* tris = reinterpret_cast<float4*>(static_cast<char*>(ctx->accel) + nodeBytes);
     launchAccelBuild(sd.internalNodes, sd.leafNodes, sd.bvhNodes, n, sd.vertices, sd.faces,
@@ -494,7 +495,8 @@ int traceOrdered(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
     // Of the kernels without and with counts the former takes more spill
     // memory; both find room after either.
     static_assert(2 * kTracePairs >= dev::kStackPairs, "spill covers the counting walks");
-    rc = ensureTraceSpill(ctx, (size_t)grid * kOrdBlock * 2 * (2 * kTracePairs - kOrdHalf) * sizeof(uint32_t));
+    rc = ensureTraceSpill(ctx, (size_t)grid * kOrdBlock * 2 * (2 * kTracePairs - kOrdHalf) * sizeof(uint32_t),
+                          stream);
     if (rc) return rc;
     clr_scene_dev sd{};
     sd.vertices = vertices;

@@ -1,6 +1,7 @@
 """The memory of clr_trace_closest's walk of many rays: it grows without
 touching what captured calls use, without ending captures of other streams,
-and calls on several streams may share it."""
+and calls on several streams may share it. The blocks of the other walks stay
+while a captured call refers to them."""
 import numpy as np
 import pytest
 
@@ -61,8 +62,9 @@ def by_parts(ctx, s):
     return hit, t
 
 
+@pytest.mark.parametrize("larger", ["reference", "ordered", "wide"])
 @pytest.mark.parametrize("walk", ["ordered", "wide"])
-def test_captured_traces_outlive_larger_ones(ctx, walk):
+def test_captured_traces_outlive_larger_ones(ctx, walk, larger):
     import torch
 
     small, large = Scene(ctx, 5000, 20000, 1), Scene(ctx, 60000, 1 << 17, 2)
@@ -72,13 +74,49 @@ def test_captured_traces_outlive_larger_ones(ctx, walk):
     with torch.cuda.graph(g, capture_error_mode="thread_local"):
         small.trace(ctx, **{walk: True})
     for k in range(3):
-        print(f"[trace scratch] {walk}: replay {k}", flush=True)
-        large.trace(ctx)
+        print(f"[trace scratch] {walk}, then {larger}: replay {k}", flush=True)
+        large.trace(ctx, **({} if larger == "reference" else {larger: True}))
         small.clear()
         torch.cuda.synchronize()
         g.replay()
         equal(small.out(), want)
-    equal(large.out(), by_parts(ctx, large))
+    if larger == "reference":
+        equal(large.out(), by_parts(ctx, large))
+    else:  # the same hits from a context with nothing captured
+        got = large.out()
+        fresh = ca.Context(0)
+        large.trace(fresh, **{larger: True})
+        equal(large.out(), got)
+        fresh.close()
+    assert ctx.device_status() == 0
+
+
+def test_captured_render_outlives_a_larger_scene(ctx):
+    import torch
+
+    W, H, spp, depth = 48, 40, 2, 4
+    host, big = ca.HostScene(ca.SCENE_CORNELL, W, H, detail=3), Scene(ctx, 60000, 1 << 15, 7)
+    ds = ca.DeviceScene(ctx, host)
+    states, pixels = ca.new_image(W, H)
+
+    def frame():
+        ca.seed_pixel_states(ctx, W, H, states)
+        pixels.zero_()
+        ca.render(ctx, ds, spp, depth, states, pixels)
+
+    frame()
+    torch.cuda.synchronize()
+    want = pixels.cpu().numpy()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+        frame()
+    for k in range(3):
+        print(f"[trace scratch] render replay {k}", flush=True)
+        big.trace(ctx, wide=True)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(pixels.cpu().numpy(), want)
     assert ctx.device_status() == 0
 
 
