@@ -55,21 +55,27 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_closest(
     }
 }
 
-// Triangle record of face i (see GeomScene): p0 | alpha flag, the two edges.
-__device__ __forceinline__ void storeTri(const clr_float3* __restrict__ verts, const clr_face* __restrict__ faces,
-                                         uint32_t i, float4* __restrict__ atris) {
-    const clr_face& f = faces[i];
+// Triangle record (see GeomScene) of a face at `o`: p0 | tag, the two edges.
+__device__ __forceinline__ void storeTri(const clr_float3* __restrict__ verts, const clr_face& f, uint32_t tag,
+                                         float4* __restrict__ o) {
     const dev::V3 p0 = dev::loadV3(verts, f.p0), p1 = dev::loadV3(verts, f.p1), p2 = dev::loadV3(verts, f.p2);
-    const uint32_t flag = f.uv0 != dev::kNone && f.alphaTexPtr != dev::kNone ? 1u : 0u;
     const dev::V3 e1 = p1 - p0, e2 = p2 - p0;
-    float4* o = atris + 3 * (size_t)i;
-    o[0] = make_float4(p0.x, p0.y, p0.z, __uint_as_float(flag));
+    o[0] = make_float4(p0.x, p0.y, p0.z, __uint_as_float(tag));
     o[1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
     o[2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
 }
+// Face i's, tagged with its alpha flag.
+__device__ __forceinline__ void storeFace(const clr_float3* __restrict__ verts, const clr_face* __restrict__ faces,
+                                          uint32_t i, float4* __restrict__ atris) {
+    const clr_face& f = faces[i];
+    storeTri(verts, f, f.uv0 != dev::kNone && f.alphaTexPtr != dev::kNone ? 1u : 0u, atris + 3 * (size_t)i);
+}
 
 // Traversal layout (see GeomScene): node i gets both children's boxes and
-// references (unless anodes is null), face i its triangle record.
+// references (unless anodes is null), face i its triangle record. BY_LEAF
+// (ReferenceWalk): leaf children and triangle records by leaf, tagged with the
+// face.
+template <bool BY_LEAF>
 __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const clr_lbvh_leaf* __restrict__ leaves,
                               uint32_t n, const clr_float3* __restrict__ verts, const clr_face* __restrict__ faces,
                               float4* __restrict__ anodes, float4* __restrict__ atris) {
@@ -94,7 +100,7 @@ __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const c
                                    : reinterpret_cast<const float4*>(inodes + ci);
             box[k][0] = p[0];
             box[k][1] = p[1];
-            ref[k] = leaf ? (leaves[ci].objIdx | dev::kLeafRef) : ci;
+            ref[k] = !leaf ? ci : (BY_LEAF ? ci : leaves[ci].objIdx) | dev::kLeafRef;
         }
         float4* o = anodes + 4 * (size_t)i;
         o[0] = make_float4(box[0][0].x, box[0][0].y, box[0][0].z, __uint_as_float(ref[0]));
@@ -102,7 +108,13 @@ __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const c
         o[2] = make_float4(box[1][0].x, box[1][0].y, box[1][0].z, 0.0f);
         o[3] = make_float4(box[1][1].x, box[1][1].y, box[1][1].z, 0.0f);
     }
-    if (i < n) storeTri(verts, faces, i, atris);
+    if (i >= n) return;
+    if constexpr (BY_LEAF) {
+        const uint32_t face = leaves[i].objIdx;
+        storeTri(verts, faces[face], face, atris + 3 * (size_t)i);
+    } else {
+        storeFace(verts, faces, i, atris);
+    }
 }
 
 // Traversal layout of a CPU midpoint BVH, indexed by node number: internal
@@ -134,7 +146,7 @@ __global__ void k_accel_build_bvh(const float4* __restrict__ bvh, uint32_t n, co
             o[3] = make_float4(box[1][1].x, box[1][1].y, box[1][1].z, 0.0f);
         }
     }
-    if (i < n) storeTri(verts, faces, i, atris);
+    if (i < n) storeFace(verts, faces, i, atris);
 }
 
 // 4-wide records (GeomScene::wnodes) of the LBVH: record i holds the
@@ -468,7 +480,7 @@ void launchAccelBuild(const clr_lbvh_inode* inodes, const clr_lbvh_leaf* leaves,
         k_accel_build_bvh<<<(2 * n - 1 + 255) / 256, 256, 0, stream>>>(reinterpret_cast<const float4*>(bvh), n,
                                                                         vertices, faces, anodes, atris);
     else
-        k_accel_build<<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, vertices, faces, anodes, atris);
+        k_accel_build<false><<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, vertices, faces, anodes, atris);
 }
 
 namespace {
@@ -557,7 +569,7 @@ int traceClosest(clr_ctx* ctx, const clr_lbvh_inode* inodes, const clr_lbvh_leaf
             float4* nodes = reinterpret_cast<float4*>(block);
             float4* tris = reinterpret_cast<float4*>(block + nodeBytes);
             uint32_t* spill = reinterpret_cast<uint32_t*>(block + nodeBytes + triBytes);
-            launchAccelBuild(inodes, leaves, nullptr, n, vertices, faces, nodes, tris, stream);
+            k_accel_build<true><<<(n + 255) / 256, 256, 0, stream>>>(inodes, leaves, n, vertices, faces, nodes, tris);
             g.anodes = nodes;
             g.atris = tris;
             if (stats)

@@ -756,7 +756,10 @@ struct PairStack {
 };
 
 // The reference's walk (lbvhClosest: its order, box tests, hits, counts and
-// overflow) over the binary traversal layout, for many rays. lbvhClosest is
+// overflow) over a binary traversal layout whose triangle records lie by leaf,
+// with the face in place of the alpha flag, for many rays. (By face they would
+// hold only the first numFaces; a leaf may refer to any face of the caller's.)
+// lbvhClosest is
 // bound by the latency of a pop: a node's record, then its leaves, their faces
 // and their vertices, each a dependent load, for boxes that mostly fail. Here a
 // visit tests both children's boxes, which came with the node's own record: a
@@ -783,15 +786,15 @@ struct ReferenceWalk {
 
     __device__ __forceinline__ ReferenceWalk(const GeomScene& g_, const Stack& s_) : g(g_), stack(s_) {}
 
-    __device__ __forceinline__ void leaf(uint32_t face) {
+    __device__ __forceinline__ void leaf(uint32_t i) {
         if constexpr (STATS) ++st.tests;
-        if (face >= g.n) {  // malformed nodes
+        if (i >= g.n) {  // malformed nodes
             overflowed = true;
             return;
         }
         float b1, b2;
-        uint32_t flag;
-        if (triTestPacked(g.atris, o, d, face, t, b1, b2, flag)) best = face;
+        uint32_t face;
+        if (triTestPacked(g.atris, o, d, i, t, b1, b2, face)) best = face;
     }
 
     __device__ __forceinline__ void begin(V3 o_, V3 d_, float tmax) {
@@ -812,7 +815,7 @@ struct ReferenceWalk {
         st = {0u, 0u};
         const float4* p = g.n == 1 ? reinterpret_cast<const float4*>(g.leaves) : reinterpret_cast<const float4*>(g.inodes);
         const bool pass = boxTest(p[0], p[1], o, d, t);
-        if (g.n == 1 && pass) leaf(reinterpret_cast<const uint32_t*>(p + 2)[0]);
+        if (g.n == 1 && pass) leaf(0);
         if (g.n > 1 && pass) {
             node = 0;
             cur = load(0);

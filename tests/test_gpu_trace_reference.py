@@ -94,3 +94,20 @@ def test_stack_slots_are_the_drop_in_walks(gpu_ctx, levels, miss, status):
     rays[6] = np.inf
     print(f"[trace reference] comb of {levels} levels", flush=True)
     compare(gpu_ctx, (cuda(inodes), cuda(leaves)), soup.shape[0], cuda(v), cuda(f), rays, True, status)
+
+
+@pytest.mark.parametrize("counts", [False, True])
+def test_leaves_of_faces_beyond_num_faces(gpu_ctx, counts):
+    """Leaves may refer to any face of the caller's array, as for the walk over
+    the drop-in nodes: a tree over the last faces of a longer array."""
+    n, first = 5000, 3000
+    v, f = mesh(first + n)
+    sub = np.ascontiguousarray(f[first:])
+    tv, tf = cuda(v), cuda(f)
+    nodes = ca.node_buffers(n)
+    ca.LBVHBuilder(gpu_ctx, n, 10).perform(tv, cuda(sub), n, 10, *nodes)
+    leaves = nodes[1].cpu().numpy().view(np.uint32).reshape(-1, 12)
+    leaves[:, 8] += first
+    nodes = (nodes[0], cuda(leaves))
+    print(f"[trace reference] faces beyond numFaces, counts={counts}", flush=True)
+    compare(gpu_ctx, nodes, n, tv, tf, edge_rays(MANY + 3, seed=11), counts)
