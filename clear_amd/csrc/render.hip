@@ -181,7 +181,7 @@ struct ImageJob {
 // pixel after the other (the terms, their order and the random numbers of
 // tracePath, so images and states are bit-identical), and every lane one ray at
 // a time: a camera or extension ray, or a light sample's shadow ray. A lane
-// whose ray is finished waits until kServeMin lanes wait (or none walks); they
+// whose ray is finished waits until most lanes wait (or none walks); they
 // are then served together: shaded, given their next ray, next sample or next
 // pixel. Serving all lanes only when the last one has finished its ray keeps
 // lanes idle for as long as the longest walk (17.5 % of VALU lanes active);
@@ -197,7 +197,13 @@ struct ImageJob {
 // order, the order in which the closest hit is defined.
 // JOB: loads and stores a pixel, and observes the path's radiance terms
 // (nothing for images, derivatives for the adjoint).
-constexpr uint32_t kServeMin = 56;
+// Most: all but an eighth of the lanes that have a pixel. At 1080p over 3.1 M
+// triangles and 32 spp, where all lanes have one, 8 / 16 / 24 / 36 / 48 / 56 / 64 of
+// them took 293 / 200 / 163 / 139 / 127 / 124 / 161 ms. Fewer are left in tiles at an
+// edge and while a wave runs out of pixels; a fixed 56, for which these waited for
+// all, took 6.96 ms where this takes 6.56 on 160x160 Cornell at 16 spp, 1.71 and 1.65
+// on 96x96 at 4 spp, 2.37 and 2.39 on 256x256 of the showcase scene at 4 spp.
+constexpr int kServeShift = 3;
 
 template <class Job, class Stack, class Source>
 __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint32_t maxDepth, uint32_t flags,
@@ -395,11 +401,12 @@ __device__ __forceinline__ void tracePixels(const RScene& S, uint32_t spp, uint3
         }
         if (ray) w.begin(org, dir, bound, anyRay, boundFace);
         if (__ballot(live) == 0) break;
+        const int lanes = __popcll(__ballot(live)), serve = lanes - (lanes >> kServeShift);
         // Walk until enough lanes wait. Every walk ends (its visits are
         // bounded), so the loop does.
         do {
             if (!w.done()) w.step();
-        } while (__ballot(!w.done()) != 0 && __popcll(__ballot(live && w.done())) < (int)kServeMin);
+        } while (__ballot(!w.done()) != 0 && __popcll(__ballot(live && w.done())) < serve);
     }
     if (over) atomicOr(S.status, kStatusStackOverflow);
 }
@@ -615,9 +622,18 @@ __device__ __forceinline__ uint32_t nextTile(uint32_t* tileCounter) {
 // counter: tiles [first, end) of one image, whose first tile is number
 // `first` of the counter's. A tile beyond `end` ends the source and stays in
 // `tile` for the caller (the next image of a batch, or past the last one).
+// A wave takes its next tile when it has finished the last one, or (below
+// `early`) as soon as one of its lanes is free: in images of more tiles than the
+// grid has waves, where every wave still to start has a tile (1280x720 Cornell
+// at 2 spp 3.16 ms against 3.52). Where each tile has a wave, a tile taken early is
+// taken from a wave about to start (20 scenes of 53x53 at 2 spp 738 us, 636 without);
+// and in a batch the next tile lies a whole grid further on, mostly in another
+// scene, so it would be held until the wave has drained (32 scenes of 128x128 at
+// 32 spp 37.9 ms, 30.8 without; 160x160 at 2 spp 2.06 and 1.89).
 struct TileSource {
     uint32_t* counter;
     uint32_t width, height, tilesX, first, end;
+    uint32_t early;     // below this tile the next one is taken early
     uint32_t tile;      // current tile
     uint32_t next = 0;  // its next position, 0..64
     bool open = true;
@@ -628,6 +644,7 @@ struct TileSource {
             const uint64_t idle = __ballot(want && !got);
             if (idle == 0) break;
             if (next >= 64u) {
+                if (tile >= early && __ballot(!want || got) != 0) break;
                 tile = nextTile(counter);
                 next = 0;
                 if (tile >= end) open = false;
@@ -657,7 +674,8 @@ __device__ __forceinline__ void renderImage(const dev::RScene& scene, uint32_t w
     dev::RScene S = scene;  // resolved copy; the kernel argument itself stays read-only
     dev::finishScene(S);
     const uint32_t tilesX = (width + kTile - 1) / kTile;
-    TileSource src{tileCounter, width, height, tilesX, 0u, tilesX * ((height + kTile - 1) / kTile),
+    const uint32_t tiles = tilesX * ((height + kTile - 1) / kTile);
+    TileSource src{tileCounter, width, height, tilesX, 0u, tiles, tiles > gridDim.x ? tiles : 0u,
                    nextTile(tileCounter)};
     src.open = src.tile < src.end;
     const MegaStack<LDS> stk = megaStack<LDS>(s_stack, spill);
@@ -686,7 +704,7 @@ __device__ __forceinline__ void renderBatch(const dev::RScene* __restrict__ tabl
         const dev::RScene S = dev::tableScene(table, s);
         dev::ImageJob job{reinterpret_cast<uint4*>(states) + npix * s, reinterpret_cast<float4*>(pixels) + npix * s,
                           width};
-        TileSource src{tileCounter, width, height, tilesX, s * tilesPerScene, (s + 1) * tilesPerScene, tile};
+        TileSource src{tileCounter, width, height, tilesX, s * tilesPerScene, (s + 1) * tilesPerScene, 0u, tile};
         dev::tracePixels(S, spp, maxDepth, flags, stk, job, src);
         tile = src.tile;
     }
@@ -704,8 +722,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 
 // Images of at most kMegaFewTiles tiles per CU cannot fill many waves per
 // CU, so their waves keep the whole stack in LDS and all the registers they
-// want (no spills).
-constexpr uint32_t kMegaFewTiles = 4;
+// want (no spills; 185 VGPRs, two waves per SIMD). The line, k_render_mega /
+// this kernel: 5 tiles per CU (320x256 Cornell at 4 spp) 2.00 / 1.84 ms, (showcase
+// 320x240, 16 spp) 8.60 / 8.12; 8 (32 scenes of 64x64, 4 spp) 1.41 / 1.36; 10 (12 of
+// 120x120, 2 spp) 0.71 / 0.68; 16 (showcase 512x512, 1 spp) 0.94 / 1.02, (512x512
+// gradient step) 22.9 / 26.5.
+constexpr uint32_t kMegaFewTiles = 8;
 __global__ __launch_bounds__(64) void k_render_mega_few(dev::RScene scene, uint32_t width, uint32_t height,
                                                         uint32_t spp, uint32_t maxDepth, uint32_t flags,
                                                         uint32_t* __restrict__ states, clr_float3* __restrict__ pixels,

@@ -254,3 +254,15 @@ def test_bvh_visualizer(gpu_ctx, walk, kind):
     print(f"[render parity] visualizer kind={kind} {walk}: equal pixels {ok.mean():.5f}, "
           f"mean {ref.mean():.4f}", flush=True)
     assert ok.mean() >= 0.999
+
+
+@pytest.mark.parametrize("size", [(53, 53), (512, 256), (520, 256), (512, 512), (520, 512)])
+def test_megakernel_schedules_agree(gpu_ctx, size):
+    """Sizes on both sides of the megakernel's lines (on 256 CUs: 2048 tiles
+    for the kernel without spills, 4096 waves of the grid) and tiles cut off
+    by the image's edge: the image is the wavefront renderer's."""
+    host = ca.HostScene(ca.SCENE_CORNELL, *size, detail=2)
+    print(f"[megakernel schedules] {size[0]}x{size[1]}", flush=True)
+    a, b = (gpu_render(gpu_ctx, host, 2, 4, mode=m) for m in (ca.RENDER_MEGAKERNEL, ca.RENDER_WAVEFRONT))
+    np.testing.assert_array_equal(a[0], b[0])
+    np.testing.assert_array_equal(a[1], b[1])
