@@ -394,17 +394,15 @@ struct RareAlpha {
 // the reference's walk over the CPU midpoint BVH.
 enum : int { kWalkLbvh = 0, kWalkOrdered = 1, kWalkMidpoint = 2 };
 
-// rayIntersection with hit parameters, by WALK. Returns false (face = kNone)
-// on a miss.
+// rayIntersection with hit parameters, by WALK (one of the reference's; the
+// ordered traversal runs in tracePixels). Returns false (face = kNone) on a miss.
 template <int WALK, class Stack>
 __device__ __forceinline__ bool intersect(const RScene& S, V3 org, V3 dir, const Stack& stack, SurfPt& sp) {
     float t = INFINITY, b1 = 0.0f, b2 = 0.0f;
     TraceStats st{0u, 0u};
     bool over = false;
     uint32_t face;
-    if constexpr (WALK == kWalkOrdered)  // over the 4-wide records (every render builds them)
-        face = wideHit(S.g, org, dir, t, stack, b1, b2, RareAlpha{&S}, over);
-    else if constexpr (WALK == kWalkMidpoint)
+    if constexpr (WALK == kWalkMidpoint)
         face = bvhWalk<false, false>(S.g, org, dir, t, stack, st, &b1, &b2, TexAlpha{&S}, &over);
     else
         face = lbvhClosest<false, TexAlpha>(S.g, org, dir, t, stack, st, &b1, &b2, TexAlpha{&S}, &over);

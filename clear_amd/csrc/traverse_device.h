@@ -914,11 +914,10 @@ private:
 };
 
 // The walk over the 4-wide records that every renderer and every trace
-// without counts uses. It finds the hit of Ordered and Wide: the smallest
-// (t, face) over the accepted triangles, whatever boxes are entered on the
-// way, as long as none that holds an accepted triangle is passed over. That
-// leaves the box arithmetic free, and a visit is bound by its instructions
-// (few lanes are active, so every instruction counts in full):
+// without counts uses: the boxes, entry distances and leaf tests of Wide, and
+// so its hits, the smallest (t, face) over the accepted triangles. A visit is
+// bound by its instructions (few lanes are active, so every instruction counts
+// in full):
 //   * near and far planes are chosen by the ray's direction signs: two planes
 //     an axis instead of four and a min and max each. The plane distances, pads
 //     and comparisons are slabEnter's, in its order, so a box is admitted exactly
@@ -1116,21 +1115,6 @@ struct WideWalk {
         else mode |= kOver;
     }
 };
-
-// The walk run to completion for one ray. Returns the face (kNone when
-// nothing was accepted) and updates t, b1, b2.
-template <class Alpha, class Stack>
-__device__ __forceinline__ uint32_t wideHit(const GeomScene& g, V3 o, V3 d, float& t, const Stack& stack, float& b1,
-                                            float& b2, const Alpha& alpha, bool& overflow) {
-    WideWalk<Alpha, Stack> w(g, stack, alpha);
-    w.begin(o, d, t);
-    while (!w.done()) w.step();
-    t = w.t;
-    b1 = w.b1;
-    b2 = w.b2;
-    if (w.over()) overflow = true;
-    return w.best;
-}
 
 // The binary ordered walk run to completion for one ray. Returns the face
 // (kNone when nothing was accepted), updates t, b1, b2 and sets the counts.

@@ -108,8 +108,8 @@ const char* clr_last_error(const clr_ctx* ctx);
 /* Bytes currently held by the context's scratch pool. */
 int clr_scratch_bytes(const clr_ctx* ctx, uint64_t* bytes);
 /* Device-side failure flags raised by kernels since the last clear: bit 0 a
- * radix-sort look-back wait, bit 1 a hierarchy hand-off wait exceeded its
- * bound (the result is then wrong), bit 2 a traversal stack overflowed, bit 3
+ * radix-sort look-back wait exceeded its bound (the result is then wrong), bit 1
+ * unused, bit 2 a traversal stack overflowed or nodes were malformed, bit 3
  * the hierarchy met a node with more than two children (unsorted keys), bit 4
  * a segmented build rejected its scene offsets.
  * Synchronises the device. No reference counterpart: the reference has no
@@ -129,7 +129,7 @@ int clr_device_status(clr_ctx* ctx, uint32_t* flags, int clear);
  * the build (LBVHBuilder.cpp:228-229): the call is fully stream-ordered and
  * may be captured into a hipGraph once the scratch pool is large enough
  * (see clr_lbvh_reserve); every replay is a build of the inputs' contents at
- * that time (the hierarchy's hand-off tags advance on the device).
+ * that time.
  * numFaces == 1 writes leafNodes[0] only. */
 int clr_lbvh_build(clr_ctx* ctx, const clr_float3* vertices, const clr_face* faces,
                    uint32_t numFaces, uint32_t numBitsPerDim,

@@ -6,9 +6,8 @@ so each can be captured (here through torch.cuda.graph, whose capture stream
 is the call's stream) and replayed. Every replay must build from the inputs'
 contents at replay time: the triangles change between replays (eager copies
 and synchronisations in between), and each replay's nodes must equal the
-oracle's build of those triangles byte for byte. The hierarchy's box
-hand-off tags each exchange word with a build epoch kept in device memory,
-so a replay never accepts a word from the previous replay as fresh.
+oracle's build of those triangles byte for byte: nothing that an earlier
+replay left in the scratch memory counts.
 """
 import numpy as np
 import pytest
