@@ -319,7 +319,7 @@ __device__ __forceinline__ void traceTwo(W& w0, W& w1, const float* __restrict__
 // scene before they meet anything), so a visit's own latency counts: one ray
 // per lane, both children's records requested before their boxes are tested.
 // 1,000,003 triangles, 524,309 rays: 8.07 ms with k_trace_closest, 5.61 with two
-// rays per lane and no early requests, 4.25 now; with 2,000,000
+// rays per lane and no early requests, 4.0 now; with 2,000,000
 // triangles and 1,000,000 rays 21.0 and 7.1 (first and last). A third
 // request for the stack's top was slower (3.7 -> 4.2 ms): a visit is bound by
 // its instructions.

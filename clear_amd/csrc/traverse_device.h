@@ -53,7 +53,7 @@ __device__ __forceinline__ T* asGlobal(T* p) {
 // per internal node i, 4 x float4 = {min of child 0 | ref0, max of child 0 |
 // ref1, min of child 1, max of child 1} (refs in the .w lanes as bits: an
 // internal child's index, or a leaf child's face index | 0x80000000), and per
-// face its three vertices as float4s. One 64-B load per visited node and one
+// face its first vertex | alpha flag and two edges as float4s. One 64-B load per visited node and one
 // 48-B load per triangle test, where the drop-in layout needs two dependent
 // round trips for each.
 struct GeomScene {
@@ -938,13 +938,13 @@ private:
 // face) order, so an any walk bounded by a light's own hit answers whether
 // that hit is the closest.
 // Stack: PairStack. Alpha: as in Ordered, asked only for flagged triangles.
-// Against the counting walk in the same kernels: 2^22 random rays on 2^24
-// triangles 8.72 -> 8.10 ms, 512x512 at 8 spp of the differentiation scene
-// 31.9 -> 26.3 ms (forward and adjoint), 640x360 at 16 spp of the showcase
-// scene on the wavefront renderer 24.3 -> 21.4 ms. Records of 64 bytes (child
-// boxes as bytes on the record's own grid, 9.27 -> 8.22 ms on the random rays,
-// 110 -> 107 ms on 1080p at 32 spp) hold planes in fewer bits than the boxes
-// have, and a plane far from the record's corner lost hits: not used.
+// Against the counting walk: 2^22 random rays on 2^24 triangles 11.3 -> 8.8 ms
+// (1.8 of it building the layout); in the loops that ran both, 512x512 at 8 spp of
+// the differentiation scene 31.9 -> 26.3 ms (forward and adjoint), 640x360 at 16
+// spp of the showcase scene on the wavefront renderer 24.3 -> 21.4 ms. Records of
+// 64 bytes (child boxes as bytes on the record's own grid; 8.2 ms on the random
+// rays, 107 against 110 ms on 1080p at 32 spp) hold planes in fewer bits than the
+// boxes have, and a plane far from the record's corner lost hits: not used.
 template <class Alpha, class Stack>
 struct WideWalk {
     const float4* wn;
