@@ -110,8 +110,12 @@ __global__ void k_accel_build(const clr_lbvh_inode* __restrict__ inodes, const c
     }
     if (i >= n) return;
     if constexpr (BY_LEAF) {
+        // A leaf that nothing refers to may hold anything: no face has the bit
+        // of leaf references, and its record (no edges) is never hit.
         const uint32_t face = leaves[i].objIdx;
-        storeTri(verts, faces[face], face, atris + 3 * (size_t)i);
+        float4* o = atris + 3 * (size_t)i;
+        if (face & dev::kLeafRef) o[0] = o[1] = o[2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        else storeTri(verts, faces[face], face, o);
     } else {
         storeFace(verts, faces, i, atris);
     }

@@ -53,9 +53,9 @@ __device__ __forceinline__ T* asGlobal(T* p) {
 // per internal node i, 4 x float4 = {min of child 0 | ref0, max of child 0 |
 // ref1, min of child 1, max of child 1} (refs in the .w lanes as bits: an
 // internal child's index, or a leaf child's face index | 0x80000000), and per
-// face its first vertex | alpha flag and two edges as float4s. One 64-B load per visited node and one
-// 48-B load per triangle test, where the drop-in layout needs two dependent
-// round trips for each.
+// face its first vertex | alpha flag and its two edges as float4s. One 64-B
+// load per visited node and one 48-B load per triangle test, where the drop-in
+// layout needs two dependent round trips for each.
 struct GeomScene {
     const clr_lbvh_inode* inodes;
     const clr_lbvh_leaf* leaves;

@@ -111,3 +111,15 @@ def test_leaves_of_faces_beyond_num_faces(gpu_ctx, counts):
     nodes = (nodes[0], cuda(leaves))
     print(f"[trace reference] faces beyond numFaces, counts={counts}", flush=True)
     compare(gpu_ctx, nodes, n, tv, tf, edge_rays(MANY + 3, seed=11), counts)
+
+
+@pytest.mark.parametrize("word", [0xFFFFFFFF, 0xABABABAB, 0x80000000])
+def test_leaves_that_no_node_refers_to(gpu_ctx, word):
+    """Only the leaves of the tree count, as for the walk over the drop-in
+    nodes: the others may hold anything."""
+    levels = 20
+    soup, inodes, leaves = comb(levels, 0)
+    leaves[2 * levels + 1:, 8] = word
+    v, f = ca.soup_to_mesh(soup)
+    print(f"[trace reference] unused leaves of {word:#x}", flush=True)
+    compare(gpu_ctx, (cuda(inodes), cuda(leaves)), soup.shape[0], cuda(v), cuda(f), edge_rays(MANY, seed=12), True)
